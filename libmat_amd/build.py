@@ -24,7 +24,10 @@ HOST_SRCS = ["csrc/host/rpd_prep.cpp", "csrc/host/rpd_compat.cpp",
 # (rpd_cellhost.cpp) for programs that compile LibMAT's voronoi_defs.cxx
 CORE_OUT = os.path.join(HERE, "_lib", "librpd_amd_core.so")
 CELLHOST_OBJ = "rpd_cellhost.cpp.o"
-HIP_SRCS = ["csrc/device/rpd_engine.hip"]
+# (source, object suffix, extra flags): the clip's shapes build side by side
+HIP_SRCS = [("csrc/device/rpd_engine.hip", "", [])] + [
+    ("csrc/device/rpd_kernels.hip", f".{k}", [f"-DRPD_CLIP_PART={k}"])
+    for k in range(5)]
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
           "-fno-fast-math", f"-I{INC}"]
 
@@ -44,7 +47,7 @@ def _run(cmd):
     return r
 
 
-def build(jobs=4, verbose=False):
+def build(jobs=6, verbose=False):
     os.makedirs(BUILD, exist_ok=True)
     os.makedirs(os.path.dirname(OUT), exist_ok=True)
     hipcc = _hipcc()
@@ -54,9 +57,9 @@ def build(jobs=4, verbose=False):
         cmds.append(["g++"] + COMMON + ["-Wall", "-c",
                                         os.path.join(HERE, src), "-o", obj])
         objs.append(obj)
-    for src in HIP_SRCS:
-        obj = os.path.join(BUILD, os.path.basename(src) + ".o")
-        cmds.append([hipcc, f"--offload-arch={ARCH}"] + COMMON + [
+    for src, suffix, flags in HIP_SRCS:
+        obj = os.path.join(BUILD, os.path.basename(src) + suffix + ".o")
+        cmds.append([hipcc, f"--offload-arch={ARCH}"] + COMMON + flags + [
             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
             "-Wno-unused-command-line-argument", "-c",
             os.path.join(HERE, src), "-o", obj])

@@ -23,7 +23,7 @@
 #include "rpd_device.h"
 #include "rpd_prep.h"
 #include "../common/rpd_classgrid.h"
-#include "rpd_kernels.hip"
+#include "rpd_stages.hip"
 #include "rpd_learn.hip"
 #include "rpd_nbr.hip"
 #include "rpd_cells.hip"
@@ -763,62 +763,10 @@ CapsRT small_caps(int id) {
   }
 }
 
-static int launch_clip(rpd_ctx* ctx, int tier, int G, ClipArgs& a,
-                       int caps_id = 0) {
+int launch_clip(rpd_ctx* ctx, int tier, int G, const ClipArgs& a,
+                int caps_id = 0) {
   if (a.n_items <= 0) return 0;
-  const int blocks = ceil_div(a.n_items, G);
-#define RPD_LAUNCH(GG, CAPS, EX)                                           \
-  do {                                                                    \
-    if (a.cert.tet_off)                                                   \
-      hipLaunchKernelGGL((k_clip<GG, CAPS, EX, true>), dim3(blocks),      \
-                         dim3(64), 0, ctx->stream, a);                    \
-    else                                                                  \
-      hipLaunchKernelGGL((k_clip<GG, CAPS, EX, false>), dim3(blocks),     \
-                         dim3(64), 0, ctx->stream, a);                    \
-  } while (0)
-  if (tier == 0) {
-    if (caps_id == 2 || caps_id == 3) {
-      if (caps_id == 2) {
-        switch (G) {
-          case 4: RPD_LAUNCH(4, TightCaps, false); break;
-          case 8: RPD_LAUNCH(8, TightCaps, false); break;
-          default: RPD_LAUNCH(16, TightCaps, false); break;
-        }
-      } else {
-        switch (G) {
-          case 4: RPD_LAUNCH(4, MidCaps, false); break;
-          case 8: RPD_LAUNCH(8, MidCaps, false); break;
-          default: RPD_LAUNCH(16, MidCaps, false); break;
-        }
-      }
-    } else if (caps_id == 1) {
-      switch (G) {
-        case 1: RPD_LAUNCH(1, WideCaps, false); break;
-        case 2: RPD_LAUNCH(2, WideCaps, false); break;
-        case 4: RPD_LAUNCH(4, WideCaps, false); break;
-        case 8: RPD_LAUNCH(8, WideCaps, false); break;
-        default: RPD_LAUNCH(16, WideCaps, false); break;
-      }
-    } else {
-      switch (G) {
-        case 1: RPD_LAUNCH(1, SmallCaps, false); break;
-        case 2: RPD_LAUNCH(2, SmallCaps, false); break;
-        case 4: RPD_LAUNCH(4, SmallCaps, false); break;
-        case 8: RPD_LAUNCH(8, SmallCaps, false); break;
-        default: RPD_LAUNCH(16, SmallCaps, false); break;
-      }
-    }
-  } else if (tier == 1) {
-    switch (G) {
-      case 1: RPD_LAUNCH(1, LargeCaps, false); break;
-      case 2: RPD_LAUNCH(2, LargeCaps, false); break;
-      default: RPD_LAUNCH(4, LargeCaps, false); break;
-    }
-  } else {
-    RPD_LAUNCH(1, LargeCaps, true);
-  }
-#undef RPD_LAUNCH
-  HIP_TRY(hipGetLastError());
+  HIP_TRY(clip_launch(ctx->stream, tier, G, a, caps_id));
   return 0;
 }
 

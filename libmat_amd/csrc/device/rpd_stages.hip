@@ -1,0 +1,931 @@
+// HIP kernels of the restricted power diagram (RPD) for CDNA4 (gfx950).
+//
+// Pipeline of one rpd_run (see rpd_engine.hip for the host side):
+//   k_site_bbox    one wavefront per flagged sphere: clips the domain box by
+//                  the neighbour bisectors pushed outwards by the largest
+//                  tet radius; the bbox of that polytope contains the
+//                  centroid of every tet the sphere can relate to
+//   k_bin_*        spheres registered into a uniform grid of tet centroids
+//   k_tet_count /  one thread per tet: the reference's tet-sphere relation
+//   k_tet_fill     (voronoi.cu:154-193) over the spheres of its bin, emitted
+//                  in ascending site id, plus the mask of neighbour planes
+//                  that may cut the tet
+//   k_clip         (rpd_kernels.hip) the clip; tiers: small capacity, full
+//                  capacity, full capacity with exact arithmetic
+//   k_compact_*    deterministic compaction into the output stream
+#include <hip/hip_runtime.h>
+
+#include "rpd_capi.h"
+#include "rpd_clip.h"
+#include "rpd_device.h"
+#include "rpd_geom.h"
+
+namespace rpd {
+
+__global__ __launch_bounds__(256) void k_fill32(int32_t* p, int64_t n,
+                                                int32_t v) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = v;
+}
+
+// A captured run's re-run lists (cnt[1] small-tier overflows, cnt[2] exact
+// re-runs, cnt[6] middle-tier overflows): after a clip launch's tiers the
+// counts are checked against the list positions the host reserved
+// (*overflow otherwise); with next_large >= 0 the counters then start at
+// the positions reserved for the next launch.
+__global__ void k_check_rerun_counts(int32_t* cnt, int32_t lim_large,
+                                     int32_t lim_exact, int32_t lim_full,
+                                     int32_t* overflow, int32_t next_large,
+                                     int32_t next_exact, int32_t next_full) {
+  if (threadIdx.x != 0) return;
+  if (cnt[1] > lim_large || cnt[2] > lim_exact || cnt[6] > lim_full)
+    *overflow = 1;
+  if (next_large >= 0) {
+    cnt[1] = next_large;
+    cnt[2] = next_exact;
+    cnt[6] = next_full;
+  }
+}
+
+// ================================================= candidate gathering
+struct BinGrid {
+  double org[3];
+  double inv_bs;
+  int32_t dim[3];
+  int32_t pad;
+};
+
+// One instance of a batch: its domain box, the largest distance of a tet
+// corner from its tet's centroid (rho, with margin), and its candidate bin
+// grid, whose bins are numbered from bin_base in the batch-wide bin space.
+struct InstInfo {
+  BinGrid g;
+  int64_t bin_base;
+  double dom[6];
+  double rho;
+  BinGrid sg;        // grid of sphere centres (learned proposals)
+  int64_t sg_base;
+  int32_t site_off;  // first site of the instance, number of sites
+  int32_t n_site;
+};
+
+__device__ __forceinline__ int bin_coord(double x, double org, double inv,
+                                         int dim) {
+  double f = floor((x - org) * inv);
+  int c = f < 0 ? 0 : (f >= dim ? dim - 1 : (int)f);
+  return c;
+}
+
+// One wavefront per sphere.  Polytope = domain box clipped by the
+// neighbour bisectors, each pushed out by rho (max tet circum-radius about
+// the centroid plus a margin).  Output bbox (lo, hi); empty if lo > hi.
+// The bisectors are applied nearest first (ascending signed distance of
+// the sphere centre to the bisector), so the polytope shrinks early and
+// later planes rarely cut; that order is also written to knn_near, where
+// the relation test uses it to meet a rejecting neighbour early (the test
+// itself does not depend on the order).
+constexpr int kBoxV = 128;      // vertices (overflow: whole-domain box)
+constexpr int kBoxP = 128;      // 6 box planes + 122 neighbours
+constexpr int kNearMax = 128;   // longest list ranked (else kept as is)
+
+// inline neighbour word: the site id, with bit 31 set when the site is not
+// flagged (it bounds cells but has none of its own)
+constexpr uint32_t kNearUnflagged = 0x80000000u;
+__device__ __forceinline__ int32_t near_word(const DevSites& S, int m) {
+  return (int32_t)((uint32_t)m | (S.flags[m] == 1u ? 0u : kNearUnflagged));
+}
+__device__ __forceinline__ int near_id(int32_t w) { return w & 0x7fffffff; }
+
+__global__ __launch_bounds__(64) void k_site_bbox(DevSites S,
+                                                  const InstInfo* inst,
+                                                  const int32_t* site_inst,
+                                                  double* bbox,  // 6/site
+                                                  int32_t* knn_near,
+                                                  double4* knn_site_near,
+                                                  int32_t* n_fallback) {
+  __shared__ double4 s_pl[kBoxP];
+  __shared__ double4 s_X[2][kBoxV];
+  __shared__ uint32_t s_t[2][kBoxV];
+  __shared__ uint8_t s_out[kBoxV];
+  __shared__ double s_key[kNearMax];
+  __shared__ int32_t s_near[kNearMax];
+  __shared__ int32_t s_new;
+  const int i = blockIdx.x;
+  const int lane = threadIdx.x;
+  if (i >= S.n_site) return;
+  const InstInfo& I = inst[site_inst[i]];
+  const double* dom = I.dom;
+  const double rho = I.rho;
+  double* out = bbox + 6 * (int64_t)i;
+  if (S.flags[i] != 1u) {
+    if (lane == 0) {
+      out[0] = out[1] = out[2] = 1.0;
+      out[3] = out[4] = out[5] = -1.0;
+    }
+    return;
+  }
+  const int64_t k0 = S.knn_off[i];
+  const int deg = (int)(S.knn_off[i + 1] - k0);
+  bool fail = deg > kBoxP - 6;
+  const rpd_d4 si = ld4(S.site + i);
+  const bool ranked = deg <= kNearMax;
+  if (ranked) {
+    for (int k = lane; k < deg; k += 64) {
+      const rpd_d4 e = rpd_bisector(si, ld4(S.site + S.knn_ids[k0 + k]));
+      const double nn = e.x * e.x + e.y * e.y + e.z * e.z;
+      double key = (e.x * si.x + e.y * si.y + e.z * si.z + e.w) / sqrt(nn);
+      if (!(key == key)) key = -INFINITY;  // keep a strict total order
+      s_key[k] = key;
+    }
+    wsync();
+    // rank = position in ascending (key, index) order: a permutation
+    for (int k = lane; k < deg; k += 64) {
+      const double kk = s_key[k];
+      int r = 0;
+      for (int u = 0; u < deg; ++u) {
+        const double ku = s_key[u];
+        r += (ku < kk) || (ku == kk && u < k);
+      }
+      s_near[r] = S.knn_ids[k0 + k];
+    }
+    wsync();
+    for (int k = lane; k < deg; k += 64) {
+      const int m = s_near[k];
+      knn_near[k0 + k] = near_word(S, m);
+      knn_site_near[k0 + k] = S.site[m];
+    }
+  } else {
+    for (int k = lane; k < deg; k += 64) {
+      const int m = S.knn_ids[k0 + k];
+      knn_near[k0 + k] = near_word(S, m);
+      knn_site_near[k0 + k] = S.site[m];
+    }
+  }
+  // box planes: x >= x0, x <= x1, y >= y0, y <= y1, z >= z0, z <= z1
+  if (lane < 6) {
+    int a = lane >> 1;
+    double4 p = make_double4(0, 0, 0, 0);
+    double* pp = &p.x;
+    if ((lane & 1) == 0) {
+      pp[a] = 1.0;
+      p.w = -dom[a];
+    } else {
+      pp[a] = -1.0;
+      p.w = dom[3 + a];
+    }
+    s_pl[lane] = p;
+  }
+  wsync();
+  int nv = 8, cur = 0;
+  if (lane < 8) {
+    int a = lane & 1, b = 2 + ((lane >> 1) & 1), c = 4 + ((lane >> 2) & 1);
+    rpd_d4 X, Q;
+    rpd_vertex_homog(ld4(&s_pl[a]), ld4(&s_pl[b]), ld4(&s_pl[c]), X, Q);
+    s_X[0][lane] = make_double4(X.x, X.y, X.z, X.w);
+    s_t[0][lane] = a | (b << 10) | (c << 20);
+  }
+  wsync();
+  bool empty = false;
+  for (int k = 0; k < deg && !fail && !empty; ++k) {
+    const int m = ranked ? s_near[k] : S.knn_ids[k0 + k];
+    rpd_d4 e = rpd_bisector(si, ld4(S.site + m));
+    double nrm = sqrt(e.x * e.x + e.y * e.y + e.z * e.z);
+    e.w += nrm * rho;
+    const int p = 6 + k;
+    if (lane == 0) s_pl[p] = make_double4(e.x, e.y, e.z, e.w);
+    int n_out = 0;
+    for (int v = lane; v < nv; v += 64) {
+      double4 X = s_X[cur][v];
+      double s = e.x * X.x + e.y * X.y + e.z * X.z + e.w * X.w;
+      bool o = (s < 0 && X.w > 0) || (s > 0 && X.w < 0);
+      s_out[v] = o;
+    }
+    wsync();
+    for (int v0 = 0; v0 < nv; v0 += 64) {
+      int v = v0 + lane;
+      n_out += __popcll(ballot(v < nv && s_out[v]));
+    }
+    if (n_out == 0) continue;
+    if (n_out == nv) {
+      empty = true;
+      break;
+    }
+    if (lane == 0) s_new = 0;
+    wsync();
+    const int nxt = cur ^ 1;
+    const int n_keep = nv - n_out;
+    // compact kept vertices in order
+    int base = 0;
+    for (int v0 = 0; v0 < nv; v0 += 64) {
+      int v = v0 + lane;
+      bool keep = v < nv && !s_out[v];
+      uint64_t bm = ballot(keep);
+      if (keep) {
+        int pos = base + __popcll(bm & ((1ull << lane) - 1));
+        s_X[nxt][pos] = s_X[cur][v];
+        s_t[nxt][pos] = s_t[cur][v];
+      }
+      base += __popcll(bm);
+    }
+    // new vertices on edges between removed and kept vertices
+    bool lfail = false;
+    for (int v = lane; v < nv; v += 64) {
+      if (!s_out[v]) continue;
+      uint32_t tv = s_t[cur][v];
+      int pv[3] = {(int)(tv & 1023), (int)((tv >> 10) & 1023),
+                   (int)((tv >> 20) & 1023)};
+      for (int q = 0; q < 3; ++q) {
+        int a = pv[q], b = pv[(q + 1) % 3];
+        int other = -1;
+        for (int u = 0; u < nv; ++u) {
+          if (u == v) continue;
+          uint32_t tu = s_t[cur][u];
+          int u0 = tu & 1023, u1 = (tu >> 10) & 1023, u2 = (tu >> 20) & 1023;
+          bool ha = u0 == a || u1 == a || u2 == a;
+          bool hb = u0 == b || u1 == b || u2 == b;
+          if (ha && hb) {
+            other = u;
+            break;
+          }
+        }
+        if (other < 0) {
+          lfail = true;
+          continue;
+        }
+        if (s_out[other]) continue;
+        int slot = atomicAdd(&s_new, 1);
+        if (n_keep + slot >= kBoxV) {
+          lfail = true;
+          continue;
+        }
+        rpd_d4 X, Q;
+        rpd_vertex_homog(ld4(&s_pl[a]), ld4(&s_pl[b]), ld4(&s_pl[p]), X, Q);
+        s_X[nxt][n_keep + slot] = make_double4(X.x, X.y, X.z, X.w);
+        s_t[nxt][n_keep + slot] = a | (b << 10) | (p << 20);
+      }
+    }
+    fail = fail || (ballot(lfail) != 0);
+    wsync();
+    nv = n_keep + min(s_new, kBoxV - n_keep);
+    cur = nxt;
+    wsync();
+  }
+  if (fail) {
+    if (lane == 0) {
+      for (int a = 0; a < 6; ++a) out[a] = dom[a];
+      atomicAdd(n_fallback, 1);
+    }
+    return;
+  }
+  if (empty) {
+    if (lane == 0) {
+      out[0] = out[1] = out[2] = 1.0;
+      out[3] = out[4] = out[5] = -1.0;
+    }
+    return;
+  }
+  double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+  for (int v = lane; v < nv; v += 64) {
+    double4 X = s_X[cur][v];
+    double x = X.x / X.w, y = X.y / X.w, z = X.z / X.w;
+    lo[0] = fmin(lo[0], x);
+    lo[1] = fmin(lo[1], y);
+    lo[2] = fmin(lo[2], z);
+    hi[0] = fmax(hi[0], x);
+    hi[1] = fmax(hi[1], y);
+    hi[2] = fmax(hi[2], z);
+  }
+  for (int off = 32; off > 0; off >>= 1)
+    for (int a = 0; a < 3; ++a) {
+      lo[a] = fmin(lo[a], __shfl_xor(lo[a], off));
+      hi[a] = fmax(hi[a], __shfl_xor(hi[a], off));
+    }
+  if (lane == 0) {
+    double ext = fmax(fmax(dom[3] - dom[0], dom[4] - dom[1]), dom[5] - dom[2]);
+    double eps = 1e-7 * ext;  // covers the rounding of the vertices
+    for (int a = 0; a < 3; ++a) {
+      out[a] = lo[a] - eps;
+      out[3 + a] = hi[a] + eps;
+    }
+  }
+}
+
+// bin range of a sphere's candidate box; false if empty
+__device__ __forceinline__ bool bin_range(const double* b, const BinGrid& g,
+                                          int r[6]) {
+  if (b[0] > b[3] || b[1] > b[4] || b[2] > b[5]) return false;
+  for (int a = 0; a < 3; ++a) {
+    r[a] = bin_coord(b[a], g.org[a], g.inv_bs, g.dim[a]);
+    r[3 + a] = bin_coord(b[3 + a], g.org[a], g.inv_bs, g.dim[a]);
+  }
+  return true;
+}
+
+// number of bins each sphere registers into
+__global__ __launch_bounds__(256) void k_bin_nreg(int32_t n_site,
+                                                  const double* bbox,
+                                                  const InstInfo* inst,
+                                                  const int32_t* site_inst,
+                                                  int64_t* nreg) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i > n_site) return;
+  if (i == n_site) {
+    nreg[i] = 0;
+    return;
+  }
+  int r[6];
+  nreg[i] = bin_range(bbox + 6 * (int64_t)i, inst[site_inst[i]].g, r)
+                ? (int64_t)(r[3] - r[0] + 1) * (r[4] - r[1] + 1) *
+                      (r[5] - r[2] + 1)
+                : 0;
+}
+
+// one thread per registration: key = bin << 32 | sphere
+__global__ __launch_bounds__(256) void k_bin_expand(int32_t n_site,
+                                                    int64_t n_reg,
+                                                    const double* bbox,
+                                                    const InstInfo* inst,
+                                                    const int32_t* site_inst,
+                                                    const int64_t* reg_off,
+                                                    uint64_t* keys,
+                                                    const int64_t* n_reg_dev,
+                                                    uint64_t pad) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n_reg) return;
+  if (n_reg_dev && q >= dev_count(n_reg, n_reg_dev)) {
+    keys[q] = pad;  // sorts after every registration
+    return;
+  }
+  // sphere i with reg_off[i] <= q < reg_off[i+1]
+  int lo = 0, hi = n_site;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (reg_off[mid] <= q)
+      lo = mid;
+    else
+      hi = mid;
+  }
+  const int i = lo;
+  const InstInfo& I = inst[site_inst[i]];
+  const BinGrid& g = I.g;
+  int r[6];
+  bin_range(bbox + 6 * (int64_t)i, g, r);
+  const int64_t k = q - reg_off[i];
+  const int64_t nx = r[3] - r[0] + 1, ny = r[4] - r[1] + 1;
+  const int64_t x = r[0] + k % nx, y = r[1] + (k / nx) % ny,
+                z = r[2] + k / (nx * ny);
+  const uint64_t bin = (uint64_t)I.bin_base + x +
+                       (uint64_t)g.dim[0] * (y + (uint64_t)g.dim[1] * z);
+  keys[q] = (bin << 32) | (uint32_t)i;
+}
+
+// bin_start[b] = first registration of bin >= b in the sorted keys
+__global__ __launch_bounds__(256) void k_bin_starts(int64_t n_bins,
+                                                    int64_t n_reg_cap,
+                                                    const uint64_t* keys,
+                                                    int32_t* bin_start,
+                                                    int32_t* bin_ids,
+                                                    const int64_t* n_reg_dev) {
+  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t n_reg = dev_count(n_reg_cap, n_reg_dev);
+  if (b < n_reg) bin_ids[b] = (int32_t)(keys[b] & 0xffffffffu);
+  if (b > n_bins) return;
+  int64_t lo = 0, hi = n_reg;  // first index with key >> 32 >= b
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) >> 1;
+    if ((int64_t)(keys[mid] >> 32) < b)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  bin_start[b] = (int32_t)lo;
+}
+
+struct TetLoad {
+  double4 V[4];
+  int4 tv;
+};
+
+__device__ __forceinline__ void load_tet(const DevMesh& M, int t,
+                                         TetLoad& L) {
+  L.tv = M.tet_v[t];
+  L.V[0] = M.vert[L.tv.x];
+  L.V[1] = M.vert[L.tv.y];
+  L.V[2] = M.vert[L.tv.z];
+  L.V[3] = M.vert[L.tv.w];
+}
+
+// reference relation test (voronoi.cu:154-193) in binary64: sphere i
+// relates to the tet iff for every neighbour m some corner v has
+// pd(v, m) > pd(v, i).  The neighbours are visited nearest bisector first
+// (the outcome does not depend on the order), their spheres read inline,
+// one ahead.  *iters counts the neighbour tests made.
+__device__ __forceinline__ bool relation(const DevSites& S, const TetLoad& L,
+                                         int i, uint32_t* iters) {
+  if (S.flags[i] != 1u) return false;
+  const rpd_d4 si = ld4(S.site + i);
+  double pdi[4];
+  for (int k = 0; k < 4; ++k)
+    pdi[k] = rpd_power_dist(L.V[k].x, L.V[k].y, L.V[k].z, si);
+  const int64_t k0 = S.knn_off[i], k1 = S.knn_off[i + 1];
+  if (k0 == k1) return true;
+  double4 nxt = S.knn_site_near[k0];
+  for (int64_t q = k0; q < k1; ++q) {
+    const rpd_d4 sm{nxt.x, nxt.y, nxt.z, nxt.w};
+    if (q + 1 < k1) nxt = S.knn_site_near[q + 1];
+    ++*iters;
+    bool ok = false;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      ok = ok || rpd_power_dist(L.V[k].x, L.V[k].y, L.V[k].z, sm) > pdi[k];
+    if (!ok) return false;
+  }
+  return true;
+}
+
+__device__ __forceinline__ void tet_centroid(const TetLoad& L, double c[3]) {
+  c[0] = (((L.V[0].x + L.V[1].x) + L.V[2].x) + L.V[3].x) * 0.25;
+  c[1] = (((L.V[0].y + L.V[1].y) + L.V[2].y) + L.V[3].y) * 0.25;
+  c[2] = (((L.V[0].z + L.V[1].z) + L.V[2].z) + L.V[3].z) * 0.25;
+}
+
+__device__ __forceinline__ int64_t tet_bin(const double c[3],
+                                           const BinGrid& g) {
+  int x = bin_coord(c[0], g.org[0], g.inv_bs, g.dim[0]);
+  int y = bin_coord(c[1], g.org[1], g.inv_bs, g.dim[1]);
+  int z = bin_coord(c[2], g.org[2], g.inv_bs, g.dim[2]);
+  return x + (int64_t)g.dim[0] * (y + (int64_t)g.dim[1] * z);
+}
+
+__global__ __launch_bounds__(256) void k_tet_count(DevMesh M, DevSites S,
+                                                   const InstInfo* inst,
+                                                   const int32_t* tet_inst,
+                                                   const int32_t* bin_start,
+                                                   const int32_t* bin_ids,
+                                                   int64_t* tet_count,
+                                                   uint64_t* tet_pass,
+                                                   unsigned long long* work,
+                                                   const uint8_t* tet_sel) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= M.n_tet) return;
+  if (tet_sel && !tet_sel[t]) {  // outside the tet subset: no candidates
+    tet_count[t] = 0;
+    return;
+  }
+  TetLoad L;
+  load_tet(M, t, L);
+  double c[3];
+  tet_centroid(L, c);
+  const InstInfo& I = inst[tet_inst[t]];
+  const int64_t b = I.bin_base + tet_bin(c, I.g);
+  int64_t n = 0;
+  // bit r of (pass0, pass1): the r-th site of the bin list relates
+  uint64_t pass0 = 0, pass1 = 0;
+  uint32_t iters = 0;
+  const int q0 = bin_start[b], q1 = bin_start[b + 1];
+  for (int q = q0; q < q1; ++q) {
+    const int i = bin_ids[q];
+    // (the candidate-box test of the centroid is left to the binning: it
+    // passes 3 of 4 entries and costs more than it saves)
+    const bool r = relation(S, L, i, &iters);
+    n += r;
+    const int d = q - q0;
+    if (r && d < 64) pass0 |= 1ull << d;
+    if (r && d >= 64 && d < 128) pass1 |= 1ull << (d - 64);
+  }
+  tet_count[t] = n;
+  tet_pass[t] = pass0;
+  tet_pass[(int64_t)M.n_tet + t] = pass1;
+  if (work) {  // entries, neighbour tests (count_work)
+    unsigned long long* w = work + 4 * (blockIdx.x & 63);
+    atomicAdd(w + 0, (unsigned long long)(q1 - q0));
+
+    atomicAdd(w + 1, (unsigned long long)iters);
+  }
+}
+
+__global__ __launch_bounds__(256) void k_tet_fill(
+    DevMesh M, DevSites S, const InstInfo* inst, const int32_t* tet_inst,
+    const int32_t* bin_start, const int32_t* bin_ids, const int64_t* tet_off,
+    const uint64_t* tet_pass, Cand* cand, int32_t* rel_ids,
+    const uint8_t* tet_sel, int64_t cap, int32_t* overflow) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= M.n_tet) return;
+  if (tet_sel && !tet_sel[t]) return;
+  // over a captured pipeline's capacity: the entries below it are still
+  // written (every slot a later launch reads holds a pair of this run)
+  if (tet_off[t + 1] > cap && (tet_off[t] < cap || t == 0)) overflow[0] = 1;
+  if (tet_off[t] >= cap) return;
+  TetLoad L;
+  load_tet(M, t, L);
+  double c[3];
+  tet_centroid(L, c);
+  const InstInfo& I = inst[tet_inst[t]];
+  const int64_t b = I.bin_base + tet_bin(c, I.g);
+  int64_t o = tet_off[t];
+  const uint64_t pass0 = tet_pass[t];
+  const uint64_t pass1 = tet_pass[(int64_t)M.n_tet + t];
+  const int q0 = bin_start[b];
+  for (int q = q0; q < bin_start[b + 1]; ++q) {
+    const int i = bin_ids[q];
+    // the first 128 outcomes come from the counting pass
+    uint32_t iters = 0;
+    const int d = q - q0;
+    const bool r = d < 64    ? ((pass0 >> d) & 1)
+                   : d < 128 ? ((pass1 >> (d - 64)) & 1)
+                             : relation(S, L, i, &iters);
+    if (!r) continue;
+    if (o >= cap) break;
+    Cand c;
+    c.tet = t;
+    c.seed = i;
+    c.m0 = 0;
+    c.m1 = 0;
+    cand[o] = c;
+    rel_ids[o] = i;
+    ++o;
+  }
+}
+
+// the bisector table of the neighbour lists: one wavefront per site
+__global__ __launch_bounds__(64) void k_knn_bis(DevSites S, double4* bis,
+                                                float4* bisf) {
+  const int i = blockIdx.x;
+  const int64_t k0 = S.knn_off[i], k1 = S.knn_off[i + 1];
+  const rpd_d4 si = ld4(S.site + i);
+  for (int64_t q = k0 + threadIdx.x; q < k1; q += 64) {
+    const int m = S.knn_ids[q];
+    double4 e = make_double4(0, 0, 0, 0);
+    if (m >= 0) {
+      const rpd_d4 b = rpd_bisector(si, ld4(S.site + m));
+      e = make_double4(b.x, b.y, b.z, b.w);
+    }
+    bis[q] = e;
+    bisf[q] = make_float4(rpd_mask_coef(e.x), rpd_mask_coef(e.y),
+                          rpd_mask_coef(e.z), rpd_mask_coef(e.w));
+  }
+}
+
+// The tet's four corners as the clip kernel's initial vertices: homogeneous
+// coordinates X and cofactor magnitudes Q of the dual triangles (1,3,2),
+// (0,2,3), (0,3,1), (0,1,2) of its binary64 face planes; sQ = the sum of
+// a corner's four magnitudes.
+struct CornerFrames {
+  rpd_d4 X[4];
+  double sQ[4];
+  // dot(e, X~) is certainly negative (no conflict) at all four corners, so
+  // the plane e cannot cut any state of a cell of this tet (every vertex of
+  // the cell lies in the convex hull of the corners); decided from the
+  // binary32 table entry f of e (rpd_mask_negative), one 16-byte load per
+  // plane.  The few planes it leaves undecided that a tighter test would
+  // skip are only clipped without effect.
+  __device__ __forceinline__ bool inactive(const float4& f) const {
+    return rpd_mask_negative(f.x, f.y, f.z, f.w, X, sQ);
+  }
+};
+__device__ __forceinline__ void corner_frames(const TetLoad& L,
+                                              CornerFrames& F) {
+  rpd_d4 pl[4], Q[4];
+  tet_planes(L.V, pl);
+  rpd_vertex_homog(pl[1], pl[3], pl[2], F.X[0], Q[0]);
+  rpd_vertex_homog(pl[0], pl[2], pl[3], F.X[1], Q[1]);
+  rpd_vertex_homog(pl[0], pl[3], pl[1], F.X[2], Q[2]);
+  rpd_vertex_homog(pl[0], pl[1], pl[2], F.X[3], Q[3]);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) F.sQ[k] = ((Q[k].x + Q[k].y) + Q[k].z) + Q[k].w;
+}
+// a cell's number of clip steps: mask bits, plus the list positions past
+// 128 (always clipped), saturated to a byte
+__device__ __forceinline__ uint8_t clip_steps(uint64_t m0, uint64_t m1,
+                                              int deg) {
+  const int n = __popcll(m0) + __popcll(m1) + (deg > 128 ? deg - 128 : 0);
+  return (uint8_t)(n < 255 ? n : 255);
+}
+
+// One thread per candidate cell: bit k of the mask is set unless the k-th
+// neighbour's bisector is certainly positive at all four corners of the
+// tet cell (then it cannot cut any state of the cell: every cell vertex
+// lies in the convex hull of the corners).
+// With trips != nullptr it also writes each cell's number of clip steps
+// (mask bits below the degree, plus the positions past 128) and its index
+// c0 + c for the step-count ordering of the clip launch.
+__global__ __launch_bounds__(256) void k_cand_mask(DevMesh M, DevSites S,
+                                                   int64_t n_cand,
+                                                   Cand* cand,
+                                                   uint8_t* trips,
+                                                   int32_t* trip_ids,
+                                                   int64_t c0,
+                                                   const int64_t* n_dev) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= n_cand) return;
+  if (n_dev && c >= dev_count(n_cand, n_dev, c0)) {
+    if (trips) {  // past the count: sorts after every cell
+      trips[c] = 0;
+      trip_ids[c] = (int32_t)(c0 + c);
+    }
+    return;
+  }
+  const int t = cand[c].tet, i = cand[c].seed;
+  TetLoad L;
+  load_tet(M, t, L);
+  CornerFrames F;
+  corner_frames(L, F);
+  const int64_t k0 = S.knn_off[i];
+  const int deg = (int)(S.knn_off[i + 1] - k0);
+  uint64_t m0 = 0, m1 = 0;
+  const int lim = deg < 128 ? deg : 128;
+  // the next plane's load is issued before this plane's test (the test's
+  // corner branches keep the compiler from hoisting it)
+  float4 nxt = lim > 0 ? S.knn_bisf[k0] : make_float4(0, 0, 0, 0);
+  for (int k = 0; k < lim; ++k) {
+    const float4 f = nxt;
+    if (k + 1 < lim) nxt = S.knn_bisf[k0 + k + 1];
+    if (!F.inactive(f)) {
+      if (k < 64)
+        m0 |= 1ull << k;
+      else
+        m1 |= 1ull << (k - 64);
+    }
+  }
+  cand[c].m0 = m0;
+  cand[c].m1 = m1;
+  if (trips) {
+    trips[c] = clip_steps(m0, m1, deg);
+    trip_ids[c] = (int32_t)(c0 + c);
+  }
+}
+
+// ========================================================== compaction
+// per cell: location of its final slot; tier 0 small (index = cell),
+// tier 1 large / 2 exact (index = re-run position)
+__global__ __launch_bounds__(256) void k_mark_rerun(const int32_t* list,
+                                                    int32_t r0, int32_t r1,
+                                                    int32_t tier,
+                                                    int32_t* loc,
+                                                    const int32_t* r1_dev) {
+  const int r = r0 + blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= (r1_dev ? min(r1, *r1_dev) : r1)) return;
+  loc[list[r]] = (tier << 28) | r;
+}
+
+struct Sizes3 {
+  int64_t cells, words, areas;
+};
+struct Sizes3Sum {
+  __host__ __device__ Sizes3 operator()(const Sizes3& a,
+                                        const Sizes3& b) const {
+    return Sizes3{a.cells + b.cells, a.words + b.words, a.areas + b.areas};
+  }
+};
+
+struct TierViews {
+  SlotView t[4];  // small, full capacity, exact, middle
+};
+
+// Compaction in blocks of kCB consecutive output positions r (cell
+// perm[r], or r when perm is null).  A cell's sizes pack into one u64
+// (cells in bits 0-15, areas 16-35, words 36-63), so one integer sum
+// scans all three: a block holds at most 256 cells, 256 x 64 areas and
+// 256 x 312 words.
+constexpr int kCB = 256;
+
+struct CellRef {
+  int tier;
+  int64_t idx;
+  uint32_t hdr;
+};
+
+__device__ __forceinline__ CellRef cell_ref(int64_t r, const int32_t* perm,
+                                            const int32_t* loc,
+                                            const TierViews& tv) {
+  const int64_t c = perm ? perm[r] : r;
+  const int32_t l = loc[c];
+  CellRef x;
+  x.tier = l >> 28;
+  x.idx = x.tier ? (l & ((1 << 28) - 1)) : c;
+  x.hdr = tv.t[x.tier].hdr[x.idx];
+  return x;
+}
+
+__device__ __forceinline__ uint64_t packed_size(uint32_t hd) {
+  if ((hd >> 24) != RPD_SUCCESS) return 0;
+  const uint64_t nv = hd & 255, np = (hd >> 8) & 255, ne = (hd >> 16) & 255;
+  return 1ull | (np << 16) | ((nv + np + ne) << 36);
+}
+
+// per block: totals of its cells (bsum[b]) and the dropped cells by status
+// per-status counts of the cells not emitted, spread over kDropSlots copies
+// of the 9 counters (a block adds to copy blockIdx % kDropSlots) so that
+// the blocks' atomics do not all meet at one address
+constexpr int kDropSlots = 64;
+__global__ __launch_bounds__(kCB) void k_block_sizes(int64_t n_cells,
+                                                     const int32_t* perm,
+                                                     const int32_t* loc,
+                                                     TierViews tv,
+                                                     Sizes3* bsum,
+                                                     int64_t* drops,
+                                                     const int64_t* n_dev) {
+  typedef hipcub::BlockReduce<uint64_t, kCB> Red;
+  n_cells = dev_count(n_cells, n_dev);
+  __shared__ typename Red::TempStorage tmp;
+  __shared__ int32_t h[9];
+  if (threadIdx.x < 9) h[threadIdx.x] = 0;
+  __syncthreads();
+  const int64_t r = (int64_t)blockIdx.x * kCB + threadIdx.x;
+  uint64_t z = 0;
+  if (r < n_cells) {
+    const CellRef x = cell_ref(r, perm, loc, tv);
+    const uint32_t st = x.hdr >> 24;
+    z = packed_size(x.hdr);
+    if (st != RPD_SUCCESS && st < 9) atomicAdd(&h[st], 1);
+  }
+  const uint64_t tot = Red(tmp).Sum(z);
+  if (threadIdx.x == 0)
+    bsum[blockIdx.x] = Sizes3{(int64_t)(tot & 0xffff),
+                              (int64_t)(tot >> 36),
+                              (int64_t)((tot >> 16) & 0xfffff)};
+  __syncthreads();
+  if (threadIdx.x < 9 && h[threadIdx.x])
+    atomicAdd((unsigned long long*)&drops[9 * (blockIdx.x % kDropSlots) +
+                                          threadIdx.x],
+              (unsigned long long)h[threadIdx.x]);
+}
+
+// block b writes its cells from boff[b] on: cell records and geometry one
+// per thread, payload words and areas by the whole block over the block's
+// contiguous output range (each output element finds its cell by binary
+// search in the block's offsets), so every store is coalesced.
+__global__ __launch_bounds__(kCB) void k_compact(
+    int64_t n_cells, const int32_t* perm, const Cand* cand,
+    const int32_t* loc, TierViews tv, const Sizes3* boff, rpd_cell* out_cells,
+    uint32_t* out_words, double* out_geom, double* out_areas,
+    int32_t geometry, const int64_t* n_dev, Sizes3 cap, int32_t* overflow) {
+  typedef hipcub::BlockScan<uint64_t, kCB> Scan;
+  __shared__ typename Scan::TempStorage tmp;
+  __shared__ uint32_t s_w[kCB + 1];
+  __shared__ uint32_t s_a[kCB + 1];
+  __shared__ const uint32_t* s_wsrc[kCB];
+  __shared__ const double* s_asrc[kCB];
+  // a slot holds the edges at 0 and the vertices and plane sources after
+  // them; the stream holds vertices, plane sources, edges
+  __shared__ uint32_t s_lay[kCB];  // nb_v | nb_p << 8 | nb_e << 16
+  const int i = threadIdx.x;
+  const int64_t r = (int64_t)blockIdx.x * kCB + i;
+  n_cells = dev_count(n_cells, n_dev);
+  {  // a captured pipeline's output capacity: the block's whole range
+    const Sizes3 B0 = boff[blockIdx.x], B1 = boff[blockIdx.x + 1];
+    if (B1.cells > cap.cells || B1.words > cap.words ||
+        B1.areas > cap.areas) {
+      if (i == 0) overflow[0] = 1;
+      return;
+    }
+    (void)B0;
+  }
+  CellRef x{0, 0, 0};
+  int64_t c = 0;
+  uint64_t z = 0;
+  if (r < n_cells) {
+    c = perm ? perm[r] : r;
+    x = cell_ref(r, perm, loc, tv);
+    z = packed_size(x.hdr);
+  }
+  uint64_t off, tot;
+  Scan(tmp).ExclusiveSum(z, off, tot);
+  const Sizes3 B = boff[blockIdx.x];
+  const uint32_t w_off = (uint32_t)(off >> 36);
+  const uint32_t a_off = (uint32_t)((off >> 16) & 0xfffff);
+  const int64_t c_off = B.cells + (int64_t)(off & 0xffff);
+  s_w[i] = w_off;
+  s_a[i] = a_off;
+  if (i == 0) {
+    s_w[kCB] = (uint32_t)(tot >> 36);
+    s_a[kCB] = (uint32_t)((tot >> 16) & 0xfffff);
+  }
+  const SlotView& sv = tv.t[x.tier];
+  s_wsrc[i] = sv.words + x.idx * sv.stride_words;
+  s_asrc[i] = sv.areas + x.idx * sv.stride_areas;
+  s_lay[i] = x.hdr & 0xffffffu;
+  if (z) {
+    rpd_cell rc;
+    rc.tet_id = cand[c].tet;
+    rc.seed = cand[c].seed;
+    rc.nb_v = (uint8_t)(x.hdr & 255);
+    rc.nb_p = (uint8_t)((x.hdr >> 8) & 255);
+    rc.nb_e = (uint8_t)((x.hdr >> 16) & 255);
+    rc.status = RPD_SUCCESS;
+    rc.reserved = 0;
+    rc.word_off = (uint64_t)(B.words + w_off);
+    rc.area_off = (uint64_t)(B.areas + a_off);
+    out_cells[c_off] = rc;
+    if (geometry) {
+      const double* gs = sv.geom + 4 * x.idx;
+      double* gd = out_geom + 4 * c_off;
+      gd[0] = gs[0];
+      gd[1] = gs[1];
+      gd[2] = gs[2];
+      gd[3] = gs[3];
+    }
+  }
+  __syncthreads();
+  // the cell holding element e: the last k with s[k] <= e (cells without
+  // output have s[k] == s[k + 1] and are skipped by "last")
+  auto owner = [](const uint32_t* sa, uint32_t e) {
+    int lo = 0, hi = kCB;  // sa[lo] <= e < sa[hi]
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (sa[mid] <= e)
+        lo = mid;
+      else
+        hi = mid;
+    }
+    return lo;
+  };
+  // Each wavefront copies a contiguous quarter of the block's elements, 64
+  // consecutive ones per step (coalesced stores); a lane finds the cell of
+  // its first element by binary search and then walks forward, past about
+  // 64 / (elements per cell) cells a step.  kU steps at a time: their
+  // sources first, then their loads together, then their stores.
+  constexpr int kU = 4;
+  const int wv = i >> 6, ln = i & 63;
+  auto range = [&](uint32_t n, uint32_t* q0, uint32_t* q1) {
+    *q0 = (uint32_t)((uint64_t)n * wv / (kCB / 64));
+    *q1 = (uint32_t)((uint64_t)n * (wv + 1) / (kCB / 64));
+  };
+  const uint32_t W = s_w[kCB];
+  uint32_t* wd = out_words + B.words;
+  {
+    uint32_t q0, q1;
+    range(W, &q0, &q1);
+    int k = q0 + ln < q1 ? owner(s_w, q0 + ln) : 0;
+    for (uint32_t e0 = q0 + ln; e0 < q1; e0 += 64 * kU) {
+      const uint32_t* src[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const uint32_t e = e0 + 64 * u;
+        src[u] = nullptr;
+        if (e < q1) {
+          while (s_w[k + 1] <= e) ++k;
+          const uint32_t w = e - s_w[k], lay = s_lay[k];
+          const uint32_t nvp = (lay & 255) + ((lay >> 8) & 255);
+          src[u] = s_wsrc[k] + (w < nvp ? (lay >> 16) + w : w - nvp);
+        }
+      }
+      uint32_t v[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) v[u] = src[u] ? *src[u] : 0u;
+#pragma unroll
+      for (int u = 0; u < kU; ++u)
+        if (src[u]) wd[e0 + 64 * u] = v[u];
+    }
+  }
+  if (geometry) {
+    const uint32_t A = s_a[kCB];
+    double* ad = out_areas + B.areas;
+    uint32_t q0, q1;
+    range(A, &q0, &q1);
+    int k = q0 + ln < q1 ? owner(s_a, q0 + ln) : 0;
+    for (uint32_t e0 = q0 + ln; e0 < q1; e0 += 64 * kU) {
+      const double* src[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const uint32_t e = e0 + 64 * u;
+        src[u] = nullptr;
+        if (e < q1) {
+          while (s_a[k + 1] <= e) ++k;
+          src[u] = s_asrc[k] + (e - s_a[k]);
+        }
+      }
+      double v[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) v[u] = src[u] ? *src[u] : 0.0;
+#pragma unroll
+      for (int u = 0; u < kU; ++u)
+        if (src[u]) ad[e0 + 64 * u] = v[u];
+    }
+  }
+}
+
+// active-plane statistics of the candidate masks
+__global__ __launch_bounds__(256) void k_mask_stats(int64_t n, const Cand* cand,
+                                                    DevSites S,
+                                                    unsigned long long* acc) {
+  __shared__ unsigned long long s_a, s_b;
+  if (threadIdx.x == 0) s_a = s_b = 0;
+  __syncthreads();
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c < n) {
+    const Cand cd = cand[c];
+    const int64_t deg = S.knn_off[cd.seed + 1] - S.knn_off[cd.seed];
+    int64_t act = __popcll(cd.m0) + __popcll(cd.m1);
+    if (deg > 128) act += deg - 128;
+    atomicAdd(&s_a, (unsigned long long)act);
+    atomicAdd(&s_b, (unsigned long long)deg);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    atomicAdd(&acc[0], s_a);
+    atomicAdd(&acc[1], s_b);
+  }
+}
+
+}  // namespace rpd
