@@ -23,6 +23,7 @@
 #include "rpd_device.h"
 #include "rpd_prep.h"
 #include "../common/rpd_classgrid.h"
+#include "../common/rpd_nbrlist.h"
 #include "rpd_stages.hip"
 #include "rpd_learn.hip"
 #include "rpd_nbr.hip"
@@ -272,6 +273,9 @@ struct rpd_ctx {
   Buf edg_ka, edg_kb, edg_va, edg_vb, edg_par, edg_flag, edg_pos, edg_start,
       edg_runs, edg_rec;
   Buf site_cells, site_cc, site_eul, adj_soff, adj_eul_s, adj_root_s;
+  // neighbour builder
+  Buf nb_sph, nb_box, nb_start, nb_ids, nb_valid, nb_cnt, nb_lists, nb_rerun,
+      nb_cnt64, nb_off, nb_pack, nb_cellw;
   rpd_adj_sizes adj{};
   bool adj_ready = false;
   RunCaps seen{};  // sizes of the last eager plain run
@@ -2880,6 +2884,7 @@ int rpd_power_neighbors_gpu(rpd_ctx* ctx, int32_t n, const double* xyzw,
   NbGrids G{};
   std::vector<int64_t> starts;
   std::vector<int32_t> ids;
+  std::vector<float> cell_w;
   for (int c = 0; c < kRpdClasses; ++c) {
     const RpdClassGrid& g = grids[c];
     NbGrid& d = G.g[c];
@@ -2893,51 +2898,110 @@ int rpd_power_neighbors_gpu(rpd_ctx* ctx, int32_t n, const double* xyzw,
     d.wmax = g.wmax;
     d.cell_base = (int64_t)starts.size();
     const int64_t id_base = (int64_t)ids.size();
-    for (int64_t v : g.start) starts.push_back(id_base + v);
+    for (size_t q = 0; q < g.start.size(); ++q) {
+      // the cell's largest weight, rounded up to binary32
+      double w = 0;
+      if (q + 1 < g.start.size())
+        for (int64_t v = g.start[q]; v < g.start[q + 1]; ++v)
+          w = std::max(w, xyzw[4 * (int64_t)g.ids[v] + 3]);
+      starts.push_back(id_base + g.start[q]);
+      cell_w.push_back(std::nextafter((float)w, INFINITY));
+    }
     ids.insert(ids.end(), g.ids.begin(), g.ids.end());
   }
-  Buf d_sph, d_box, d_start, d_ids, d_valid, d_cnt, d_lists;
   const int64_t nn = std::max<int32_t>(n, 1);
-  HIP_TRY(d_sph.need(nn * 32));
-  HIP_TRY(d_box.need(6 * 8));
-  HIP_TRY(d_start.need(std::max<size_t>(starts.size(), 1) * 8));
-  HIP_TRY(d_ids.need(std::max<size_t>(ids.size(), 1) * 4));
-  HIP_TRY(d_valid.need(nn * 4));
-  HIP_TRY(d_cnt.need(nn * 4));
-  HIP_TRY(d_lists.need(nn * kNbOut * 4));
-  HIP_TRY(hipMemcpyAsync(d_sph.p, xyzw, (size_t)n * 32, hipMemcpyHostToDevice,
-                         s));
-  HIP_TRY(hipMemcpyAsync(d_box.p, box, 6 * 8, hipMemcpyHostToDevice, s));
+  HIP_TRY(ctx->nb_sph.need(nn * 32));
+  HIP_TRY(ctx->nb_box.need(6 * 8));
+  HIP_TRY(ctx->nb_start.need(std::max<size_t>(starts.size(), 1) * 8));
+  HIP_TRY(ctx->nb_ids.need(std::max<size_t>(ids.size(), 1) * 4));
+  HIP_TRY(ctx->nb_valid.need(nn * 4));
+  HIP_TRY(ctx->nb_cnt.need(nn * 4));
+  HIP_TRY(ctx->nb_lists.need(nn * kNbOut * 4));
+  HIP_TRY(ctx->nb_rerun.need((nn + 2) * 4));  // 2 counters, then the list
+  HIP_TRY(ctx->nb_cnt64.need((nn + 1) * 8));
+  HIP_TRY(ctx->nb_off.need((nn + 1) * 8));
+  HIP_TRY(hipMemcpyAsync(ctx->nb_sph.p, xyzw, (size_t)n * 32,
+                         hipMemcpyHostToDevice, s));
+  HIP_TRY(hipMemcpyAsync(ctx->nb_box.p, box, 6 * 8, hipMemcpyHostToDevice, s));
   if (!starts.empty())
-    HIP_TRY(hipMemcpyAsync(d_start.p, starts.data(), starts.size() * 8,
+    HIP_TRY(hipMemcpyAsync(ctx->nb_start.p, starts.data(), starts.size() * 8,
+                           hipMemcpyHostToDevice, s));
+  HIP_TRY(ctx->nb_cellw.need(std::max<size_t>(cell_w.size(), 1) * 4));
+  if (!cell_w.empty())
+    HIP_TRY(hipMemcpyAsync(ctx->nb_cellw.p, cell_w.data(), cell_w.size() * 4,
                            hipMemcpyHostToDevice, s));
   if (!ids.empty())
-    HIP_TRY(hipMemcpyAsync(d_ids.p, ids.data(), ids.size() * 4,
+    HIP_TRY(hipMemcpyAsync(ctx->nb_ids.p, ids.data(), ids.size() * 4,
                            hipMemcpyHostToDevice, s));
+  int32_t* const counters = ctx->nb_rerun.as<int32_t>();
+  HIP_TRY(zero32(s, counters, 2));
   HIP_TRY(hipEventRecord(ctx->ev[14], s));
-  if (n > 0)
-    hipLaunchKernelGGL(k_power_nbrs, dim3(n), dim3(64), 0, s, n,
-                       d_sph.as<double4>(), d_box.as<double>(), G,
-                       d_start.as<int64_t>(), d_ids.as<int32_t>(),
-                       d_valid.as<int32_t>(), d_cnt.as<int32_t>(),
-                       d_lists.as<int32_t>());
+  if (n > 0) {
+    hipLaunchKernelGGL((k_power_nbrs<1, 64>), dim3(n), dim3(64), 0, s, n,
+                       (const int32_t*)nullptr, (const int32_t*)nullptr,
+                       ctx->nb_sph.as<double4>(), ctx->nb_box.as<double>(), G,
+                       ctx->nb_start.as<int64_t>(), ctx->nb_ids.as<int32_t>(),
+                       ctx->nb_cellw.as<float>(), ctx->nb_valid.as<int32_t>(), ctx->nb_cnt.as<int32_t>(),
+                       ctx->nb_lists.as<int32_t>(), counters + 2, counters);
+    HIP_TRY(hipGetLastError());
+    // the few larger cells: a fixed grid walks the list
+    hipLaunchKernelGGL((k_power_nbrs<kNbV / 64, kNbP>),
+                       dim3(std::min(n, 2048)), dim3(64), 0, s, n,
+                       (const int32_t*)(counters + 2),
+                       (const int32_t*)counters, ctx->nb_sph.as<double4>(),
+                       ctx->nb_box.as<double>(), G,
+                       ctx->nb_start.as<int64_t>(), ctx->nb_ids.as<int32_t>(),
+                       ctx->nb_cellw.as<float>(), ctx->nb_valid.as<int32_t>(), ctx->nb_cnt.as<int32_t>(),
+                       ctx->nb_lists.as<int32_t>(), (int32_t*)nullptr,
+                       (int32_t*)nullptr);
+  }
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(ctx->ev[15], s));
-  std::vector<int32_t> valid(n), cnt(n), lists((size_t)n * kNbOut);
-  if (n > 0) {
-    HIP_TRY(hipMemcpyAsync(valid.data(), d_valid.p, (size_t)n * 4,
-                           hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(cnt.data(), d_cnt.p, (size_t)n * 4,
-                           hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(lists.data(), d_lists.p, (size_t)n * kNbOut * 4,
-                           hipMemcpyDeviceToHost, s));
-  }
-  HIP_TRY(wait_stream(ctx, s));
+  hipLaunchKernelGGL(k_nbr_check, dim3(ceil_div(((int64_t)n + 1) * 32, 256)),
+                     dim3(256), 0, s, n, ctx->nb_valid.as<int32_t>(),
+                     ctx->nb_cnt.as<int32_t>(), ctx->nb_lists.as<int32_t>(),
+                     ctx->nb_cnt64.as<int64_t>(), counters + 1);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(exclusive_sum<int64_t>(ctx, ctx->nb_cnt64.as<int64_t>(),
+                                 ctx->nb_off.as<int64_t>(), (int64_t)n + 1));
+  int32_t n_odd = 0;
+  int64_t total = 0;
+  HIP_TRY(read_back(ctx, s, {{&n_odd, counters + 1, 4},
+                             {&total, ctx->nb_off.as<int64_t>() + n, 8}}));
   if (ms_out) {
     float m = 0;
     HIP_TRY(hipEventElapsedTime(&m, ctx->ev[14], ctx->ev[15]));
     *ms_out = m;
   }
+  std::vector<int32_t> valid(n);
+  if (n > 0)
+    HIP_TRY(hipMemcpyAsync(valid.data(), ctx->nb_valid.p, (size_t)n * 4,
+                           hipMemcpyDeviceToHost, s));
+  if (n_odd == 0) {  // the lists are their own symmetric closure
+    std::vector<int64_t> off((size_t)n + 1);
+    std::vector<int32_t> nid((size_t)total);
+    HIP_TRY(hipMemcpyAsync(off.data(), ctx->nb_off.p, ((size_t)n + 1) * 8,
+                           hipMemcpyDeviceToHost, s));
+    if (total > 0) {
+      HIP_TRY(ctx->nb_pack.need((size_t)total * 4));
+      hipLaunchKernelGGL(k_nbr_pack, dim3(ceil_div((int64_t)n * 32, 256)),
+                         dim3(256), 0, s, n, ctx->nb_lists.as<int32_t>(),
+                         ctx->nb_off.as<int64_t>(),
+                         ctx->nb_pack.as<int32_t>());
+      HIP_TRY(hipGetLastError());
+      HIP_TRY(hipMemcpyAsync(nid.data(), ctx->nb_pack.p, (size_t)total * 4,
+                             hipMemcpyDeviceToHost, s));
+    }
+    HIP_TRY(wait_stream(ctx, s));
+    *out = rpd_nbr_adopt(std::move(valid), std::move(off), std::move(nid));
+    return 0;
+  }
+  std::vector<int32_t> cnt(n), lists((size_t)n * kNbOut);
+  HIP_TRY(hipMemcpyAsync(cnt.data(), ctx->nb_cnt.p, (size_t)n * 4,
+                         hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipMemcpyAsync(lists.data(), ctx->nb_lists.p, (size_t)n * kNbOut * 4,
+                         hipMemcpyDeviceToHost, s));
+  HIP_TRY(wait_stream(ctx, s));
   for (int32_t i = 0; i < n; ++i)
     if (valid[i] < 0)
       return fail(ctx, "rpd_power_neighbors_gpu: sphere " + std::to_string(i) +

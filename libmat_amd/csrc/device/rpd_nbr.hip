@@ -33,25 +33,31 @@ struct NbGrids {
   NbGrid g[8];
 };
 
+// k / d for 0 <= k and 0 < d, by a reciprocal below 2^21 (there the
+// product's error, at most (k + 0.5) / d * 2^-22, stays under 0.5 / d)
+__device__ __forceinline__ int quot(int k, int d) {
+  return k < (1 << 21)
+             ? (int)(((float)k + 0.5f) * __builtin_amdgcn_rcpf((float)d))
+             : k / d;
+}
+
 // cell of Chebyshev shell r (k in [0, shell size)) around the origin
 __device__ __forceinline__ void shell_cell(int r, int k, int& dx, int& dy,
                                            int& dz) {
-  if (r == 0) {
-    dx = dy = dz = 0;
-    return;
-  }
   const int side = 2 * r + 1, face = side * side;
   if (k < 2 * face) {  // the two z faces
     dz = k < face ? -r : r;
-    const int q = k % face;
-    dy = q / side - r;
-    dx = q % side - r;
+    const int q = k < face ? k : k - face;
+    const int row = quot(q, side);
+    dy = row - r;
+    dx = q - row * side - r;
     return;
   }
   const int q = k - 2 * face;  // rings of the slabs between them
   const int per = 8 * r;
-  dz = -r + 1 + q / per;
-  const int p = q % per;
+  const int slab = quot(q, per);
+  dz = -r + 1 + slab;
+  const int p = q - slab * per;
   if (p < side) {
     dy = -r;
     dx = -r + p;
@@ -69,38 +75,126 @@ __device__ __forceinline__ int shell_size(int r) {
   return r == 0 ? 1 : 2 * (2 * r + 1) * (2 * r + 1) + (2 * r - 1) * 8 * r;
 }
 
-// sign of the bisector e at vertex (planes p1, p2, p3; homogeneous X, Q)
-__device__ __forceinline__ int nb_side(const rpd_d4& p1, const rpd_d4& p2,
-                                       const rpd_d4& p3, const rpd_d4& X,
-                                       const rpd_d4& Q, const rpd_d4& e) {
-  int s = rpd_filtered_sign4(e, X, Q);
-  if (s == 0) s = rpd_exact_det4_sign(p1, p2, p3, e);
-  int w = rpd_filtered_sign_w(X, Q);
-  if (w == 0) w = rpd_exact_w_sign(p1, p2, p3);
-  return s * w;
+// v of lane l (l the same in every lane)
+__device__ __forceinline__ double lane_value(double v, int l) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)u, l);
+  const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ float lane_value(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int l) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+__device__ __forceinline__ int lanes_below(uint64_t m, int lane) {
+  return __popcll(m & ((1ull << lane) - 1));
+}
+__device__ __noinline__ int nb_exact_w(rpd_d4 p1, rpd_d4 p2, rpd_d4 p3) {
+  return rpd_exact_w_sign(p1, p2, p3);
+}
+// dot(e, X) and the filter bound of its sign: rpd_filtered_sign4 with
+// sum |e_r| Q_r replaced by the larger max |e_r| * sum Q_r (the sum and the
+// product fall short by at most 4u relative, which the 8 % slack of the
+// constant over gamma_10 covers; products may fuse into the sums, no
+// monomial then passing through more roundings).  An unrepresentable bound
+// is infinite: nothing is decided.
+__device__ __forceinline__ void nb_dot(const rpd_d4& e, double me,
+                                       const rpd_d4& X, double sq, double& s,
+                                       double& eps) {
+#pragma clang fp contract(fast)
+  s = e.x * X.x + e.y * X.y + e.z * X.z + e.w * X.w;
+  const double b = me * sq;
+  eps = b < RPD_FILTER_MAX ? RPD_FILTER_C * b + RPD_FILTER_ABS : INFINITY;
 }
 
-// One wavefront per sphere.  valid[i]: 1 valid, 0 hidden, -1 capacity or
-// topology failure; counts[i] / lists[i * kNbOut ..]: neighbour ids.
-__global__ __launch_bounds__(64) void k_power_nbrs(
-    int32_t n, const double4* __restrict__ sph, const double* box, NbGrids G,
-    const int64_t* __restrict__ start, const int32_t* __restrict__ ids,
-    int32_t* valid, int32_t* counts, int32_t* lists) {
-  __shared__ double4 s_pl[kNbP];
-  __shared__ int32_t s_src[kNbP];
-  __shared__ double4 s_X[2][kNbV];
-  __shared__ double4 s_Q[2][kNbV];
-  __shared__ uint32_t s_t[2][kNbV];
-  __shared__ uint8_t s_out[kNbV];
-  __shared__ uint8_t s_used[kNbP];
-  __shared__ int16_t s_map[kNbP];
-  __shared__ int32_t s_new;
-  const int i = blockIdx.x;
+// One wavefront per sphere.  The cell's vertices live in registers, vertex
+// slot 64 q + lane in slot q of a lane: homogeneous coordinates X with
+// X.w > 0 (the plane triple is ordered for it), the sum of its cofactor
+// permanents, the triple.  Only the planes are in LDS.
+//
+// What bounds it is the chain of clips per sphere (each a few dependent LDS
+// and lane exchanges), so a clip is kept short and unneeded ones are not
+// started: candidates are taken 64 at a time, one per lane, in the order of
+// the search (class, shell, 64 cells of it, member number, cell: it decides
+// which of several bisectors through one point carries a face), and each
+// lane first tests its bisector against every vertex of the cell as it is
+// now; a bisector certainly positive everywhere cannot cut the cell or any
+// later state of it.  The rest are clipped one after the other.  In a clip
+// the edges that the plane cuts are the pairs (removed, kept) of vertices
+// that share two planes: for each removed vertex every lane compares its
+// own triple.  New vertices take the free slots.
+//
+// kVS = 1 (64 vertices, 64 planes) holds nearly every cell; a sphere whose
+// cell outgrows it is listed and done again from the start with kVS = 4
+// (256 vertices, 192 planes), whose launch reads the list's length on the
+// device.  50,000 spheres of the boundary rule: one kernel of 256-vertex
+// cells in LDS (42 KB a wavefront, every candidate clipped, the cut edges
+// found by one lane per removed vertex scanning all vertices) took
+// 203 ms, this one 14 ms with the larger cells (5,003 uniform spheres: 2.3
+// and 0.7 ms).  The small tier at 2, 3 and 4 wavefronts per SIMD (the
+// register limit): 14.7, 11.8 and 15.0 ms (4 spills).
+//
+// valid[i]: 1 valid, 0 hidden, -1 capacity or topology failure; counts[i] /
+// lists[i * kNbOut ..]: neighbour ids, ascending.
+template <int kVS, int kP>
+__device__ __forceinline__ void power_cell(
+    int i, const double4* __restrict__ sph, const double* box,
+    const NbGrids& G, const int64_t* __restrict__ start,
+    const int32_t* __restrict__ ids, int32_t* valid, int32_t* counts,
+    int32_t* lists, int32_t* rerun, int32_t* n_rerun, double4* s_pl,
+    int32_t* s_src, uint32_t* s_new, int32_t* s_q, uint8_t* s_used,
+    uint8_t* s_map, const float* __restrict__ cell_w) {
+  constexpr bool kSmall = kP < kNbP;
   const int lane = threadIdx.x;
-  if (i >= n) return;
   const double4 sd = sph[i];
   const rpd_d4 si{sd.x, sd.y, sd.z, sd.w};
+  rpd_d4 X[kVS];
+  double sq[kVS];
+  uint32_t tr[kVS];     // planes a | b << 8 | c << 16, bit 31: X.w is 0
+  uint64_t alive[kVS];  // slots in use
+  float ux[kVS], uy[kVS], uz[kVS];  // position less the sphere's centre
+#pragma unroll
+  for (int q = 0; q < kVS; ++q) {
+    X[q] = rpd_d4{0, 0, 0, 1};
+    sq[q] = 0;
+    tr[q] = 0;
+    ux[q] = uy[q] = uz[q] = 0;
+    alive[q] = q == 0 ? 0xffull : 0;
+  }
+  int nv = 8, np = 6;
+  bool empty = false, fail = false;
+  bool lost = false;  // small tier: a sign this lane could not decide
+
+  // vertex of the planes a, b, c as this lane's slot q
+  auto set_vertex = [&](rpd_d4& Xq, double& sqq, uint32_t& trq, float& uxq,
+                        float& uyq, float& uzq, uint32_t a, uint32_t b,
+                        uint32_t c) {
+    const rpd_d4 pa = ld4(&s_pl[a]), pb = ld4(&s_pl[b]), pc = ld4(&s_pl[c]);
+    rpd_d4 Y, Q;
+    rpd_vertex_homog(pa, pb, pc, Y, Q);
+    int sw = rpd_filtered_sign_w(Y, Q);
+    if constexpr (kSmall)
+      lost = lost || sw == 0;
+    else if (sw == 0)
+      sw = nb_exact_w(pa, pb, pc);
+    if (sw < 0) {
+      Y = rpd_d4{-Y.x, -Y.y, -Y.z, -Y.w};
+      trq = b | (a << 8) | (c << 16);
+    } else {
+      trq = a | (b << 8) | (c << 16) | (sw == 0 ? 0x80000000u : 0u);
+    }
+    Xq = Y;
+    sqq = ((Q.x + Q.y) + Q.z) + Q.w;
+    const double iw = rcp64(Y.w);
+    uxq = (float)(Y.x * iw - si.x);
+    uyq = (float)(Y.y * iw - si.y);
+    uzq = (float)(Y.z * iw - si.z);
+  };
+
   // the domain box: x >= x0, x <= x1, y >= y0, y <= y1, z >= z0, z <= z1
+  wsync();
   if (lane < 6) {
     const int a = lane >> 1;
     double4 p = make_double4(0, 0, 0, 0);
@@ -116,80 +210,105 @@ __global__ __launch_bounds__(64) void k_power_nbrs(
     s_src[lane] = -1 - lane;
   }
   wsync();
-  if (lane < 8) {
-    const int a = lane & 1, b = 2 + ((lane >> 1) & 1), c = 4 + ((lane >> 2) & 1);
-    rpd_d4 X, Q;
-    rpd_vertex_homog(ld4(&s_pl[a]), ld4(&s_pl[b]), ld4(&s_pl[c]), X, Q);
-    s_X[0][lane] = make_double4(X.x, X.y, X.z, X.w);
-    s_Q[0][lane] = make_double4(Q.x, Q.y, Q.z, Q.w);
-    s_t[0][lane] = a | (b << 10) | (c << 20);
-  }
-  wsync();
-  int nv = 8, np = 6, cur = 0;
-  bool empty = false, fail = false;
-  auto radius2 = [&]() {
-    double r2 = 0;
-    for (int v = lane; v < nv; v += 64) {
-      const double4 X = s_X[cur][v];
-      const double x = X.x / X.w - si.x, y = X.y / X.w - si.y,
-                   z = X.z / X.w - si.z;
-      r2 = fmax(r2, x * x + y * y + z * z);
-    }
-    for (int off = 32; off > 0; off >>= 1) r2 = fmax(r2, __shfl_xor(r2, off));
-    return r2;
-  };
-  double R2 = radius2();
-
-  // clip the cell by the bisector of sphere j (every lane calls it)
-  auto clip = [&](int j) {
-    const double4 s2 = sph[j];
-    const rpd_d4 e = rpd_bisector(si, rpd_d4{s2.x, s2.y, s2.z, s2.w});
-    int n_out = 0;
-    for (int v0 = 0; v0 < nv; v0 += 64) {
-      const int v = v0 + lane;
-      bool o = false;
-      if (v < nv) {
-        const uint32_t t = s_t[cur][v];
-        const double4 X = s_X[cur][v], Q = s_Q[cur][v];
-        o = nb_side(ld4(&s_pl[t & 1023]), ld4(&s_pl[(t >> 10) & 1023]),
-                    ld4(&s_pl[(t >> 20) & 1023]),
-                    rpd_d4{X.x, X.y, X.z, X.w}, rpd_d4{Q.x, Q.y, Q.z, Q.w},
-                    e) < 0;
-        s_out[v] = o;
+  if (lane < 8)
+    set_vertex(X[0], sq[0], tr[0], ux[0], uy[0], uz[0], lane & 1,
+               2 + ((lane >> 1) & 1), 4 + ((lane >> 2) & 1));
+  // bounds of the cell about the centre c, in binary32: R2 no less than
+  // the largest |v - c|^2, and a ball (centre m, radius rm) that holds every
+  // vertex; 1e-5 covers the rounding of the positions and sums
+  float R2 = 0, mx = 0, my = 0, mz = 0, rm = 0;
+  auto set_bounds = [&]() {
+    float r2 = 0, sx = 0, sy = 0, sz = 0;
+#pragma unroll
+    for (int q = 0; q < kVS; ++q)
+      if ((alive[q] >> lane) & 1) {
+        r2 = fmaxf(r2, ux[q] * ux[q] + uy[q] * uy[q] + uz[q] * uz[q]);
+        sx += ux[q];
+        sy += uy[q];
+        sz += uz[q];
       }
-      n_out += __popcll(ballot(o));
+    for (int off = 32; off > 0; off >>= 1) {
+      r2 = fmaxf(r2, __shfl_xor(r2, off));
+      sx += __shfl_xor(sx, off);
+      sy += __shfl_xor(sy, off);
+      sz += __shfl_xor(sz, off);
     }
-    wsync();
+    const float inv = 1.0f / (float)nv;
+    mx = sx * inv;
+    my = sy * inv;
+    mz = sz * inv;
+    float d2 = 0;
+#pragma unroll
+    for (int q = 0; q < kVS; ++q)
+      if ((alive[q] >> lane) & 1) {
+        const float dx = ux[q] - mx, dy = uy[q] - my, dz = uz[q] - mz;
+        d2 = fmaxf(d2, dx * dx + dy * dy + dz * dz);
+      }
+    for (int off = 32; off > 0; off >>= 1) d2 = fmaxf(d2, __shfl_xor(d2, off));
+    R2 = r2 * 1.00001f;
+    rm = sqrtf(d2) * 1.00001f + 1e-5f * sqrtf(r2);
+  };
+  set_bounds();
+
+  // clip the cell by e, the bisector of sphere j (the same in every lane)
+  auto clip = [&](int j, const rpd_d4& e, double me) {
+    uint64_t out[kVS];
+    int n_out = 0;
+#pragma unroll
+    for (int q = 0; q < kVS; ++q) {
+      out[q] = 0;
+      if (alive[q] == 0) continue;
+      bool o = false;
+      if (((alive[q] >> lane) & 1) && !(tr[q] >> 31)) {
+        double s, eps;
+        nb_dot(e, me, X[q], sq[q], s, eps);
+        o = s < -eps;
+        const bool open = !o && !(s > eps);
+        if constexpr (kSmall)
+          lost = lost || open;
+        else if (open)
+          o = conflict_exact(ld4(&s_pl[tr[q] & 255]),
+                             ld4(&s_pl[(tr[q] >> 8) & 255]),
+                             ld4(&s_pl[(tr[q] >> 16) & 255]), e) < 0;
+      }
+      out[q] = ballot(o);
+      n_out += __popcll(out[q]);
+    }
+    if (kSmall && ballot(lost) != 0) {
+      fail = true;
+      return;
+    }
     if (n_out == 0) return;
     if (n_out == nv) {
       empty = true;
       return;
     }
-    if (np >= kNbP) {
+    if (np >= kP) {
       // planes no vertex uses any more are dropped and the rest renumbered
       // (box planes stay at 0..5)
       for (int q = lane; q < np; q += 64) s_used[q] = q < 6;
       wsync();
-      for (int v = lane; v < nv; v += 64) {
-        const uint32_t t = s_t[cur][v];
-        s_used[t & 1023] = 1;
-        s_used[(t >> 10) & 1023] = 1;
-        s_used[(t >> 20) & 1023] = 1;
-      }
+#pragma unroll
+      for (int q = 0; q < kVS; ++q)
+        if ((alive[q] >> lane) & 1) {
+          s_used[tr[q] & 255] = 1;
+          s_used[(tr[q] >> 8) & 255] = 1;
+          s_used[(tr[q] >> 16) & 255] = 1;
+        }
       wsync();
       int kept = 0;
       for (int q0 = 0; q0 < np; q0 += 64) {
         const int q = q0 + lane;
         const bool u = q < np && s_used[q];
         const uint64_t bm = ballot(u);
-        const int to = kept + __popcll(bm & ((1ull << lane) - 1));
+        const int to = kept + lanes_below(bm, lane);
         double4 pl = make_double4(0, 0, 0, 0);
         int32_t sr = 0;
         if (u) {
           pl = s_pl[q];
           sr = s_src[q];
+          s_map[q] = (uint8_t)to;
         }
-        if (q < np) s_map[q] = (int16_t)(u ? to : -1);
         wsync();
         if (u) {
           s_pl[to] = pl;
@@ -198,88 +317,130 @@ __global__ __launch_bounds__(64) void k_power_nbrs(
         wsync();
         kept += __popcll(bm);
       }
-      for (int v = lane; v < nv; v += 64) {
-        const uint32_t t = s_t[cur][v];
-        s_t[cur][v] = (uint32_t)s_map[t & 1023] |
-                      ((uint32_t)s_map[(t >> 10) & 1023] << 10) |
-                      ((uint32_t)s_map[(t >> 20) & 1023] << 20);
-      }
+#pragma unroll
+      for (int q = 0; q < kVS; ++q)
+        if ((alive[q] >> lane) & 1)
+          tr[q] = (uint32_t)s_map[tr[q] & 255] |
+                  ((uint32_t)s_map[(tr[q] >> 8) & 255] << 8) |
+                  ((uint32_t)s_map[(tr[q] >> 16) & 255] << 16) |
+                  (tr[q] & 0x80000000u);
       wsync();
       np = kept;
-      if (np >= kNbP) {
+      if (np >= kP) {
         fail = true;
         return;
       }
     }
-    const int p = np;
+    const uint32_t p = (uint32_t)np;
     if (lane == 0) {
       s_pl[p] = make_double4(e.x, e.y, e.z, e.w);
       s_src[p] = j;
-      s_new = 0;
     }
-    wsync();
-    const int nxt = cur ^ 1;
-    const int n_keep = nv - n_out;
-    int base = 0;
-    for (int v0 = 0; v0 < nv; v0 += 64) {
-      const int v = v0 + lane;
-      const bool keep = v < nv && !s_out[v];
-      const uint64_t bm = ballot(keep);
-      if (keep) {
-        const int pos = base + __popcll(bm & ((1ull << lane) - 1));
-        s_X[nxt][pos] = s_X[cur][v];
-        s_Q[nxt][pos] = s_Q[cur][v];
-        s_t[nxt][pos] = s_t[cur][v];
-      }
-      base += __popcll(bm);
-    }
-    // new vertices where an edge joins a removed and a kept vertex: each
-    // removed vertex looks across its three edges
-    bool lfail = false;
-    for (int v = lane; v < nv; v += 64) {
-      if (!s_out[v]) continue;
-      const uint32_t tv = s_t[cur][v];
-      const int pv[3] = {(int)(tv & 1023), (int)((tv >> 10) & 1023),
-                         (int)((tv >> 20) & 1023)};
-      for (int q = 0; q < 3; ++q) {
-        const int a = pv[q], b = pv[(q + 1) % 3];
-        int other = -1;
-        for (int u = 0; u < nv; ++u) {
-          if (u == v) continue;
-          const uint32_t tu = s_t[cur][u];
-          const int u0 = tu & 1023, u1 = (tu >> 10) & 1023,
-                    u2 = (tu >> 20) & 1023;
-          const bool ha = u0 == a || u1 == a || u2 == a;
-          const bool hb = u0 == b || u1 == b || u2 == b;
-          if (ha && hb) {
-            other = u;
-            break;
-          }
+    // a new vertex where an edge joins a removed and a kept vertex
+    int n_new = 0, n_edge = 0;
+#pragma unroll
+    for (int q = 0; q < kVS; ++q) {
+      uint64_t todo = out[q];
+      while (todo) {
+        const int r = __ffsll((long long)todo) - 1;
+        todo &= todo - 1;
+        const uint32_t t = lane_value(tr[q], r);
+        const uint32_t a = t & 255, b = (t >> 8) & 255, c = (t >> 16) & 255;
+#pragma unroll
+        for (int u = 0; u < kVS; ++u) {
+          if (alive[u] == 0) continue;
+          const uint32_t x = tr[u] & 255, y = (tr[u] >> 8) & 255,
+                         z = (tr[u] >> 16) & 255;
+          const bool ha = x == a || y == a || z == a;
+          const bool hb = x == b || y == b || z == b;
+          const bool hc = x == c || y == c || z == c;
+          const bool two = ha ? hb != hc : hb && hc;
+          const uint64_t edge = ballot(two) & alive[u];
+          n_edge += __popcll(edge);
+          const uint64_t nw = edge & ~out[u];
+          const int at = n_new + lanes_below(nw, lane);
+          if (((nw >> lane) & 1) && at < 64 * kVS)
+            s_new[at] = !ha ? b | (c << 8) : !hb ? a | (c << 8) : a | (b << 8);
+          n_new += __popcll(nw);
         }
-        if (other < 0) {
-          lfail = true;
-          continue;
-        }
-        if (s_out[other]) continue;
-        const int slot = atomicAdd(&s_new, 1);
-        if (n_keep + slot >= kNbV) {
-          lfail = true;
-          continue;
-        }
-        rpd_d4 X, Q;
-        rpd_vertex_homog(ld4(&s_pl[a]), ld4(&s_pl[b]), ld4(&s_pl[p]), X, Q);
-        s_X[nxt][n_keep + slot] = make_double4(X.x, X.y, X.z, X.w);
-        s_Q[nxt][n_keep + slot] = make_double4(Q.x, Q.y, Q.z, Q.w);
-        s_t[nxt][n_keep + slot] = a | (b << 10) | (p << 20);
       }
     }
-    fail = fail || (ballot(lfail) != 0);
+    // every removed vertex has three edges
+    if (n_edge != 3 * n_out || nv - n_out + n_new > 64 * kVS) {
+      fail = true;
+      return;
+    }
     wsync();
-    nv = n_keep + min(s_new, kNbV - n_keep);
-    np = p + 1;
-    cur = nxt;
+    int base = 0;  // the new vertices take the free slots
+#pragma unroll
+    for (int q = 0; q < kVS; ++q) {
+      alive[q] &= ~out[q];
+      const uint64_t fr = ~alive[q];
+      const int at = base + lanes_below(fr, lane);
+      const bool take = ((fr >> lane) & 1) && at < n_new;
+      if (take) {
+        const uint32_t ab = s_new[at];
+        set_vertex(X[q], sq[q], tr[q], ux[q], uy[q], uz[q], ab & 255, ab >> 8,
+                   p);
+      }
+      base += __popcll(fr);
+      alive[q] |= ballot(take);
+      if (base >= n_new) {
+#pragma unroll
+        for (int u = q + 1; u < kVS; ++u) alive[u] &= ~out[u];
+        break;
+      }
+    }
     wsync();
-    R2 = radius2();
+    nv += n_new - n_out;
+    np = (int)p + 1;
+  };
+
+  // the first cnt spheres of s_q, one per lane
+  auto flush = [&](int cnt) {
+    const int j = lane < cnt ? s_q[lane] : -1;
+    rpd_d4 e{0, 0, 0, 0};
+    double me = 0;
+    bool may = false;
+    if (j >= 0) {
+      const double4 sj = sph[j];
+      const double dx = sj.x - si.x, dy = sj.y - si.y, dz = sj.z - si.z;
+      const double d = sqrt(dx * dx + dy * dy + dz * dz);
+      const double Rc = sqrt((double)R2) * (1 + 1e-9) + 1e-12;
+      const double bj = Rc + sqrt(fmax(0.0, Rc * Rc - si.w + sj.w));
+      may = !(d > bj * (1 + 1e-9) + 1e-12);
+      e = rpd_bisector(si, rpd_d4{sj.x, sj.y, sj.z, sj.w});
+      me = fmax(fmax(fabs(e.x), fabs(e.y)), fmax(fabs(e.z), fabs(e.w)));
+    }
+    const uint64_t reach = ballot(may);
+    if (reach == 0) return;
+    bool cuts = false;
+    uint64_t todo = 0;
+#pragma unroll
+    for (int q = 0; q < kVS; ++q) {
+      uint64_t v = alive[q];
+      while (v) {
+        const int l = __ffsll((long long)v) - 1;
+        v &= v - 1;
+        const rpd_d4 Y{lane_value(X[q].x, l), lane_value(X[q].y, l),
+                       lane_value(X[q].z, l), lane_value(X[q].w, l)};
+        double s, eps;
+        nb_dot(e, me, Y, lane_value(sq[q], l), s, eps);
+        cuts = cuts || !(s > eps);
+        todo = ballot(may && cuts);
+        if (todo == reach) break;
+      }
+      if (todo == reach) break;
+    }
+    if (todo == 0) return;
+    while (todo && !empty && !fail) {
+      const int l = __ffsll((long long)todo) - 1;
+      todo &= todo - 1;
+      const rpd_d4 ej{lane_value(e.x, l), lane_value(e.y, l),
+                      lane_value(e.z, l), lane_value(e.w, l)};
+      clip((int)lane_value((uint32_t)j, l), ej, lane_value(me, l));
+    }
+    if (!empty && !fail) set_bounds();
   };
 
   for (int c = 0; c < 8 && !empty && !fail; ++c) {
@@ -295,19 +456,66 @@ __global__ __launch_bounds__(64) void k_power_nbrs(
       if (-lo > rmin) rmin = -lo;  // rings before the grid: none
       if (hi > rmin) rmin = hi;
     }
-    for (int64_t r = rmin; r <= rmax && !empty && !fail; ++r) {
+    const float csf = (float)g.cs, wi = (float)si.w;
+    // (d2: squared distance of a vertex to a cell's box, vv: to the centre)
+    auto reaches = [&](float d2, float vv, float wl) {
+      return !(d2 > vv - wi + wl + 1e-5f * (vv + fabsf(wi) + wl + d2));
+    };
+    int qn = 0;  // spheres waiting in s_q
+    bool done = false;
+    for (int64_t r = rmin; !done && !empty && !fail; ++r) {
+      const double R = sqrt((double)R2) * (1 + 1e-9) + 1e-12;
       {
-        const double R = sqrt(R2) * (1 + 1e-9) + 1e-12;
         const double bound = R + sqrt(fmax(0.0, R * R - si.w + g.wmax));
-        if (r >= 1 && (double)(r - 1) * g.cs > bound * (1 + 1e-9) + 1e-12)
-          break;
+        done = r > rmax ||
+               (r >= 1 && (double)(r - 1) * g.cs > bound * (1 + 1e-9) + 1e-12);
       }
-      const int S = shell_size((int)r);
-      for (int k0 = 0; k0 < S && !empty && !fail; k0 += 64) {
-        // this lane's cell of the shell and its member range
+      // the shell's cells in [k_lo[u], k_hi[u]): the rows of its two z
+      // faces that lie in the grid, and the slabs that do
+      int k_lo[3] = {0, 0, 0}, k_hi[3] = {0, 0, 0};
+      if (!done) {
+        const int ri = (int)r, side = 2 * ri + 1, face = side * side;
+        const int y0 = (int)(q0[1] - r < 0 ? r - q0[1] : 0);
+        const int y1 = (int)min((int64_t)(side - 1), g.dim[1] - 1 - q0[1] + r);
+        for (int u = 0; u < 2; ++u) {
+          const int64_t z = u == 0 ? q0[2] - r : q0[2] + r;
+          if (z >= 0 && z < g.dim[2] && y0 <= y1 && (u == 0 || r > 0)) {
+            k_lo[u] = u * face + y0 * side;
+            k_hi[u] = u * face + (y1 + 1) * side;
+          }
+        }
+        const int64_t s0 = max((int64_t)0, r - 1 - q0[2]);
+        const int64_t s1 = min(2 * r - 2, g.dim[2] - 1 - q0[2] + r - 1);
+        if (s0 <= s1) {
+          k_lo[2] = 2 * face + (int)s0 * 8 * ri;
+          k_hi[2] = 2 * face + (int)(s1 + 1) * 8 * ri;
+        }
+      }
+      // the next chunk of 64 cells (from a multiple of 64) at or after k
+      // that meets one of the ranges; INT_MAX: none
+      auto chunk_from = [&](int k) {
+        int best = 0x7fffffff;
+        for (int u = 0; u < 3; ++u)
+          if (k < k_hi[u])
+            best = min(best, max(k, k_lo[u] & ~63));
+        return best;
+      };
+      int k0 = chunk_from(0);
+      for (;;) {
+        // this lane's cell of the shell and its member range, if a sphere
+        // of the cell may cut the polytope: a sphere j of its box cuts a
+        // vertex v off only if dist(v, box)^2 - max w_j < |v - c|^2 - w.
+        // First with the ball about m and R2 for every vertex, then vertex
+        // by vertex (binary32 about the centre c, 1e-5 of every term for
+        // its rounding): lanes take the cells and the vertices are
+        // broadcast, or the other way round, whichever loop is shorter
         int64_t a0 = 0, a1 = 0;
         const int k = k0 + lane;
-        if (k < S) {
+        float lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0}, wc = 0;
+        bool near = false;
+        if (k0 != 0x7fffffff &&
+            ((k >= k_lo[0] && k < k_hi[0]) || (k >= k_lo[1] && k < k_hi[1]) ||
+             (k >= k_lo[2] && k < k_hi[2]))) {
           int dx, dy, dz;
           shell_cell((int)r, k, dx, dy, dz);
           const int64_t x = q0[0] + dx, y = q0[1] + dy, z = q0[2] + dz;
@@ -317,36 +525,103 @@ __global__ __launch_bounds__(64) void k_power_nbrs(
                 g.cell_base + x + (int64_t)g.dim[0] * (y + (int64_t)g.dim[1] * z);
             a0 = start[cell];
             a1 = start[cell + 1];
-          }
-        }
-        int len = (int)(a1 - a0);
-        for (int off = 32; off > 0; off >>= 1) len = max(len, __shfl_xor(len, off));
-        for (int m = 0; m < len && !empty && !fail; ++m) {
-          // each lane offers its m-th member if it may reach the cell
-          int j = -1;
-          if (a0 + m < a1) {
-            j = ids[a0 + m];
-            if (j == i) {
-              j = -1;
-            } else {
-              const double4 sj = sph[j];
-              const double ddx = sj.x - si.x, ddy = sj.y - si.y,
-                           ddz = sj.z - si.z;
-              const double d = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
-              const double Rc = sqrt(R2) * (1 + 1e-9) + 1e-12;
-              const double bj = Rc + sqrt(fmax(0.0, Rc * Rc - si.w + sj.w));
-              if (d > bj * (1 + 1e-9) + 1e-12) j = -1;
+            wc = cell_w[cell];
+            const double bx[3] = {g.org[0] + (double)x * g.cs - si.x,
+                                  g.org[1] + (double)y * g.cs - si.y,
+                                  g.org[2] + (double)z * g.cs - si.z};
+            for (int a = 0; a < 3; ++a) {
+              lo[a] = (float)bx[a] - 1e-5f * csf;
+              hi[a] = (float)bx[a] + 1.00001f * csf;
             }
-          }
-          uint64_t todo = ballot(j >= 0);
-          while (todo && !empty && !fail) {
-            const int src = __ffsll((long long)todo) - 1;
-            todo &= todo - 1;
-            clip(__shfl(j, src));
+            const float ex = fmaxf(0.f, fmaxf(lo[0] - mx, mx - hi[0]));
+            const float ey = fmaxf(0.f, fmaxf(lo[1] - my, my - hi[1]));
+            const float ez = fmaxf(0.f, fmaxf(lo[2] - mz, mz - hi[2]));
+            const float far = sqrtf(ex * ex + ey * ey + ez * ez) * 0.99999f;
+            const float sl = R2 - wi + wc + 1e-5f * (R2 + fabsf(wi) + wc);
+            near = a0 < a1 && !(far > rm && (far - rm) * (far - rm) > sl);
           }
         }
+        uint64_t nearm = ballot(near);
+        if (nearm != 0) {
+          if (__popcll(nearm) < nv) {
+            uint64_t todo = nearm;
+            while (todo) {
+              const int l = __ffsll((long long)todo) - 1;
+              todo &= todo - 1;
+              const float x0 = lane_value(lo[0], l), y0 = lane_value(lo[1], l),
+                          z0 = lane_value(lo[2], l), x1 = lane_value(hi[0], l),
+                          y1 = lane_value(hi[1], l), z1 = lane_value(hi[2], l),
+                          wl = lane_value(wc, l);
+              bool cuts = false;
+#pragma unroll
+              for (int q = 0; q < kVS; ++q) {
+                const float uu =
+                    ux[q] * ux[q] + uy[q] * uy[q] + uz[q] * uz[q];
+                const float ex = fmaxf(0.f, fmaxf(x0 - ux[q], ux[q] - x1));
+                const float ey = fmaxf(0.f, fmaxf(y0 - uy[q], uy[q] - y1));
+                const float ez = fmaxf(0.f, fmaxf(z0 - uz[q], uz[q] - z1));
+                cuts = cuts || (((alive[q] >> lane) & 1) &&
+                                reaches(ex * ex + ey * ey + ez * ez, uu, wl));
+              }
+              if (ballot(cuts) == 0) nearm &= ~(1ull << l);
+            }
+          } else {
+            bool cuts = false;
+            uint64_t cm = 0;
+#pragma unroll
+            for (int q = 0; q < kVS; ++q) {
+              const float uu = ux[q] * ux[q] + uy[q] * uy[q] + uz[q] * uz[q];
+              uint64_t v = alive[q];
+              while (v && cm != nearm) {
+                const int l = __ffsll((long long)v) - 1;
+                v &= v - 1;
+                const float vx = lane_value(ux[q], l),
+                            vy = lane_value(uy[q], l),
+                            vz = lane_value(uz[q], l), vv = lane_value(uu, l);
+                const float ex = fmaxf(0.f, fmaxf(lo[0] - vx, vx - hi[0]));
+                const float ey = fmaxf(0.f, fmaxf(lo[1] - vy, vy - hi[1]));
+                const float ez = fmaxf(0.f, fmaxf(lo[2] - vz, vz - hi[2]));
+                cuts = cuts || reaches(ex * ex + ey * ey + ez * ez, vv, wc);
+                cm = ballot(near && cuts);
+              }
+            }
+            nearm = cm;
+          }
+          near = (nearm >> lane) & 1;
+        }
+        if (!near) a1 = a0;
+        const int kn = k0 == 0x7fffffff ? k0 : chunk_from(k0 + 64);
+        // waiting spheres are clipped when 64 are there, at the end of the
+        // first shells (whose spheres shrink the cell) and of the class
+        const bool last = kn == 0x7fffffff && (done || (r > 0 && r < rmin + 4));
+        for (int m = 0; !empty && !fail; ++m) {
+          const bool more = ballot(a0 + m < a1) != 0;
+          if (more) {
+            const int j = a0 + m < a1 ? ids[a0 + m] : i;
+            const uint64_t bm = ballot(j != i);
+            if (j != i) s_q[qn + lanes_below(bm, lane)] = j;
+            qn += __popcll(bm);
+            wsync();
+          }
+          if (qn >= 64 || (!more && last && qn > 0)) {
+            const int cnt = min(qn, 64);
+            flush(cnt);
+            const int rest = lane < qn - cnt ? s_q[64 + lane] : 0;
+            wsync();
+            if (lane < qn - cnt) s_q[lane] = rest;
+            qn -= cnt;
+            wsync();
+          }
+          if (!more && !(last && qn > 0)) break;
+        }
+        k0 = kn;
+        if (k0 == 0x7fffffff || empty || fail) break;
       }
     }
+  }
+  if (kSmall && (fail || ballot(lost) != 0)) {
+    if (lane == 0) rerun[atomicAdd(n_rerun, 1)] = i;
+    return;
   }
   if (fail || empty || nv == 0) {
     if (lane == 0) {
@@ -355,31 +630,95 @@ __global__ __launch_bounds__(64) void k_power_nbrs(
     }
     return;
   }
-  // neighbours: the bisectors that carry a vertex of the cell
+  // neighbours: the bisectors that carry a vertex of the cell, ascending
+  wsync();
   for (int p = lane; p < np; p += 64) s_used[p] = 0;
   wsync();
-  for (int v = lane; v < nv; v += 64) {
-    const uint32_t t = s_t[cur][v];
-    s_used[t & 1023] = 1;
-    s_used[(t >> 10) & 1023] = 1;
-    s_used[(t >> 20) & 1023] = 1;
-  }
+#pragma unroll
+  for (int q = 0; q < kVS; ++q)
+    if ((alive[q] >> lane) & 1) {
+      s_used[tr[q] & 255] = 1;
+      s_used[(tr[q] >> 8) & 255] = 1;
+      s_used[(tr[q] >> 16) & 255] = 1;
+    }
   wsync();
   int cnt = 0;
-  for (int p0 = 6; p0 < np; p0 += 64) {
-    const int p = p0 + lane;
-    const bool u = p < np && s_used[p];
-    const uint64_t bm = ballot(u);
-    if (u) {
-      const int pos = cnt + __popcll(bm & ((1ull << lane) - 1));
-      if (pos < kNbOut) lists[(int64_t)i * kNbOut + pos] = s_src[p];
-    }
-    cnt += __popcll(bm);
+  for (int p = 6; p < np; ++p) cnt += s_used[p];
+  for (int p = 6 + lane; p < np; p += 64) {
+    if (!s_used[p]) continue;
+    const int j = s_src[p];
+    int pos = 0;  // a sphere may carry two planes only if it came twice
+    for (int u = 6; u < np; ++u) pos += s_used[u] && s_src[u] < j;
+    if (pos < kNbOut) lists[(int64_t)i * kNbOut + pos] = j;
   }
   if (lane == 0) {
     valid[i] = cnt > kNbOut ? -1 : 1;
     counts[i] = min(cnt, kNbOut);
   }
+}
+
+template <int kVS, int kP>
+__global__ __launch_bounds__(64, (kVS == 1 ? 3 : 1)) void k_power_nbrs(
+    int32_t n, const int32_t* items, const int32_t* n_items,
+    const double4* __restrict__ sph, const double* box, NbGrids G,
+    const int64_t* __restrict__ start, const int32_t* __restrict__ ids,
+    const float* __restrict__ cell_w, int32_t* valid, int32_t* counts,
+    int32_t* lists, int32_t* rerun, int32_t* n_rerun) {
+  __shared__ double4 s_pl[kP];
+  __shared__ int32_t s_src[kP];
+  __shared__ uint32_t s_new[64 * kVS];
+  __shared__ int32_t s_q[128];
+  __shared__ uint8_t s_used[kP];
+  __shared__ uint8_t s_map[kP];
+  const int32_t m = items ? min(n, *n_items) : n;
+  for (int32_t q = blockIdx.x; q < m; q += gridDim.x)
+    power_cell<kVS, kP>(items ? items[q] : q, sph, box, G, start, ids, valid,
+                        counts, lists, rerun, n_rerun, s_pl, s_src, s_new,
+                        s_q, s_used, s_map, cell_w);
+}
+
+// One thread per list entry (i, k): every entry's sphere must be valid and
+// name i back; *n_odd counts the entries where it does not (bisectors
+// through one point) -- then the host closes the lists
+// (rpd_nbr_from_lists) -- and the spheres that failed.
+__global__ __launch_bounds__(256) void k_nbr_check(int32_t n,
+                                                   const int32_t* valid,
+                                                   const int32_t* counts,
+                                                   const int32_t* lists,
+                                                   int64_t* cnt64,
+                                                   int32_t* n_odd) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t i = q / 32;
+  if (i > n) return;
+  const int c = i < n ? counts[i] : 0;
+  if (q % 32 == 0) cnt64[i] = c;
+  if (i == n) return;
+  bool odd = valid[i] < 0;
+  for (int k = (int)(q % 32); k < c; k += 32) {
+    const int64_t j = lists[i * kNbOut + k];
+    const int cj = counts[j];
+    int lo = 0, hi = cj;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (lists[j * kNbOut + mid] < (int32_t)i)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    odd = odd || !(lo < cj && lists[j * kNbOut + lo] == (int32_t)i);
+  }
+  if (odd) atomicAdd(n_odd, 1);
+}
+__global__ __launch_bounds__(256) void k_nbr_pack(int32_t n,
+                                                  const int32_t* lists,
+                                                  const int64_t* off,
+                                                  int32_t* ids) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t i = q / 32;
+  if (i >= n) return;
+  const int64_t o = off[i];
+  const int c = (int)(off[i + 1] - o);
+  for (int k = (int)(q % 32); k < c; k += 32) ids[o + k] = lists[i * kNbOut + k];
 }
 
 }  // namespace rpd

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../common/rpd_classgrid.h"
+#include "../common/rpd_nbrlist.h"
 #include "../common/rpd_predicates.h"
 
 namespace {
@@ -401,13 +402,6 @@ struct Poly {
 
 }  // namespace
 
-struct rpd_nbr {
-  std::vector<int32_t> valid;
-  std::vector<int64_t> offsets;
-  std::vector<int32_t> ids;
-  int32_t max_degree = 0;
-};
-
 namespace {
 // CSR of the symmetric closure over valid spheres: j is a neighbour of i
 // iff either list names the other and both are valid; ascending ids
@@ -552,6 +546,19 @@ extern "C" int rpd_power_neighbors(int32_t n, const double* xyzw,
   symmetrize(n, nb, res);
   *out = res;
   return 0;
+}
+
+rpd_nbr* rpd_nbr_adopt(std::vector<int32_t>&& valid,
+                       std::vector<int64_t>&& offsets,
+                       std::vector<int32_t>&& ids) {
+  auto* res = new rpd_nbr();
+  res->valid = std::move(valid);
+  res->offsets = std::move(offsets);
+  res->ids = std::move(ids);
+  for (size_t i = 0; i + 1 < res->offsets.size(); ++i)
+    res->max_degree = std::max(
+        res->max_degree, (int32_t)(res->offsets[i + 1] - res->offsets[i]));
+  return res;
 }
 
 extern "C" int rpd_nbr_from_lists(int32_t n, const int32_t* valid,
