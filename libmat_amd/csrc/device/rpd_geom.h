@@ -150,4 +150,64 @@ __device__ __forceinline__ bool has_key(const uint64_t* keys, int64_t n,
   return lo < n && keys[lo] == k;
 }
 
+// ------------------------------------- polytopes held by one wavefront
+// Vertex slot 64 q + lane is slot q of a lane: its plane triple in tr[q] as
+// bytes a | b << 8 | c << 16; alive[q] marks the slots in use.
+// v of lane l (l the same in every lane)
+__device__ __forceinline__ double lane_value(double v, int l) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)u, l);
+  const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ float lane_value(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int l) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+__device__ __forceinline__ int lanes_below(uint64_t m, int lane) {
+  return __popcll(m & ((1ull << lane) - 1));
+}
+// The edges that a plane cuts when it removes the vertices out: the pairs
+// (removed, kept) that share two planes.  Every lane compares its own
+// triples with one removed vertex at a time.  s_new[0 .. n_new) receives
+// the shared planes a | b << 8 (as far as 64 kVS); n_edge counts the edges
+// at removed vertices, three each in a sound polytope.
+template <int kVS>
+__device__ __forceinline__ void cut_edges(const uint32_t (&tr)[kVS],
+                                          const uint64_t (&alive)[kVS],
+                                          const uint64_t (&out)[kVS],
+                                          int lane, uint32_t* s_new,
+                                          int& n_new, int& n_edge) {
+  n_new = n_edge = 0;
+#pragma unroll
+  for (int q = 0; q < kVS; ++q) {
+    uint64_t todo = out[q];
+    while (todo) {
+      const int r = __ffsll((long long)todo) - 1;
+      todo &= todo - 1;
+      const uint32_t t = lane_value(tr[q], r);
+      const uint32_t a = t & 255, b = (t >> 8) & 255, c = (t >> 16) & 255;
+#pragma unroll
+      for (int u = 0; u < kVS; ++u) {
+        if (alive[u] == 0) continue;
+        const uint32_t x = tr[u] & 255, y = (tr[u] >> 8) & 255,
+                       z = (tr[u] >> 16) & 255;
+        const bool ha = x == a || y == a || z == a;
+        const bool hb = x == b || y == b || z == b;
+        const bool hc = x == c || y == c || z == c;
+        const bool two = ha ? hb != hc : hb && hc;
+        const uint64_t edge = ballot(two) & alive[u];
+        n_edge += __popcll(edge);
+        const uint64_t nw = edge & ~out[u];
+        const int at = n_new + lanes_below(nw, lane);
+        if (((nw >> lane) & 1) && at < 64 * kVS)
+          s_new[at] = !ha ? b | (c << 8) : !hb ? a | (c << 8) : a | (b << 8);
+        n_new += __popcll(nw);
+      }
+    }
+  }
+}
+
 }  // namespace rpd

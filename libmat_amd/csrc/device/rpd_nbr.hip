@@ -75,22 +75,6 @@ __device__ __forceinline__ int shell_size(int r) {
   return r == 0 ? 1 : 2 * (2 * r + 1) * (2 * r + 1) + (2 * r - 1) * 8 * r;
 }
 
-// v of lane l (l the same in every lane)
-__device__ __forceinline__ double lane_value(double v, int l) {
-  const uint64_t u = (uint64_t)__double_as_longlong(v);
-  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)u, l);
-  const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
-  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-__device__ __forceinline__ float lane_value(float v, int l) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-__device__ __forceinline__ uint32_t lane_value(uint32_t v, int l) {
-  return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
-}
-__device__ __forceinline__ int lanes_below(uint64_t m, int lane) {
-  return __popcll(m & ((1ull << lane) - 1));
-}
 __device__ __noinline__ int nb_exact_w(rpd_d4 p1, rpd_d4 p2, rpd_d4 p3) {
   return rpd_exact_w_sign(p1, p2, p3);
 }
@@ -336,35 +320,8 @@ __device__ __forceinline__ void power_cell(
       s_pl[p] = make_double4(e.x, e.y, e.z, e.w);
       s_src[p] = j;
     }
-    // a new vertex where an edge joins a removed and a kept vertex
-    int n_new = 0, n_edge = 0;
-#pragma unroll
-    for (int q = 0; q < kVS; ++q) {
-      uint64_t todo = out[q];
-      while (todo) {
-        const int r = __ffsll((long long)todo) - 1;
-        todo &= todo - 1;
-        const uint32_t t = lane_value(tr[q], r);
-        const uint32_t a = t & 255, b = (t >> 8) & 255, c = (t >> 16) & 255;
-#pragma unroll
-        for (int u = 0; u < kVS; ++u) {
-          if (alive[u] == 0) continue;
-          const uint32_t x = tr[u] & 255, y = (tr[u] >> 8) & 255,
-                         z = (tr[u] >> 16) & 255;
-          const bool ha = x == a || y == a || z == a;
-          const bool hb = x == b || y == b || z == b;
-          const bool hc = x == c || y == c || z == c;
-          const bool two = ha ? hb != hc : hb && hc;
-          const uint64_t edge = ballot(two) & alive[u];
-          n_edge += __popcll(edge);
-          const uint64_t nw = edge & ~out[u];
-          const int at = n_new + lanes_below(nw, lane);
-          if (((nw >> lane) & 1) && at < 64 * kVS)
-            s_new[at] = !ha ? b | (c << 8) : !hb ? a | (c << 8) : a | (b << 8);
-          n_new += __popcll(nw);
-        }
-      }
-    }
+    int n_new, n_edge;
+    cut_edges<kVS>(tr, alive, out, lane, s_new, n_new, n_edge);
     // every removed vertex has three edges
     if (n_edge != 3 * n_out || nv - n_out + n_new > 64 * kVS) {
       fail = true;
