@@ -128,13 +128,14 @@ typedef struct {
                                  (with count_work, else 0)               */
   int64_t n_bbox_fallback;    /* spheres whose candidate box fell back to
                                  the whole domain                        */
-  int64_t n_bin_registrations; /* (sphere, bin) pairs of the candidate grid */
+  int64_t n_bin_registrations; /* (sphere, bin) pairs of the spheres' boxes
+                                 and the candidate grid                  */
   int32_t tet_k;              /* max candidates of one tet               */
   int32_t site_k;             /* max neighbours of one site              */
   double ms_total;            /* device time of the last rpd_run         */
   double ms_phase[8];         /* candidates, clip, re-runs, compaction   */
-  double ms_kernel[8];        /* site boxes, binning, relation count,
-                                 relation fill, plane masks, clip (small
+  double ms_kernel[8];        /* site boxes, their scan, relation, its
+                                 lists in tet order, plane masks, clip (small
                                  tier), compaction                       */
   int64_t work[3][4];         /* with count_work, per clip tier (small,
                                  capacity re-runs, exact): FP64 conflict
@@ -143,8 +144,8 @@ typedef struct {
                                  finished with success, exact-arithmetic
                                  determinants; otherwise 0               */
   int64_t relation_work[4];   /* with count_work: (tet, site) pairs of the
-                                 candidate bin lists tested, neighbour
-                                 tests of the relation, 0, related pairs */
+                                 candidate grid tested, neighbour tests
+                                 of the relation, 0, related pairs       */
   int64_t learned[4];         /* learned runs: first-round candidates,
                                  tets re-run (the fallback: closure over
                                  missing facet neighbours or the full
@@ -323,8 +324,8 @@ int rpd_site_centroids(rpd_ctx* ctx, double* out, const double** dev_out);
  * at the capacity.  rpd_graph_run replays the graph on the current data
  * (rpd_update_sites_batch may replace spheres and neighbour lists between
  * runs) and reads the counts back once; if one went past its capacity, or
- * the batch's per-instance tet or site counts, the tet subset switch or a
- * device buffer changed, it captures again through rpd_graph_build (whose
+ * the batch's per-instance tet or site counts, its mesh, the tet subset
+ * switch or a device buffer changed, it captures again through rpd_graph_build (whose
  * eager run gives the results) and sets *replayed = 0, else 1.  Results
  * are read as after rpd_run.  Plain and learned paths (cfg->learned 0, 1
  * or 2); count_work = 0, small_tier = 1.  A learned capture holds the

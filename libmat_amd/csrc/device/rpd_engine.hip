@@ -173,6 +173,8 @@ void Arena::restore() {
   saved.clear();
 }
 
+constexpr int kCounters = 16 + 128;
+
 struct TierBufs {
   Buf hdr, words, geom, areas;
   SlotView view(int V, int P, int E) const {
@@ -207,10 +209,10 @@ struct TierBufs {
   }
 };
 
-// sizes of one plain run: sphere-bin registrations, candidates, middle /
-// full / exact re-run entries, output stream
+// sizes of one plain run: candidates, middle / full / exact re-run entries,
+// output stream
 struct RunCaps {
-  int64_t n_reg = 0, n_cand = 0, n_mid = 0, n_full = 0, n_exact = 0;
+  int64_t n_cand = 0, n_mid = 0, n_full = 0, n_exact = 0;
   int64_t cells = 0, words = 0, areas = 0;
   // learned path: closure rounds run; the largest miss list, unique pairs
   // and new candidates of a round; the merged pairs, tets re-run on the
@@ -246,10 +248,20 @@ struct rpd_ctx {
   Buf knn_bis;
   Buf knn_bisf;
   // pipeline
-  Buf bbox, reg_n, reg_off, keys_a, keys_b, bin_start, bin_ids;
-  Buf tet_count, tet_off, tet_pass, cand, rel_ids;
-  Buf counters;  // int32[8]: fallback, n_rerun_large, n_rerun_exact, ...,
-                 // [6] n_rerun_full (after the middle tier)
+  Buf bbox, rel_pl, rel_aux, parts, part_off, keys_a, keys_b;
+  Buf tet_count, tet_off, pairs, pair_seg, tet_fill, cand, rel_ids;
+  // int32[kCounters]: fallback, n_rerun_large, n_rerun_exact, ...,
+  // [6] n_rerun_full (after the middle tier), [7] overflow of a captured
+  // run, [8] related pairs, from [16] 64 int64 box bins
+  Buf counters;
+  // the tets in the order of the candidate grid: all of them, and those of
+  // the subset; built by the first run that needs them
+  struct Bins {
+    Buf first, tet, c0, c1, c2;
+    bool ready = false;
+  } bins, sub_bins;
+  Buf bin_n, bin_rank;
+  int64_t mesh_id = 0;  // counts the uploads
   Buf rerun_large, rerun_full, rerun_exact, loc, sizes, offs, drops, stats64,
       work, rel_work;
   Buf scan_tmp;
@@ -286,6 +298,7 @@ struct rpd_ctx {
   RunCaps graph_cap{};
   rpd_run_cfg graph_cfg{};
   double graph_headroom = 0;
+  int64_t graph_bins = 0;  // cells of the candidate grid
   std::vector<int64_t> graph_sig;
   // learned proposals: features, model (fp32 master, Adam state, bf16
   // copies), certificate and fallback
@@ -691,6 +704,8 @@ int rpd_upload_batch(rpd_ctx* ctx, int32_t n_inst,
   ctx->n_tet = (int32_t)nt_tot;
   ctx->has_sites = false;
   ctx->has_subset = false;
+  ctx->bins.ready = ctx->sub_bins.ready = false;
+  ++ctx->mesh_id;
   ctx->has_results = false;
   ctx->adj_ready = false;
   HIP_TRY(ctx->vert.need((size_t)nv_tot * 32));
@@ -823,7 +838,7 @@ int init_state(rpd_ctx* ctx, RunState& R) {
                  ctx->knn_off.as<int64_t>(), ctx->knn_ids.as<int32_t>(),
                  ctx->knn_near.as<int32_t>(),
                  ctx->knn_site_near.as<double4>(), nullptr};
-  HIP_TRY(ctx->counters.need(8 * 4));
+  HIP_TRY(ctx->counters.need(kCounters * 4));
   R.cnt = ctx->counters.as<int32_t>();
   // the bisector of every neighbour-list entry, read by the plane masks
   // and the clip instead of two dependent loads and the arithmetic
@@ -926,96 +941,157 @@ int sort_keys(rpd_ctx* ctx, hipStream_t s, Buf& a, Buf& b, int64_t n,
   return 0;
 }
 
-// plain path: site boxes, binning, reference relation over the bins
+// the tets (of the subset) in the order of the candidate grid
+int ensure_bins(rpd_ctx* ctx, hipStream_t s, int64_t n_bins,
+                const InstInfo* inst_d) {
+  const bool sub = ctx->has_subset;
+  rpd_ctx::Bins& B = sub ? ctx->sub_bins : ctx->bins;
+  if (B.ready) return 0;
+  if (t_capture) return fail(ctx, "rpd_graph_build: tet bins not built");
+  const int32_t nt = ctx->n_tet;
+  const DevMesh M{ctx->n_vert, nt, ctx->vert.as<double4>(),
+                  ctx->tet_v.as<int4>(), ctx->tet_fid.as<int4>(),
+                  ctx->tet_meta.as<TetMeta>()};
+  const uint8_t* sel = sub ? ctx->tet_sel.as<uint8_t>() : nullptr;
+  HIP_TRY(B.first.need(((size_t)n_bins + 1) * 4));
+  HIP_TRY(B.tet.need((size_t)nt * 4));
+  HIP_TRY(B.c0.need((size_t)nt * 16));
+  HIP_TRY(B.c1.need((size_t)nt * 16));
+  HIP_TRY(B.c2.need((size_t)nt * 16));
+  HIP_TRY(ctx->bin_n.need(((size_t)n_bins + 1) * 4));
+  HIP_TRY(ctx->bin_rank.need((size_t)nt * 8));
+  HIP_TRY(zero32(s, ctx->bin_n.p, n_bins + 1));
+  hipLaunchKernelGGL(k_tet_bin, dim3(ceil_div(nt, 256)), dim3(256), 0, s, M,
+                     inst_d, ctx->tet_inst.as<int32_t>(), sel,
+                     ctx->bin_n.as<int32_t>(), ctx->bin_rank.as<int2>());
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(exclusive_sum<int32_t>(ctx, ctx->bin_n.as<int32_t>(),
+                                 B.first.as<int32_t>(), n_bins + 1));
+  hipLaunchKernelGGL(k_tet_bin_fill, dim3(ceil_div(nt, 256)), dim3(256), 0, s,
+                     M, inst_d, ctx->tet_inst.as<int32_t>(), sel,
+                     ctx->bin_rank.as<int2>(), B.first.as<int32_t>(),
+                     B.tet.as<int32_t>(), B.c0.as<float4>(),
+                     B.c1.as<float4>(), B.c2.as<float4>());
+  HIP_TRY(hipGetLastError());
+  B.ready = true;
+  return 0;
+}
+
+// related pairs that a run on the resident batch may need, generously: the
+// cells of t tets and s sites grow about as t + t^(2/3) s^(1/3) +
+// 16 t^(1/3) s^(2/3) + 20 s (a run that needs more is sized by its count)
+int64_t pairs_guess(const rpd_ctx* ctx) {
+  double n = 4096;
+  for (const rpd_ctx::Inst& I : ctx->inst) {
+    const double t = I.n_tet, s = I.n_site;
+    n += 2 * t + 3 * std::cbrt(t * t * s) + 30 * std::cbrt(t * s * s) + 40 * s;
+  }
+  return (int64_t)n;
+}
+
+// plain path: site boxes, then the reference relation over the tets of the
+// grid rows they reach
 int plain_candidates(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out) {
   hipStream_t s = R.s;
   const int32_t nt = R.nt, ns = R.ns;
-  const int64_t n_bins = R.n_bins;
+  if (int rc = ensure_bins(ctx, s, R.n_bins, R.inst_d)) return rc;
+  const rpd_ctx::Bins& bb = ctx->has_subset ? ctx->sub_bins : ctx->bins;
+  const MeshBins B{bb.first.as<int32_t>(), bb.tet.as<int32_t>(),
+                   bb.c0.as<float4>(), bb.c1.as<float4>(),
+                   bb.c2.as<float4>()};
+  const size_t nk = (size_t)std::max<int64_t>(ctx->n_knn, 1);
   HIP_TRY(ctx->bbox.need((size_t)std::max(ns, 1) * 48));
-  if (ns > 0)
-    hipLaunchKernelGGL(k_site_bbox, dim3(ns), dim3(64), 0, s, R.S, R.inst_d,
-                       R.site_inst_d, ctx->bbox.as<double>(),
-                       ctx->knn_near.as<int32_t>(),
-                       ctx->knn_site_near.as<double4>(), R.cnt + 0);
+  HIP_TRY(ctx->rel_pl.need(nk * 16));
+  HIP_TRY(ctx->rel_aux.need(nk * 8));
+  HIP_TRY(ctx->parts.need(((size_t)ns + 1) * 8));
+  HIP_TRY(ctx->part_off.need(((size_t)ns + 1) * 8));
+  hipLaunchKernelGGL(k_site_bbox, dim3(ns + 1), dim3(64), 0, s, R.S, R.inst_d,
+                     R.site_inst_d, ctx->bbox.as<double>(),
+                     ctx->rel_pl.as<float4>(), ctx->rel_aux.as<float2>(),
+                     ctx->parts.as<int64_t>(),
+                     (unsigned long long*)(R.cnt + 16), R.cnt + 0);
   HIP_TRY(hipGetLastError());
   if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[10], s));
-  // sphere -> bin registrations: count, expand, radix sort by
-  // (bin, sphere), bin starts by binary search
-  HIP_TRY(ctx->reg_n.need(((size_t)ns + 1) * 8));
-  HIP_TRY(ctx->reg_off.need(((size_t)ns + 1) * 8));
-  hipLaunchKernelGGL(k_bin_nreg, dim3(ceil_div(ns + 1, 256)), dim3(256), 0, s,
-                     ns, ctx->bbox.as<double>(), R.inst_d, R.site_inst_d,
-                     ctx->reg_n.as<int64_t>());
-  HIP_TRY(hipGetLastError());
-  HIP_TRY(exclusive_sum<int64_t>(ctx, ctx->reg_n.as<int64_t>(),
-                                 ctx->reg_off.as<int64_t>(), ns + 1));
-  int64_t n_reg = 0;
-  if (R.graph)
-    n_reg = R.cap.n_reg;
-  else
-    HIP_TRY(read_back(ctx, s, {{&n_reg, ctx->reg_off.as<int64_t>() + ns, 8}}));
-  if (n_reg >= (1LL << 31))
-    return fail(ctx, "rpd_run: too many sphere-bin registrations");
-  ctx->st.n_bin_registrations = n_reg;
-  R.seen.n_reg = n_reg;
-  HIP_TRY(ctx->keys_a.need((size_t)std::max<int64_t>(n_reg, 1) * 8));
-  HIP_TRY(ctx->keys_b.need((size_t)std::max<int64_t>(n_reg, 1) * 8));
-  HIP_TRY(ctx->bin_start.need((n_bins + 1) * 4));
-  HIP_TRY(ctx->bin_ids.need((size_t)std::max<int64_t>(n_reg, 1) * 4));
-  if (n_reg > 0) {
-    int end_bit = 32;
-    while ((1LL << (end_bit - 32)) < n_bins + 1) ++end_bit;
-    // (a captured run pads its registrations past the device count with a
-    // key above every bin)
-    hipLaunchKernelGGL(k_bin_expand, dim3(ceil_div(n_reg, 256)), dim3(256), 0,
-                       s, ns, n_reg, ctx->bbox.as<double>(), R.inst_d,
-                       R.site_inst_d, ctx->reg_off.as<int64_t>(),
-                       ctx->keys_a.as<uint64_t>(),
-                       R.graph ? ctx->reg_off.as<int64_t>() + ns : nullptr,
-                       end_bit >= 64 ? ~0ull : (1ull << end_bit) - 1);
-    HIP_TRY(hipGetLastError());
-    if (int rc = sort_keys(ctx, s, ctx->keys_a, ctx->keys_b, n_reg, end_bit))
-      return rc;
-  }
-  hipLaunchKernelGGL(k_bin_starts,
-                     dim3(ceil_div(std::max<int64_t>(n_bins + 1, n_reg), 256)),
-                     dim3(256), 0, s, n_bins, n_reg, ctx->keys_b.as<uint64_t>(),
-                     ctx->bin_start.as<int32_t>(), ctx->bin_ids.as<int32_t>(),
-                     R.graph ? ctx->reg_off.as<int64_t>() + ns : nullptr);
-  HIP_TRY(hipGetLastError());
-  if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[11], s));
+  HIP_TRY(exclusive_sum<int64_t>(ctx, ctx->parts.as<int64_t>(),
+                                 ctx->part_off.as<int64_t>(), ns + 1));
   HIP_TRY(ctx->tet_count.need(((size_t)nt + 1) * 8));
   HIP_TRY(ctx->tet_off.need(((size_t)nt + 1) * 8));
-  HIP_TRY(ctx->tet_pass.need(((size_t)nt + 1) * 2 * 8));  // 2 words per tet
-  HIP_TRY(zero32(s, ctx->tet_count.as<int64_t>() + nt, 2));
-  hipLaunchKernelGGL(k_tet_count, dim3(ceil_div(nt, 256)), dim3(256), 0, s,
-                     R.M, R.S, R.inst_d, R.tet_inst_d,
-                     ctx->bin_start.as<int32_t>(), ctx->bin_ids.as<int32_t>(),
-                     ctx->tet_count.as<int64_t>(), ctx->tet_pass.as<uint64_t>(),
-                     R.cfg.count_work
-                         ? ctx->rel_work.as<unsigned long long>()
-                         : nullptr,
-                     ctx->has_subset ? ctx->tet_sel.as<uint8_t>() : nullptr);
-  HIP_TRY(hipGetLastError());
-  if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[12], s));
-  HIP_TRY(exclusive_sum<int64_t>(ctx, ctx->tet_count.as<int64_t>(),
-                                 ctx->tet_off.as<int64_t>(), nt + 1));
-  int64_t n_cand = 0;
-  if (R.graph)
-    n_cand = R.cap.n_cand;
-  else
-    HIP_TRY(
-        read_back(ctx, s, {{&n_cand, ctx->tet_off.as<int64_t>() + nt, 8}}));
+  HIP_TRY(zero32(s, ctx->tet_count.p, 2 * ((int64_t)nt + 1)));
+  if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[11], s));
+  uint32_t* const n_pairs = (uint32_t*)(R.cnt + 8);
+  unsigned long long* const count = ctx->tet_count.as<unsigned long long>();
+  // wavefronts that walk the parts: enough to fill the chip, few enough
+  // that most take several; their chunks of the pair list, small where the
+  // list is
+  const uint32_t waves =
+      (uint32_t)std::max<int64_t>(1, std::min<int64_t>(6144, (int64_t)ns * 8));
+  const uint32_t chunk = nt < 200000 ? 64 : 256;
+  int64_t cap = R.graph ? R.cap.n_cand : pairs_guess(ctx);
+  int64_t n_cand = 0, place_room = 0;
+  for (;;) {
+    int64_t room = cap + (int64_t)waves * chunk;
+    HIP_TRY(ctx->pairs.need((size_t)room * 8));
+    if (!R.graph)  // (what a larger run left)
+      room = std::max<int64_t>(room, ctx->pairs.cap / 8);
+    if (ns > 0)
+      hipLaunchKernelGGL(
+          k_rel_pairs, dim3(waves), dim3(64), 0, s, R.M, R.S, B, R.inst_d,
+          R.site_inst_d, ctx->bbox.as<double>(), ctx->rel_pl.as<float4>(),
+          ctx->rel_aux.as<float2>(), ctx->part_off.as<int64_t>(), count,
+          ctx->pairs.as<int2>(), n_pairs, chunk, room,
+          R.cfg.count_work ? ctx->rel_work.as<unsigned long long>() : nullptr);
+    HIP_TRY(hipGetLastError());
+    if (R.graph) {
+      hipLaunchKernelGGL(k_rel_guard, dim3(ceil_div(nt, 256)), dim3(256), 0, s,
+                         nt, n_pairs, room, count, R.cnt + 7);
+      HIP_TRY(hipGetLastError());
+    }
+    if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[12], s));
+    HIP_TRY(exclusive_sum<int64_t>(ctx, ctx->tet_count.as<int64_t>(),
+                                   ctx->tet_off.as<int64_t>(), nt + 1));
+    if (R.graph) {
+      n_cand = cap;
+      place_room = room;
+      break;
+    }
+    int64_t reg64[64], n_reg = 0;
+    uint32_t n_listed = 0;
+    HIP_TRY(read_back(ctx, s, {{&n_cand, ctx->tet_off.as<int64_t>() + nt, 8},
+                               {&n_listed, n_pairs, 4},
+                               {reg64, R.cnt + 16, sizeof(reg64)}}));
+    for (int q = 0; q < 64; ++q) n_reg += reg64[q];
+    if (n_reg >= (1LL << 31))
+      return fail(ctx, "rpd_run: too many sphere-bin registrations");
+    ctx->st.n_bin_registrations = n_reg;
+    if (n_cand >= (1LL << 31))
+      return fail(ctx, "rpd_run: too many candidates");
+    place_room = room;
+    if (n_listed <= room) break;
+    cap = n_cand;  // again, with a list that holds them
+    HIP_TRY(zero32(s, ctx->tet_count.p, 2 * ((int64_t)nt + 1)));
+    HIP_TRY(zero32(s, n_pairs, 1));
+  }
   R.seen.n_cand = n_cand;
-  HIP_TRY(ctx->cand.need((size_t)std::max<int64_t>(n_cand, 1) * sizeof(Cand)));
-  HIP_TRY(ctx->rel_ids.need((size_t)std::max<int64_t>(n_cand, 1) * 4));
-  hipLaunchKernelGGL(k_tet_fill, dim3(ceil_div(nt, 256)), dim3(256), 0, s, R.M,
-                     R.S, R.inst_d, R.tet_inst_d, ctx->bin_start.as<int32_t>(),
-                     ctx->bin_ids.as<int32_t>(), ctx->tet_off.as<int64_t>(),
-                     ctx->tet_pass.as<uint64_t>(), ctx->cand.as<Cand>(),
-                     ctx->rel_ids.as<int32_t>(),
-                     ctx->has_subset ? ctx->tet_sel.as<uint8_t>() : nullptr,
-                     n_cand, R.cnt + 7);
+  const size_t nc = (size_t)std::max<int64_t>(n_cand, 1);
+  HIP_TRY(ctx->pair_seg.need(nc * 8));
+  HIP_TRY(ctx->tet_fill.need((size_t)nt * 4));
+  HIP_TRY(zero32(s, ctx->tet_fill.p, nt));
+  HIP_TRY(ctx->cand.need(nc * sizeof(Cand)));
+  HIP_TRY(ctx->rel_ids.need(nc * 4));
+  if (n_cand > 0) {
+    // (the listed entries: the pairs and the chunks' unused ones)
+    hipLaunchKernelGGL(
+        k_pair_place,
+        dim3(ceil_div(std::min(place_room, n_cand + (int64_t)waves * chunk),
+                      256)),
+        dim3(256), 0, s, place_room, n_cand, n_pairs, ctx->pairs.as<int2>(),
+        ctx->tet_off.as<int64_t>(), ctx->tet_fill.as<int32_t>(),
+        ctx->pair_seg.as<int2>());
+    hipLaunchKernelGGL(k_pair_rank, dim3(ceil_div(n_cand, 256)), dim3(256), 0,
+                       s, n_cand, nt, ctx->pair_seg.as<int2>(),
+                       ctx->tet_off.as<int64_t>(), ctx->cand.as<Cand>(),
+                       ctx->rel_ids.as<int32_t>());
+  }
   HIP_TRY(hipGetLastError());
   if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[13], s));
   *n_cand_out = n_cand;
@@ -2011,13 +2087,13 @@ int run_config(rpd_ctx* ctx, const rpd_run_cfg* cfg_in, RunState& R) {
 int run_stages(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out,
                int64_t* n_out_out, Sizes3* tot) {
   const rpd_run_cfg& cfg = R.cfg;
-  HIP_TRY(ctx->counters.need(8 * 4));
+  HIP_TRY(ctx->counters.need(kCounters * 4));
   R.s = ctx->stream;
   hipStream_t s = R.s;
   if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[0], s));
   ctx->n_small_ev = 0;
   ctx->n_reads = 0;
-  HIP_TRY(zero32(s, ctx->counters.p, 8));
+  HIP_TRY(zero32(s, ctx->counters.p, kCounters));
   if (int rc = init_state(ctx, R)) return rc;
   if (cfg.count_work) {
     HIP_TRY(ctx->rel_work.need(64 * 4 * 8));
@@ -2505,6 +2581,7 @@ std::vector<int64_t> graph_signature(const rpd_ctx* ctx) {
     v.push_back(I.n_site);
   }
   v.push_back(ctx->has_subset);
+  v.push_back(ctx->mesh_id);  // a new mesh has its own bins and domain boxes
   v.push_back((int64_t)(intptr_t)ctx->pin_inst);
   v.push_back((int64_t)g_buf_generation.load());
   return v;
@@ -2545,7 +2622,6 @@ int rpd_graph_build(rpd_ctx* ctx, const rpd_run_cfg* cfg, double headroom) {
   const RunCaps& n = ctx->seen;
   const double f = 1.0 + headroom;
   RunCaps cap;
-  cap.n_reg = grow(n.n_reg, f, 1024);
   cap.n_cand = grow(n.n_cand, f, 1024);
   cap.n_mid = grow(n.n_mid, f, 256);
   cap.n_full = grow(n.n_full, f, 256);
@@ -2584,8 +2660,7 @@ int rpd_graph_build(rpd_ctx* ctx, const rpd_run_cfg* cfg, double headroom) {
     cap.c_full = grow(n.c_full, f, 256);
     cap.c_exact = grow(n.c_exact, f, 256);
   }
-  if (cap.n_reg >= (1LL << 31) ||
-      cap.n_cand + cap.added + cap.fb >= (1LL << 31) ||
+  if (cap.n_cand + cap.added + cap.fb >= (1LL << 31) ||
       cap.miss >= (1LL << 31) || cap.incl >= (1LL << 31))
     return fail(ctx, "rpd_graph_build: capacities over 2^31 entries");
   // the neighbour lists and the tables sized by them may lengthen in later
@@ -2594,6 +2669,10 @@ int rpd_graph_build(rpd_ctx* ctx, const rpd_run_cfg* cfg, double headroom) {
     const size_t nk = (size_t)std::max<int64_t>(grow(ctx->n_knn, f, 1024), 1);
     HIP_TRY(ctx->knn_bis.need(nk * 32));
     HIP_TRY(ctx->knn_bisf.need(nk * 16));
+    if (!R.cfg.learned) {
+      HIP_TRY(ctx->rel_pl.need(nk * 16));
+      HIP_TRY(ctx->rel_aux.need(nk * 8));
+    }
     HIP_TRY(ctx->knn_ids.need_keep(nk * 4, (size_t)ctx->n_knn * 4,
                                    ctx->stream));
     HIP_TRY(ctx->knn_near.need_keep(nk * 4, (size_t)ctx->n_knn * 4,
@@ -2661,6 +2740,7 @@ int rpd_graph_build(rpd_ctx* ctx, const rpd_run_cfg* cfg, double headroom) {
   ctx->graph_cfg = R.cfg;
   ctx->graph_headroom = headroom;
   ctx->graph_sig = graph_signature(ctx);
+  ctx->graph_bins = P.n_bins;
   ctx->st = st_eager;  // the eager run's results are the current ones
   return 0;
 }
@@ -2676,9 +2756,11 @@ int rpd_graph_run(rpd_ctx* ctx, int32_t* replayed) {
   // the batch or a buffer changed since the capture, or the neighbour
   // lists outgrew the captured bisector table: capture again (its eager run
   // gives this call's results)
-  if (graph_signature(ctx) != ctx->graph_sig ||
-      (size_t)std::max<int64_t>(ctx->n_knn, 1) * 32 > ctx->knn_bis.cap ||
-      (size_t)std::max<int64_t>(ctx->n_knn, 1) * 16 > ctx->knn_bisf.cap) {
+  const size_t nk = (size_t)std::max<int64_t>(ctx->n_knn, 1);
+  if (graph_signature(ctx) != ctx->graph_sig || nk * 32 > ctx->knn_bis.cap ||
+      nk * 16 > ctx->knn_bisf.cap ||
+      (!ctx->graph_cfg.learned &&
+       (nk * 16 > ctx->rel_pl.cap || nk * 8 > ctx->rel_aux.cap))) {
     const rpd_run_cfg c = ctx->graph_cfg;
     return rpd_graph_build(ctx, &c, ctx->graph_headroom);
   }
@@ -2698,12 +2780,16 @@ int rpd_graph_run(rpd_ctx* ctx, int32_t* replayed) {
   ctx->has_results = false;
   ctx->adj_ready = false;
   hipStream_t s = ctx->stream;
+  if (!learned && ctx->has_subset && !ctx->sub_bins.ready)  // a new subset
+    if (int rc = ensure_bins(ctx, s, ctx->graph_bins,
+                             ctx->inst_dev.as<InstInfo>()))
+      return rc;
   HIP_TRY(hipEventRecord(ctx->ev[0], s));
   HIP_TRY(hipGraphLaunch(ctx->graph_exec, s));
   HIP_TRY(hipEventRecord(ctx->ev[4], s));
   const RunCaps& cap = ctx->graph_cap;
   const int64_t nb = ceil_div(learned ? cap.incl : cap.n_cand, kCB);
-  int64_t st64[4], drops[kDropSlots * 9], n_cand = 0, n_reg = 0, n1 = 0;
+  int64_t st64[4], drops[kDropSlots * 9], n_cand = 0, n1 = 0, reg64[64];
   int32_t cnt[8], reop[64], nf = 0;
   int64_t gc[3 + 2 * kClosureRounds];
   Sizes3 tot{0, 0, 0};
@@ -2719,7 +2805,7 @@ int rpd_graph_run(rpd_ctx* ctx, int32_t* replayed) {
     items.push_back({gc, ctx->gcnt.p, (size_t)(3 + 2 * cap.rounds) * 8});
     items.push_back({&nf, ctx->flag_pos.as<int32_t>() + ctx->n_tet, 4});
   } else {
-    items.push_back({&n_reg, ctx->reg_off.as<int64_t>() + ctx->n_site, 8});
+    items.push_back({reg64, ctx->counters.as<int32_t>() + 16, sizeof(reg64)});
   }
   HIP_TRY(read_back(ctx, s, items));
   const bool mid = small_caps(ctx->graph_cfg.small_caps).V < SmallCaps::V;
@@ -2730,7 +2816,7 @@ int rpd_graph_run(rpd_ctx* ctx, int32_t* replayed) {
                         : cnt[1] > cap.n_full) ||
                    cnt[2] > cap.n_exact);
   const bool over =
-      cnt[7] != 0 || tiers_over || n_reg > cap.n_reg ||
+      cnt[7] != 0 || tiers_over ||
       (learned ? (n1 > cap.n_cand || n_cand > cap.incl)
                : n_cand > cap.n_cand) ||
       tot.cells > cap.cells || tot.words > cap.words || tot.areas > cap.areas;
@@ -2740,7 +2826,6 @@ int rpd_graph_run(rpd_ctx* ctx, int32_t* replayed) {
     if (tiers_over) why += " re-run tiers";
     if (learned ? n1 > cap.n_cand : n_cand > cap.n_cand) why += " candidates";
     if (learned && n_cand > cap.incl) why += " output candidates";
-    if (n_reg > cap.n_reg) why += " bin registrations";
     if (tot.cells > cap.cells || tot.words > cap.words ||
         tot.areas > cap.areas)
       why += " output stream";
@@ -2763,7 +2848,8 @@ int rpd_graph_run(rpd_ctx* ctx, int32_t* replayed) {
   st.n_rerun_large = cnt[1];
   st.n_rerun_exact = cnt[2];
   st.n_bbox_fallback = cnt[0];
-  st.n_bin_registrations = n_reg;
+  if (!learned)
+    for (int q = 0; q < 64; ++q) st.n_bin_registrations += reg64[q];
   st.tet_k = (int32_t)st64[2];
   st.n_host_reads = 1;  // the counts, once, after the graph
   if (learned) {
@@ -2813,6 +2899,7 @@ int rpd_set_tet_subset(rpd_ctx* ctx, int32_t n, const int32_t* tet_ids) {
                          hipMemcpyHostToDevice, ctx->stream));
   HIP_TRY(wait_stream(ctx, ctx->stream));
   ctx->has_subset = true;
+  ctx->sub_bins.ready = false;
   return 0;
 }
 
@@ -3116,12 +3203,14 @@ int rpd_run_noalloc(rpd_ctx* ctx, const rpd_instance_desc* desc,
     int32_t n_vert, n_tet, n_site;
     int64_t n_knn;
     bool has_mesh, has_sites, has_subset, last_geometry, has_results,
-        adj_ready;
+        adj_ready, bins_ready, sub_ready;
+    int64_t mesh_id;
     rpd_stats st;
   } sv{ctx->inst,          ctx->n_vert,      ctx->n_tet,
        ctx->n_site,        ctx->n_knn,       ctx->has_mesh,
        ctx->has_sites,     ctx->has_subset,  ctx->last_geometry,
-       ctx->has_results,   ctx->adj_ready,   ctx->st};
+       ctx->has_results,   ctx->adj_ready,   ctx->bins.ready,
+       ctx->sub_bins.ready, ctx->mesh_id,    ctx->st};
   Arena A;
   A.base = static_cast<char*>(ctx->scratch_dev);
   A.cap = kScratchBytes;
@@ -3146,6 +3235,9 @@ int rpd_run_noalloc(rpd_ctx* ctx, const rpd_instance_desc* desc,
       c->last_geometry = s.last_geometry;
       c->has_results = s.has_results;
       c->adj_ready = s.adj_ready;
+      c->bins.ready = s.bins_ready;
+      c->sub_bins.ready = s.sub_ready;
+      c->mesh_id = s.mesh_id;
       c->st = s.st;
     }
   } guard{ctx, A, sv};

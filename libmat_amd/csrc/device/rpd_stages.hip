@@ -5,11 +5,13 @@
 //                  the neighbour bisectors pushed outwards by the largest
 //                  tet radius; the bbox of that polytope contains the
 //                  centroid of every tet the sphere can relate to
-//   k_bin_*        spheres registered into a uniform grid of tet centroids
-//   k_tet_count /  one thread per tet: the reference's tet-sphere relation
-//   k_tet_fill     (voronoi.cu:154-193) over the spheres of its bin, emitted
-//                  in ascending site id, plus the mask of neighbour planes
-//                  that may cut the tet
+//   k_tet_bin*     the mesh's tets in the order of a uniform grid of their
+//                  centroids (once per mesh or tet subset)
+//   k_rel_pairs    wavefronts per sphere: the reference's tet-sphere relation
+//                  (voronoi.cu:154-193) over the tets of the grid rows that
+//                  its polytope reaches
+//   k_pair_*       the related pairs in tet order, ascending site id
+//   k_cand_mask    the mask of neighbour planes that may cut the tet
 //   k_clip         (rpd_kernels.hip) the clip; tiers: small capacity, full
 //                  capacity, full capacity with exact arithmetic
 //   k_compact_*    deterministic compaction into the output stream
@@ -81,9 +83,9 @@ __device__ __forceinline__ int bin_coord(double x, double org, double inv,
 // the centroid plus a margin).  Output bbox (lo, hi); empty if lo > hi.
 // The bisectors are applied nearest first (ascending signed distance of
 // the sphere centre to the bisector), so the polytope shrinks early and
-// later planes rarely cut; that order is also written to knn_near, where
-// the relation test uses it to meet a rejecting neighbour early (the test
-// itself does not depend on the order).
+// later planes rarely cut; the relation test takes the planes in that order
+// too, to meet a rejecting neighbour early (its outcome does not depend on
+// the order).
 // The chain of clips bounds it (one site's wavefront is as long as the
 // kernel for small sets), so the vertices stay in registers, two slots per
 // lane, and a clip's edges are found by comparing all of them with each
@@ -102,12 +104,61 @@ __device__ __forceinline__ int32_t near_word(const DevSites& S, int m) {
 }
 __device__ __forceinline__ int near_id(int32_t w) { return w & 0x7fffffff; }
 
+// bin range of a sphere's candidate box; false if empty
+__device__ __forceinline__ bool bin_range(const double* b, const BinGrid& g,
+                                          int r[6]) {
+  if (b[0] > b[3] || b[1] > b[4] || b[2] > b[5]) return false;
+  for (int a = 0; a < 3; ++a) {
+    r[a] = bin_coord(b[a], g.org[a], g.inv_bs, g.dim[a]);
+    r[3 + a] = bin_coord(b[3 + a], g.org[a], g.inv_bs, g.dim[a]);
+  }
+  return true;
+}
+
+// grid rows (y, z) that one part of a sphere's relation test takes: at most
+// kRelRows, fewer where a row of the box is long, so that no part holds much
+// more than a thousand tets (six a bin); a fixed 16 left single parts of
+// 6,000 tets to run alone at the end
+constexpr int kRelRows = 16;
+__device__ __forceinline__ int rel_rows(const int r[6]) {
+  return min(kRelRows, max(1, 170 / (r[3] - r[0] + 1)));
+}
+
+// A bisector for the relation test: binary32 coefficients about the centre
+// of the instance's domain box, aux.x a bound of the error of its computed
+// value at any point of the box (three fused products and the rounding of
+// plane and point: 5 u sum |e_a| h_a + 4 u |d|, h the box's half extents,
+// u = 2^-24; 4e-7 covers it) plus the rounding of the two binary64 power
+// distances that decide the relation, aux.y the distance term of a tet's
+// corners from its centroid.  Beyond aux.x the sign is the relation's.
+__device__ __forceinline__ void rel_plane(const rpd_d4& e, const rpd_d4& si,
+                                          const double4& sm, double nrm,
+                                          double rho, const double* dom,
+                                          float4& pl, float2& aux) {
+  double d = e.w, h = 0, far2 = 0;
+  for (int a = 0; a < 3; ++a) {
+    const double ea = a == 0 ? e.x : a == 1 ? e.y : e.z;
+    const double c = 0.5 * (dom[a] + dom[3 + a]);
+    const double m = fmax(fabs(dom[a]), fabs(dom[3 + a]));
+    d += ea * c;
+    h += fabs(ea) * (dom[3 + a] - dom[a]) * 0.5;
+    far2 += m * m;
+  }
+  const double s2 = si.x * si.x + si.y * si.y + si.z * si.z + fabs(si.w) +
+                    sm.x * sm.x + sm.y * sm.y + sm.z * sm.z + fabs(sm.w);
+  pl = make_float4((float)e.x, (float)e.y, (float)e.z, (float)d);
+  aux.x = (float)(4e-7 * (h + fabs(d)) + 1e-14 * (far2 + s2)) + 1e-36f;
+  aux.y = (float)(nrm * rho) * 1.000001f;
+}
+
 __global__ __launch_bounds__(64) void k_site_bbox(DevSites S,
                                                   const InstInfo* inst,
                                                   const int32_t* site_inst,
                                                   double* bbox,  // 6/site
-                                                  int32_t* knn_near,
-                                                  double4* knn_site_near,
+                                                  float4* rel_pl,
+                                                  float2* rel_aux,
+                                                  int64_t* parts,
+                                                  unsigned long long* reg64,
                                                   int32_t* n_fallback) {
   constexpr int kVS = kBoxV / 64;
   __shared__ double4 s_pl[kBoxP];
@@ -116,16 +167,31 @@ __global__ __launch_bounds__(64) void k_site_bbox(DevSites S,
   __shared__ uint32_t s_new[kBoxV];
   const int i = blockIdx.x;
   const int lane = threadIdx.x;
-  if (i >= S.n_site) return;
+  if (i >= S.n_site) {  // the block past the last site ends the part counts
+    if (lane == 0) parts[i] = 0;
+    return;
+  }
   const InstInfo& I = inst[site_inst[i]];
   const double* dom = I.dom;
   const double rho = I.rho;
   double* out = bbox + 6 * (int64_t)i;
-  if (S.flags[i] != 1u) {
-    if (lane == 0) {
-      out[0] = out[1] = out[2] = 1.0;
-      out[3] = out[4] = out[5] = -1.0;
+  // the box, the parts its grid rows make, and its bins (a statistic)
+  auto finish = [&](const double b[6]) {
+    if (lane != 0) return;
+    for (int a = 0; a < 6; ++a) out[a] = b[a];
+    int r[6];
+    int64_t rows = 0, n = 0;
+    if (bin_range(b, I.g, r)) {
+      n = rel_rows(r);
+      rows = (int64_t)(r[4] - r[1] + 1) * (r[5] - r[2] + 1);
+      atomicAdd(reg64 + (blockIdx.x & 63),
+                (unsigned long long)(rows * (r[3] - r[0] + 1)));
     }
+    parts[i] = rows ? (rows + n - 1) / n : 0;
+  };
+  const double none[6] = {1.0, 1.0, 1.0, -1.0, -1.0, -1.0};
+  if (S.flags[i] != 1u) {
+    finish(none);
     return;
   }
   const int64_t k0 = S.knn_off[i];
@@ -153,23 +219,14 @@ __global__ __launch_bounds__(64) void k_site_bbox(DevSites S,
       s_near[r] = S.knn_ids[k0 + k];
     }
     wsync();
-    for (int k = lane; k < deg; k += 64) {
-      const int m = s_near[k];
-      knn_near[k0 + k] = near_word(S, m);
-      const double4 sm = S.site[m];
-      knn_site_near[k0 + k] = sm;
-      if (k < kBoxP - 6) {  // the pushed bisector
-        const rpd_d4 e = rpd_bisector(si, rpd_d4{sm.x, sm.y, sm.z, sm.w});
-        const double nrm = sqrt(e.x * e.x + e.y * e.y + e.z * e.z);
-        s_pl[6 + k] = make_double4(e.x, e.y, e.z, e.w + nrm * rho);
-      }
-    }
-  } else {
-    for (int k = lane; k < deg; k += 64) {
-      const int m = S.knn_ids[k0 + k];
-      knn_near[k0 + k] = near_word(S, m);
-      knn_site_near[k0 + k] = S.site[m];
-    }
+  }
+  for (int k = lane; k < deg; k += 64) {
+    const double4 sm = S.site[ranked ? s_near[k] : S.knn_ids[k0 + k]];
+    const rpd_d4 e = rpd_bisector(si, rpd_d4{sm.x, sm.y, sm.z, sm.w});
+    const double nrm = sqrt(e.x * e.x + e.y * e.y + e.z * e.z);
+    if (k < kBoxP - 6)  // the pushed bisector
+      s_pl[6 + k] = make_double4(e.x, e.y, e.z, e.w + nrm * rho);
+    rel_plane(e, si, sm, nrm, rho, dom, rel_pl[k0 + k], rel_aux[k0 + k]);
   }
   // box planes: x >= x0, x <= x1, y >= y0, y <= y1, z >= z0, z <= z1
   if (lane < 6) {
@@ -249,17 +306,12 @@ __global__ __launch_bounds__(64) void k_site_bbox(DevSites S,
     nv += n_new - n_out;
   }
   if (fail) {
-    if (lane == 0) {
-      for (int a = 0; a < 6; ++a) out[a] = dom[a];
-      atomicAdd(n_fallback, 1);
-    }
+    if (lane == 0) atomicAdd(n_fallback, 1);
+    finish(dom);
     return;
   }
   if (empty) {
-    if (lane == 0) {
-      out[0] = out[1] = out[2] = 1.0;
-      out[3] = out[4] = out[5] = -1.0;
-    }
+    finish(none);
     return;
   }
   double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
@@ -280,86 +332,15 @@ __global__ __launch_bounds__(64) void k_site_bbox(DevSites S,
       lo[a] = fmin(lo[a], __shfl_xor(lo[a], off));
       hi[a] = fmax(hi[a], __shfl_xor(hi[a], off));
     }
-  if (lane == 0) {
-    double ext = fmax(fmax(dom[3] - dom[0], dom[4] - dom[1]), dom[5] - dom[2]);
-    double eps = 1e-7 * ext;  // covers the rounding of the vertices
-    for (int a = 0; a < 3; ++a) {
-      out[a] = lo[a] - eps;
-      out[3 + a] = hi[a] + eps;
-    }
-  }
+  const double ext =
+      fmax(fmax(dom[3] - dom[0], dom[4] - dom[1]), dom[5] - dom[2]);
+  const double eps = 1e-7 * ext;  // covers the rounding of the vertices
+  const double b[6] = {lo[0] - eps, lo[1] - eps, lo[2] - eps,
+                       hi[0] + eps, hi[1] + eps, hi[2] + eps};
+  finish(b);
 }
 
-// bin range of a sphere's candidate box; false if empty
-__device__ __forceinline__ bool bin_range(const double* b, const BinGrid& g,
-                                          int r[6]) {
-  if (b[0] > b[3] || b[1] > b[4] || b[2] > b[5]) return false;
-  for (int a = 0; a < 3; ++a) {
-    r[a] = bin_coord(b[a], g.org[a], g.inv_bs, g.dim[a]);
-    r[3 + a] = bin_coord(b[3 + a], g.org[a], g.inv_bs, g.dim[a]);
-  }
-  return true;
-}
-
-// number of bins each sphere registers into
-__global__ __launch_bounds__(256) void k_bin_nreg(int32_t n_site,
-                                                  const double* bbox,
-                                                  const InstInfo* inst,
-                                                  const int32_t* site_inst,
-                                                  int64_t* nreg) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i > n_site) return;
-  if (i == n_site) {
-    nreg[i] = 0;
-    return;
-  }
-  int r[6];
-  nreg[i] = bin_range(bbox + 6 * (int64_t)i, inst[site_inst[i]].g, r)
-                ? (int64_t)(r[3] - r[0] + 1) * (r[4] - r[1] + 1) *
-                      (r[5] - r[2] + 1)
-                : 0;
-}
-
-// one thread per registration: key = bin << 32 | sphere
-__global__ __launch_bounds__(256) void k_bin_expand(int32_t n_site,
-                                                    int64_t n_reg,
-                                                    const double* bbox,
-                                                    const InstInfo* inst,
-                                                    const int32_t* site_inst,
-                                                    const int64_t* reg_off,
-                                                    uint64_t* keys,
-                                                    const int64_t* n_reg_dev,
-                                                    uint64_t pad) {
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n_reg) return;
-  if (n_reg_dev && q >= dev_count(n_reg, n_reg_dev)) {
-    keys[q] = pad;  // sorts after every registration
-    return;
-  }
-  // sphere i with reg_off[i] <= q < reg_off[i+1]
-  int lo = 0, hi = n_site;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (reg_off[mid] <= q)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  const int i = lo;
-  const InstInfo& I = inst[site_inst[i]];
-  const BinGrid& g = I.g;
-  int r[6];
-  bin_range(bbox + 6 * (int64_t)i, g, r);
-  const int64_t k = q - reg_off[i];
-  const int64_t nx = r[3] - r[0] + 1, ny = r[4] - r[1] + 1;
-  const int64_t x = r[0] + k % nx, y = r[1] + (k / nx) % ny,
-                z = r[2] + k / (nx * ny);
-  const uint64_t bin = (uint64_t)I.bin_base + x +
-                       (uint64_t)g.dim[0] * (y + (uint64_t)g.dim[1] * z);
-  keys[q] = (bin << 32) | (uint32_t)i;
-}
-
-// bin_start[b] = first registration of bin >= b in the sorted keys
+// bin_start[b] = first key of bin >= b in the sorted keys (sphere grid)
 __global__ __launch_bounds__(256) void k_bin_starts(int64_t n_bins,
                                                     int64_t n_reg_cap,
                                                     const uint64_t* keys,
@@ -437,94 +418,326 @@ __device__ __forceinline__ int64_t tet_bin(const double c[3],
   return x + (int64_t)g.dim[0] * (y + (int64_t)g.dim[1] * z);
 }
 
-__global__ __launch_bounds__(256) void k_tet_count(DevMesh M, DevSites S,
-                                                   const InstInfo* inst,
-                                                   const int32_t* tet_inst,
-                                                   const int32_t* bin_start,
-                                                   const int32_t* bin_ids,
-                                                   int64_t* tet_count,
-                                                   uint64_t* tet_pass,
-                                                   unsigned long long* work,
-                                                   const uint8_t* tet_sel) {
+// The tets in grid order: bin b (its x fastest, then y, then z) holds
+// positions [first[b], first[b + 1]); per position the tet and its corners,
+// binary32 about the centre of the domain box: (x0 y0 z0 x1), (y1 z1 x2 y2),
+// (z2 x3 y3 z3).
+struct MeshBins {
+  const int32_t* first;
+  const int32_t* tet;
+  const float4* c0;
+  const float4* c1;
+  const float4* c2;
+};
+
+// bin of every (selected) tet and its rank there; bin_n was cleared.  The
+// ranks follow the atomics' order, which nothing depends on.
+__global__ __launch_bounds__(256) void k_tet_bin(DevMesh M,
+                                                 const InstInfo* inst,
+                                                 const int32_t* tet_inst,
+                                                 const uint8_t* tet_sel,
+                                                 int32_t* bin_n,
+                                                 int2* tet_bin_rank) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= M.n_tet) return;
-  if (tet_sel && !tet_sel[t]) {  // outside the tet subset: no candidates
-    tet_count[t] = 0;
-    return;
-  }
+  if (t >= M.n_tet || (tet_sel && !tet_sel[t])) return;
   TetLoad L;
   load_tet(M, t, L);
   double c[3];
   tet_centroid(L, c);
   const InstInfo& I = inst[tet_inst[t]];
-  const int64_t b = I.bin_base + tet_bin(c, I.g);
-  int64_t n = 0;
-  // bit r of (pass0, pass1): the r-th site of the bin list relates
-  uint64_t pass0 = 0, pass1 = 0;
-  uint32_t iters = 0;
-  const int q0 = bin_start[b], q1 = bin_start[b + 1];
-  for (int q = q0; q < q1; ++q) {
-    const int i = bin_ids[q];
-    // (the candidate-box test of the centroid is left to the binning: it
-    // passes 3 of 4 entries and costs more than it saves)
-    const bool r = relation(S, L, i, &iters);
-    n += r;
-    const int d = q - q0;
-    if (r && d < 64) pass0 |= 1ull << d;
-    if (r && d >= 64 && d < 128) pass1 |= 1ull << (d - 64);
-  }
-  tet_count[t] = n;
-  tet_pass[t] = pass0;
-  tet_pass[(int64_t)M.n_tet + t] = pass1;
-  if (work) {  // entries, neighbour tests (count_work)
-    unsigned long long* w = work + 4 * (blockIdx.x & 63);
-    atomicAdd(w + 0, (unsigned long long)(q1 - q0));
-
-    atomicAdd(w + 1, (unsigned long long)iters);
-  }
+  const int32_t b = (int32_t)(I.bin_base + tet_bin(c, I.g));
+  tet_bin_rank[t] = make_int2(b, atomicAdd(bin_n + b, 1));
 }
 
-__global__ __launch_bounds__(256) void k_tet_fill(
-    DevMesh M, DevSites S, const InstInfo* inst, const int32_t* tet_inst,
-    const int32_t* bin_start, const int32_t* bin_ids, const int64_t* tet_off,
-    const uint64_t* tet_pass, Cand* cand, int32_t* rel_ids,
-    const uint8_t* tet_sel, int64_t cap, int32_t* overflow) {
+__global__ __launch_bounds__(256) void k_tet_bin_fill(
+    DevMesh M, const InstInfo* inst, const int32_t* tet_inst,
+    const uint8_t* tet_sel, const int2* tet_bin_rank, const int32_t* first,
+    int32_t* tet, float4* c0, float4* c1, float4* c2) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= M.n_tet) return;
-  if (tet_sel && !tet_sel[t]) return;
-  // over a captured pipeline's capacity: the entries below it are still
-  // written (every slot a later launch reads holds a pair of this run)
-  if (tet_off[t + 1] > cap && (tet_off[t] < cap || t == 0)) overflow[0] = 1;
-  if (tet_off[t] >= cap) return;
+  if (t >= M.n_tet || (tet_sel && !tet_sel[t])) return;
+  const int2 br = tet_bin_rank[t];
+  const int32_t p = first[br.x] + br.y;
   TetLoad L;
   load_tet(M, t, L);
-  double c[3];
-  tet_centroid(L, c);
-  const InstInfo& I = inst[tet_inst[t]];
-  const int64_t b = I.bin_base + tet_bin(c, I.g);
-  int64_t o = tet_off[t];
-  const uint64_t pass0 = tet_pass[t];
-  const uint64_t pass1 = tet_pass[(int64_t)M.n_tet + t];
-  const int q0 = bin_start[b];
-  for (int q = q0; q < bin_start[b + 1]; ++q) {
-    const int i = bin_ids[q];
-    // the first 128 outcomes come from the counting pass
-    uint32_t iters = 0;
-    const int d = q - q0;
-    const bool r = d < 64    ? ((pass0 >> d) & 1)
-                   : d < 128 ? ((pass1 >> (d - 64)) & 1)
-                             : relation(S, L, i, &iters);
-    if (!r) continue;
-    if (o >= cap) break;
-    Cand c;
-    c.tet = t;
-    c.seed = i;
-    c.m0 = 0;
-    c.m1 = 0;
-    cand[o] = c;
-    rel_ids[o] = i;
-    ++o;
+  const double* dom = inst[tet_inst[t]].dom;
+  float v[12];
+  for (int a = 0; a < 3; ++a) {
+    const double c = 0.5 * (dom[a] + dom[3 + a]);
+    for (int k = 0; k < 4; ++k)
+      v[3 * k + a] = (float)((&L.V[k].x)[a] - c);
   }
+  tet[p] = t;
+  c0[p] = make_float4(v[0], v[1], v[2], v[3]);
+  c1[p] = make_float4(v[4], v[5], v[6], v[7]);
+  c2[p] = make_float4(v[8], v[9], v[10], v[11]);
+}
+
+// the relation in binary64 over the neighbour list as it is (for the few
+// pairs that the binary32 planes leave open)
+__device__ __noinline__ bool relation_exact(const DevMesh& M,
+                                            const DevSites& S, int t, int i) {
+  TetLoad L;
+  load_tet(M, t, L);
+  const rpd_d4 si = ld4(S.site + i);
+  double pdi[4];
+  for (int k = 0; k < 4; ++k)
+    pdi[k] = rpd_power_dist(L.V[k].x, L.V[k].y, L.V[k].z, si);
+  for (int64_t q = S.knn_off[i]; q < S.knn_off[i + 1]; ++q) {
+    const rpd_d4 sm = ld4(S.site + S.knn_ids[q]);
+    bool ok = false;
+    for (int k = 0; k < 4; ++k)
+      ok = ok || rpd_power_dist(L.V[k].x, L.V[k].y, L.V[k].z, sm) > pdi[k];
+    if (!ok) return false;
+  }
+  return true;
+}
+
+// Tet-sphere relation (voronoi.cu:154-193), sphere by sphere: a tet is
+// related to sphere i iff every neighbour's bisector leaves one of its
+// corners on i's side.  A part takes kRelRows grid rows (y, z) of the
+// sphere's box: one quad of lanes per row bounds the x range that the pushed
+// planes leave of it; the tets of the ranges are then tested 64 at a time,
+// their corners read contiguously, the planes read from LDS by all lanes at
+// once, nearest first, until no lane is left.  Values within a plane's error
+// bound leave a pair open, and relation_exact decides it.
+//
+// Bound by instruction issue (18 per plane and 64 tets).  One thread per tet
+// over the spheres registered in its bin, in binary64, was bound by the
+// divergence of 64 different lists and, on small meshes, by their length:
+// 1.57 M tets, 18,000 sites: binning, counting and filling 2.8 ms, this
+// with the pair lists 0.65 ms; 16 instances of 2,000 to 200,000 tets with up
+// to 20,000 sites (bin lists past 128, tested twice) 11.7 -> 0.57 ms; 6,000
+// tets 0.55 -> 0.04 ms.
+//
+// Related pairs are counted per tet (nothing waits for these atomics) and go
+// to an unordered list.  A wavefront takes list
+// entries in chunks (one atomic at one address for 64 pairs took 2.0 ms of
+// 2.5 at 3.5 M pairs) and marks what it leaves of its last one.
+constexpr int kRelPl = 128;
+__global__ __launch_bounds__(64) void k_rel_pairs(
+    DevMesh M, DevSites S, MeshBins B, const InstInfo* inst,
+    const int32_t* site_inst, const double* bbox, const float4* rel_pl,
+    const float2* rel_aux, const int64_t* part_off,
+    unsigned long long* tet_count, int2* pairs, uint32_t* n_pairs,
+    uint32_t chunk, int64_t cap, unsigned long long* work) {
+  __shared__ float4 s_pl[kRelPl];
+  __shared__ float2 s_aux[kRelPl];
+  __shared__ int32_t s_first[kRelRows];
+  __shared__ int32_t s_pref[kRelRows + 1];
+  const int lane = threadIdx.x;
+  const int n_site = S.n_site;
+  const int64_t n_parts = part_off[n_site];
+  uint32_t pos = 0, end = 0;  // the rest of this wavefront's chunk
+  for (int64_t part = blockIdx.x; part < n_parts; part += gridDim.x) {
+    // the sphere: part_off[i] <= part < part_off[i + 1]
+    int i = 0, hi = n_site;
+    while (hi - i > 1) {
+      const int step = (hi - i + 63) / 64;
+      const int at = i + lane * step;
+      const uint64_t le = ballot(at < hi && part_off[at] <= part);
+      i += (63 - __clzll((long long)le)) * step;  // lane 0 always holds
+      hi = min(hi, i + step);
+    }
+    const InstInfo& I = inst[site_inst[i]];
+    const BinGrid& g = I.g;
+    const int64_t k0 = S.knn_off[i];
+    const int deg = (int)(S.knn_off[i + 1] - k0);
+    const int np = min(deg, kRelPl);
+    wsync();
+    for (int k = lane; k < ((np + 3) & ~3); k += 64) {
+      s_pl[k] = k < np ? rel_pl[k0 + k] : make_float4(0, 0, 0, 1);
+      s_aux[k] = k < np ? rel_aux[k0 + k] : make_float2(0, 0);
+    }
+    wsync();
+    int r[6];
+    bin_range(bbox + 6 * (int64_t)i, g, r);
+    const int ny = r[4] - r[1] + 1;
+    const int rows = ny * (r[5] - r[2] + 1);
+    const int rpp = rel_rows(r);
+    const int row = (int)(part - part_off[i]) * rpp + (lane & (kRelRows - 1));
+    int len = 0;
+    if (row < rows && (lane & (kRelRows - 1)) < rpp) {
+      const int y = r[1] + row % ny, z = r[2] + row / ny;
+      // the row's box about the domain centre (the last bin of a capped
+      // grid reaches to the end of the domain), 1e-6 of a bin wider
+      const double bs = 1.0 / g.inv_bs;
+      double o[3];
+      for (int a = 0; a < 3; ++a)
+        o[a] = g.org[a] - 0.5 * (I.dom[a] + I.dom[3 + a]);
+      const float ylo = (float)(o[1] + (y - 1e-6) * bs);
+      const float yhi = y == g.dim[1] - 1
+                            ? (float)(0.500001 * (I.dom[4] - I.dom[1]) + 1e-6 * bs)
+                            : (float)(o[1] + (y + 1 + 1e-6) * bs);
+      const float zlo = (float)(o[2] + (z - 1e-6) * bs);
+      const float zhi = z == g.dim[2] - 1
+                            ? (float)(0.500001 * (I.dom[5] - I.dom[2]) + 1e-6 * bs)
+                            : (float)(o[2] + (z + 1 + 1e-6) * bs);
+      float xlo = -INFINITY, xhi = INFINITY;
+      for (int k = lane / kRelRows; k < np; k += 64 / kRelRows) {
+        const float4 p = s_pl[k];
+        const float2 q = s_aux[k];
+        // p.x x + t >= 0 for some point of the row, or no tet there relates
+        const float t = (p.w + q.y + q.x) + fmaxf(p.y * ylo, p.y * yhi) +
+                        fmaxf(p.z * zlo, p.z * zhi) + q.x;
+        const float x = -t / p.x;
+        if (p.x > 0)
+          xlo = fmaxf(xlo, x);
+        else if (p.x < 0)
+          xhi = fminf(xhi, x);
+        else if (t < 0)
+          xhi = -INFINITY;
+      }
+#pragma unroll
+      for (int off = kRelRows; off < 64; off <<= 1) {
+        xlo = fmaxf(xlo, __shfl_xor(xlo, off));
+        xhi = fminf(xhi, __shfl_xor(xhi, off));
+      }
+      // bins of [xlo, xhi], with 1e-3 of a bin for the rounding
+      const float inv = (float)g.inv_bs, ox = (float)o[0];
+      const float flo = (xlo - ox) * inv - 1e-3f, fhi = (xhi - ox) * inv + 1e-3f;
+      const int a = max(r[0], (int)fminf(fmaxf(floorf(flo), -1.f), (float)(g.dim[0] - 1)));
+      const int b = min(r[3], (int)fminf(fmaxf(floorf(fhi), -1.f), (float)(g.dim[0] - 1)));
+      if (a <= b) {
+        const int64_t base =
+            I.bin_base + (int64_t)g.dim[0] * (y + (int64_t)g.dim[1] * z);
+        const int32_t f0 = B.first[base + a];
+        len = B.first[base + b + 1] - f0;
+        if (lane < kRelRows) s_first[lane] = f0;
+      }
+    }
+    // tets before each row of the part
+    int pre = len;
+#pragma unroll
+    for (int off = 1; off < kRelRows; off <<= 1) {
+      const int v = __shfl_up(pre, off);
+      if ((lane & (kRelRows - 1)) >= off) pre += v;
+    }
+    if (lane < kRelRows) s_pref[lane + 1] = pre;
+    if (lane == 0) s_pref[0] = 0;
+    wsync();
+    const int total = s_pref[kRelRows];
+    uint32_t tests = 0;
+    for (int f0 = 0; f0 < total; f0 += 64) {
+      const int f = f0 + lane;
+      int q = 0;  // the row: s_pref[q] <= f < s_pref[q + 1]
+#pragma unroll
+      for (int w = kRelRows / 2; w > 0; w >>= 1)
+        if (s_pref[q + w] <= f) q += w;
+      bool in = f < total, open = deg > kRelPl;
+      const int at = in ? s_first[q] + (f - s_pref[q]) : 0;
+      float4 c0 = make_float4(0, 0, 0, 0), c1 = c0, c2 = c0;
+      int t = 0;
+      if (in) {
+        t = B.tet[at];
+        c0 = B.c0[at];
+        c1 = B.c1[at];
+        c2 = B.c2[at];
+      }
+      int k = 0;
+      auto plane = [&](const float4& p, float eps) {
+        const float v0 = fmaf(p.z, c0.z, fmaf(p.y, c0.y, fmaf(p.x, c0.x, p.w)));
+        const float v1 = fmaf(p.z, c1.y, fmaf(p.y, c1.x, fmaf(p.x, c0.w, p.w)));
+        const float v2 = fmaf(p.z, c2.x, fmaf(p.y, c1.w, fmaf(p.x, c1.z, p.w)));
+        const float v3 = fmaf(p.z, c2.w, fmaf(p.y, c2.z, fmaf(p.x, c2.y, p.w)));
+        const float v = fmaxf(fmaxf(v0, v1), fmaxf(v2, v3));
+        in = in && !(v < -eps);
+        open = open || !(v > eps);
+      };
+      // four planes between two looks at the lanes left (their LDS reads
+      // overlap); the list is padded with planes that every point passes
+      for (; k < np && ballot(in) != 0; k += 4) {
+        const float4 p0 = s_pl[k], p1 = s_pl[k + 1], p2 = s_pl[k + 2],
+                     p3 = s_pl[k + 3];
+        const float e0 = s_aux[k].x, e1 = s_aux[k + 1].x, e2 = s_aux[k + 2].x,
+                    e3 = s_aux[k + 3].x;
+        plane(p0, e0);
+        plane(p1, e1);
+        plane(p2, e2);
+        plane(p3, e3);
+      }
+      tests += k;
+      if (ballot(in && open) != 0)
+        if (in && open) in = relation_exact(M, S, t, i);
+      const uint64_t m = ballot(in);
+      if (m != 0) {
+        const uint32_t n = (uint32_t)__popcll(m), rest = end - pos;
+        uint32_t next = 0;  // a new chunk for what the old one has no room for
+        if (n > rest) {
+          if (lane == 0) next = atomicAdd(n_pairs, chunk);
+          next = lane_value(next, 0);
+        }
+        if (in) {
+          const uint32_t w = (uint32_t)lanes_below(m, lane);
+          const int64_t at = w < rest ? pos + w : next + (w - rest);
+          atomicAdd(tet_count + t, 1ull);
+          if (at < cap) pairs[at] = make_int2(t, i);
+        }
+        if (n > rest) {
+          pos = next + (n - rest);
+          end = next + chunk;
+        } else {
+          pos += n;
+        }
+      }
+    }
+    if (work && lane == 0) {  // pairs tested, plane tests (count_work)
+      unsigned long long* w = work + 4 * (blockIdx.x & 63);
+      atomicAdd(w + 0, (unsigned long long)total);
+      atomicAdd(w + 1, (unsigned long long)tests * 64);
+    }
+    wsync();
+  }
+  for (int64_t q = (int64_t)pos + lane; q < end; q += 64)
+    if (q < cap) pairs[q] = make_int2(-1, -1);
+}
+
+// A captured run whose pairs do not fit their list: no pairs at all, and
+// the overflow flag (no later kernel may read an entry that was not written)
+__global__ __launch_bounds__(256) void k_rel_guard(int32_t n_tet,
+                                                   const uint32_t* n_pairs,
+                                                   int64_t cap,
+                                                   unsigned long long* count,
+                                                   int32_t* overflow) {
+  // (the list's room past the captured candidates is the chunks' slack, so
+  // more candidates than captured can fit it: the host sees their count)
+  if ((int64_t)*n_pairs <= cap) return;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n_tet) count[t] = 0;
+  if (t == 0) overflow[0] = 1;
+}
+
+// pairs to their tet's segment, in the order of the atomics (k_pair_rank
+// sorts it away)
+__global__ __launch_bounds__(256) void k_pair_place(
+    int64_t room, int64_t cap, const uint32_t* n_pairs, const int2* pairs,
+    const int64_t* tet_off, int32_t* tet_fill, int2* seg) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t n = (int64_t)*n_pairs;
+  if (n > room || q >= n) return;
+  const int2 p = pairs[q];
+  if (p.x < 0) return;
+  const int64_t at = tet_off[p.x] + atomicAdd(tet_fill + p.x, 1);
+  if (at < cap) seg[at] = p;
+}
+
+// candidates in tet order, ascending sites: each pair's place is the number
+// of smaller sites in its segment
+__global__ __launch_bounds__(256) void k_pair_rank(
+    int64_t cap, int32_t n_tet, const int2* seg, const int64_t* tet_off,
+    Cand* cand, int32_t* rel_ids) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= min(cap, tet_off[n_tet])) return;
+  const int2 p = seg[q];
+  const int64_t o0 = tet_off[p.x], o1 = min(cap, tet_off[p.x + 1]);
+  int64_t at = o0;
+  for (int64_t o = o0; o < o1; ++o) at += seg[o].y < p.y;
+  Cand c;
+  c.tet = p.x;
+  c.seed = p.y;
+  c.m0 = 0;
+  c.m1 = 0;
+  cand[at] = c;
+  rel_ids[at] = p.y;
 }
 
 // the bisector table of the neighbour lists: one wavefront per site

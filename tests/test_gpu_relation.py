@@ -1,0 +1,130 @@
+"""The tet-sphere relation at the edges of its kernel: neighbour lists
+around the plane table's and the box polytope's capacities, one site, no
+site near, ties, grids of one bin, and coordinates far from the origin or
+of another scale.  The relation sets are compared with the oracle's."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+sys.path.insert(0, os.path.join(HERE, "..", "oracle"))
+import oracle  # noqa: E402
+from libmat_amd import prep  # noqa: E402
+from libmat_amd.rpd import Context  # noqa: E402
+from rpd_compare import compare_relation, compare_with_oracle  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    with Context(0) as c:
+        yield c
+
+
+def star(n):
+    """One sphere in the middle with n neighbours around it."""
+    k = np.arange(n) + 0.5
+    ph, th = np.arccos(1 - 2 * k / n), np.pi * (1 + 5 ** 0.5) * k
+    d = np.c_[np.cos(th) * np.sin(ph), np.sin(th) * np.sin(ph), np.cos(ph)]
+    return np.c_[np.r_[[[0.5] * 3], 0.5 + 0.3 * d], np.full(n + 1, 0.01)]
+
+
+def lattice(k):
+    g = (np.arange(k) + 0.5) / k
+    p = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    return np.c_[p, np.full(len(p), 0.05)]
+
+
+def check(ctx, inst):
+    orc = oracle.run(inst, mode=0)
+    ctx.upload(inst)
+    ctx.run()
+    off, ids = ctx.relation()
+    compare_relation(off, ids, orc)
+    # (combinatorics: the relation decides which cells are clipped at all)
+    compare_with_oracle(ctx.download(), orc, check_geometry=False)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 121, 122, 123, 127, 128,
+                               129, 140])
+def test_list_lengths(ctx, n):
+    verts, tets = prep.grid_mesh(4, 0.1, n)
+    check(ctx, prep.build_instance(verts, tets, star(n)))
+
+
+@pytest.mark.parametrize("n,m", [(1, 1), (1, 40), (2, 1), (7, 3), (17, 1),
+                                 (5, 900)])
+def test_uneven_sizes(ctx, n, m):
+    # one bin, one site, fewer tets than a wavefront, many sites per bin
+    verts, tets = prep.grid_mesh(n, 0.1, n)
+    check(ctx, prep.build_instance(verts, tets, prep.spheres(m, 0, n + m)))
+
+
+@pytest.mark.parametrize("k", [2, 4])
+def test_ties(ctx, k):
+    # bisectors on the grid's planes and through its vertices
+    verts, tets = prep.grid_mesh(4, 0.0, 0)
+    check(ctx, prep.build_instance(verts, tets, lattice(k)))
+
+
+@pytest.mark.parametrize("shift,scale", [(1000.0, 1.0), (-3.0e5, 1.0),
+                                         (0.0, 1e-7), (2.0, 1e6)])
+def test_frames(ctx, shift, scale):
+    verts, tets = prep.grid_mesh(6, 0.1, 2)
+    sph = prep.spheres(150, 0, 8)
+    verts = verts * scale + shift
+    sph = np.c_[sph[:, :3] * scale + shift, sph[:, 3] * scale]
+    lo, hi = -1e-6 * scale + shift, (1 + 1e-6) * scale + shift
+    check(ctx, prep.build_instance(verts, tets, sph,
+                                   box=np.array([lo] * 3 + [hi] * 3)))
+
+
+def test_subsets_and_meshes_in_turn(ctx):
+    # the tet order of the grid follows the mesh and the subset in use
+    rng = np.random.default_rng(3)
+    for n, m in ((6, 80), (9, 200), (6, 50)):
+        verts, tets = prep.grid_mesh(n, 0.1, n + m)
+        inst = prep.build_instance(verts, tets, prep.spheres(m, 0, m))
+        ctx.upload(inst)
+        ctx.run()
+        off, ids = ctx.relation()
+        for share in (0.5, 0.02, 1.0):
+            sel = np.sort(rng.choice(inst.n_tet,
+                                     max(1, int(share * inst.n_tet)),
+                                     replace=False))
+            ctx.set_tet_subset(sel)
+            ctx.run()
+            o2, i2 = ctx.relation()
+            cnt = np.zeros(inst.n_tet, np.int64)
+            cnt[sel] = np.diff(off)[sel]
+            assert np.array_equal(np.diff(o2), cnt)
+            assert np.array_equal(i2, np.concatenate(
+                [ids[off[t]:off[t + 1]] for t in sel]))
+        ctx.set_tet_subset(None)
+        ctx.run()
+        o2, i2 = ctx.relation()
+        assert np.array_equal(off, o2) and np.array_equal(ids, i2)
+
+
+def test_graph_follows_a_new_mesh_of_the_same_sizes(ctx):
+    insts = []
+    for seed, scale in ((1, 1.0), (2, 3.0)):
+        verts, tets = prep.grid_mesh(6, 0.1, seed)
+        sph = prep.spheres(40, 0, 5) * scale
+        box = np.array([-1e-6 * scale] * 3 + [(1 + 1e-6) * scale] * 3)
+        insts.append(prep.build_instance(verts * scale, tets, sph, box=box))
+    assert insts[0].n_site == insts[1].n_site
+    ctx.upload(insts[0])
+    ctx.graph_build(headroom=1.0)
+    for inst in (insts[1], insts[0], insts[0]):
+        ctx.upload(inst)
+        ctx.graph_run()
+        got = ctx.download()
+        ctx.run()
+        want = ctx.download()
+        assert np.array_equal(got.cells, want.cells)
+        assert np.array_equal(got.words, want.words)
+        assert np.array_equal(got.geom, want.geom)
