@@ -302,7 +302,8 @@ struct rpd_ctx {
   std::vector<int64_t> graph_sig;
   // learned proposals: features, model (fp32 master, Adam state, bf16
   // copies), certificate and fallback
-  Buf knn, feat, sel, omask, vowner, sg_keys_a, sg_keys_b, sg_start, sg_ids;
+  Buf knn, feat, sel, omask, vowner, sg_keys_a, sg_keys_b, sg_start, sg_ids,
+      sg_first;
   int32_t feat_n = 0;
   Buf mlp_master, mlp_m1, mlp_m2, mlp_w1t, mlp_w2t, mlp_w3t, mlp_w2, mlp_w3,
       mlp_bias;
@@ -1119,10 +1120,16 @@ int learned_features(rpd_ctx* ctx, RunState& R) {
   HIP_TRY(ctx->sg_keys_b.need((size_t)std::max(ns, 1) * 8));
   HIP_TRY(ctx->sg_start.need((size_t)(R.n_sg + 1) * 4));
   HIP_TRY(ctx->sg_ids.need((size_t)std::max(ns, 1) * 4));
+  HIP_TRY(ctx->sg_first.need(ctx->inst.size() * 4));
+  hipLaunchKernelGGL(k_fill32, dim3(ceil_div(ctx->inst.size(), 256)),
+                     dim3(256), 0, s, ctx->sg_first.as<int32_t>(),
+                     (int64_t)ctx->inst.size(), 0x7fffffff);
+  HIP_TRY(hipGetLastError());
   if (ns > 0) {
     hipLaunchKernelGGL(k_sg_keys, dim3(ceil_div(ns, 256)), dim3(256), 0, s,
-                       R.S, R.inst_d, R.site_inst_d,
-                       ctx->sg_keys_a.as<uint64_t>());
+                       R.S, R.inst_d, R.site_inst_d, R.n_sg,
+                       ctx->sg_keys_a.as<uint64_t>(),
+                       ctx->sg_first.as<int32_t>());
     HIP_TRY(hipGetLastError());
     int end_bit = 32;
     while ((1LL << (end_bit - 32)) < R.n_sg + 1) ++end_bit;
@@ -1143,7 +1150,8 @@ int learned_features(rpd_ctx* ctx, RunState& R) {
   hipLaunchKernelGGL(k_vertex_owner, dim3(ceil_div(ctx->n_vert, 256)),
                      dim3(256), 0, s, R.M, R.S, R.inst_d,
                      ctx->vert_inst.as<int32_t>(), ctx->sg_start.as<int32_t>(),
-                     ctx->sg_ids.as<int32_t>(), ctx->vowner.as<int32_t>());
+                     ctx->sg_ids.as<int32_t>(), ctx->sg_first.as<int32_t>(),
+                     ctx->vowner.as<int32_t>());
   HIP_TRY(hipGetLastError());
   if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[14], s));
   // 32-bit proposal entries hold instance-local ids of 16 bits

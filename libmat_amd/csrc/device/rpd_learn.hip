@@ -139,14 +139,32 @@ __device__ __forceinline__ double pdist(const double c[3], const double4& s) {
   return ((dx * dx + dy * dy) + dz * dz) - s.w;
 }
 
-// keys of the site grid: (cell << 32) | site, per instance grid sg
+// keys of the site grid: (cell << 32) | site, per instance grid sg.  A
+// hidden sphere that is kept as a site (no flag, no list) is in no cell: a
+// descent that began at it would end there, the tet's sets would be wrong
+// and the tet re-run on the full relation (with 90 % of the spheres hidden,
+// 125,459 of 265,000 tets, 18.8 ms).  first[b]: the first sphere of instance
+// b that is in a cell.
 __global__ __launch_bounds__(256) void k_sg_keys(DevSites S,
                                                  const InstInfo* inst,
                                                  const int32_t* site_inst,
-                                                 uint64_t* keys) {
+                                                 int64_t n_sg, uint64_t* keys,
+                                                 int32_t* first) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= S.n_site) return;
-  const InstInfo& I = inst[site_inst[i]];
+  const int b_inst = site_inst[i];
+  const bool in = S.flags[i] == 1u || S.knn_off[i + 1] > S.knn_off[i];
+  const int lane = threadIdx.x & 63;
+  // (sites are in instance order: a wavefront's first one of an instance
+  // stands for the others)
+  const uint64_t before = ballot(in) & ((1ull << lane) - 1);
+  const int prev = __shfl(b_inst, before ? 63 - __clzll((long long)before) : 0);
+  if (in && (before == 0 || prev != b_inst)) atomicMin(first + b_inst, i);
+  if (!in) {  // sorts after every cell
+    keys[i] = ((uint64_t)n_sg << 32) | (uint32_t)i;
+    return;
+  }
+  const InstInfo& I = inst[b_inst];
   const double4 s = S.site[i];
   const int x = bin_coord(s.x, I.sg.org[0], I.sg.inv_bs, I.sg.dim[0]);
   const int y = bin_coord(s.y, I.sg.org[1], I.sg.inv_bs, I.sg.dim[1]);
@@ -157,13 +175,14 @@ __global__ __launch_bounds__(256) void k_sg_keys(DevSites S,
 }
 
 // grid start for a descent at point c: least power distance among the
-// spheres of c's cell of the sphere grid (rings up to 2), else the first
-// sphere of the instance
+// spheres of c's cell of the sphere grid (rings up to 2), else the
+// instance's first sphere that is in a cell
 __device__ __forceinline__ int grid_start(const DevSites& S,
                                          const InstInfo& I,
                                          const int32_t* sg_start,
                                          const int32_t* sg_ids,
-                                         const double c[3], double* best) {
+                                         int first, const double c[3],
+                                         double* best) {
   int cur = -1;
   *best = INFINITY;
   const int cx = bin_coord(c[0], I.sg.org[0], I.sg.inv_bs, I.sg.dim[0]);
@@ -191,7 +210,7 @@ __device__ __forceinline__ int grid_start(const DevSites& S,
           }
         }
   if (cur < 0 && I.n_site > 0) {
-    cur = I.site_off;
+    cur = first != 0x7fffffff ? first : I.site_off;
     *best = pdist(c, S.site[cur]);
   }
   return cur;
@@ -222,13 +241,15 @@ __device__ __forceinline__ int descend(const DevSites& S, const double c[3],
 // owner of every mesh vertex (-1 if its instance has no sphere)
 __global__ __launch_bounds__(256) void k_vertex_owner(
     DevMesh M, DevSites S, const InstInfo* inst, const int32_t* vert_inst,
-    const int32_t* sg_start, const int32_t* sg_ids, int32_t* owner) {
+    const int32_t* sg_start, const int32_t* sg_ids, const int32_t* first,
+    int32_t* owner) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= M.n_vert) return;
   const double4 p = M.vert[v];
   const double c[3] = {p.x, p.y, p.z};
   double best;
-  const int st = grid_start(S, inst[vert_inst[v]], sg_start, sg_ids, c, &best);
+  const int b = vert_inst[v];
+  const int st = grid_start(S, inst[b], sg_start, sg_ids, first[b], c, &best);
   owner[v] = st < 0 ? -1 : descend(S, c, st, &best);
 }
 
