@@ -41,21 +41,37 @@ __global__ __launch_bounds__(256) void k_seed_starts(int32_t n_site, int64_t n,
 // one wavefront per site: out[4 s ..] = (sum vol * centroid) / sum vol,
 // sum vol; a site without volume keeps its centre (compute_new_site
 // updates only sites with cell_vol != 0)
-__global__ __launch_bounds__(256) void k_site_centroid(
-    int32_t n_site, const int64_t* start, const int32_t* idx,
-    const double* geom, const double4* site, double* out) {
-  const int lane = threadIdx.x & 63;
-  const int64_t s = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (s >= n_site) return;
-  const int64_t b = start[s], e = start[s + 1];
+// Cells that one wavefront sums; a site with more is cut into chunks of
+// kCentroidCells of its cells.  One wavefront has few loads in flight, so
+// the largest site (30,000 of 3.1 M cells) was the kernel's length: 941 us
+// with a load at a time, 673 us with 8 steps of loads in flight, 117 us with
+// 4 and chunks (three launches).
+constexpr int64_t kCentroidCells = 4096;
+
+// lane-strided sums (volume, volume times centroid) of positions [b, e) of
+// the seed order, then a fixed butterfly: every lane holds the total.  kU
+// steps of loads are in flight, added in their order.
+__device__ __forceinline__ double4 centroid_sum(int64_t b, int64_t e, int lane,
+                                                const int32_t* idx,
+                                                const double4* geom) {
+  constexpr int kU = 4;
   double v = 0, x = 0, y = 0, z = 0;
-  for (int64_t i = b + lane; i < e; i += 64) {
-    const double* g = geom + 4 * (int64_t)idx[i];
-    const double w = g[0];
-    v += w;
-    x += w * g[1];
-    y += w * g[2];
-    z += w * g[3];
+  for (int64_t i0 = b + lane; i0 < e; i0 += 64 * kU) {
+    double4 g[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int64_t i = i0 + 64 * u;
+      g[u] = i < e ? geom[idx[i]] : make_double4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      if (i0 + 64 * u >= e) break;
+      const double w = g[u].x;
+      v += w;
+      x += w * g[u].y;
+      y += w * g[u].z;
+      z += w * g[u].w;
+    }
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -64,19 +80,69 @@ __global__ __launch_bounds__(256) void k_site_centroid(
     y += __shfl_xor(y, off, 64);
     z += __shfl_xor(z, off, 64);
   }
-  if (lane == 0) {
-    const double4 c = site[s];
-    double* o = out + 4 * s;
-    if (v != 0) {
-      o[0] = x / v;
-      o[1] = y / v;
-      o[2] = z / v;
-    } else {
-      o[0] = c.x;
-      o[1] = c.y;
-      o[2] = c.z;
+  return make_double4(v, x, y, z);
+}
+__device__ __forceinline__ void centroid_write(const double4& m,
+                                               const double4& c, double* o) {
+  o[0] = m.x != 0 ? m.y / m.x : c.x;
+  o[1] = m.x != 0 ? m.z / m.x : c.y;
+  o[2] = m.x != 0 ? m.w / m.x : c.z;
+  o[3] = m.x;
+}
+
+// n_large: chunks listed, large sites listed; large[h] = site, its first
+// chunk, its number of chunks, 0; chunks[q] = site, chunk of the site
+__global__ __launch_bounds__(256) void k_site_centroid(
+    int32_t n_site, const int64_t* start, const int32_t* idx,
+    const double4* geom, const double4* site, double* out, int32_t* n_large,
+    int4* large, int2* chunks) {
+  const int lane = threadIdx.x & 63;
+  const int64_t s = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (s >= n_site) return;
+  const int64_t b = start[s], e = start[s + 1];
+  if (e - b > kCentroidCells) {
+    const int n = (int)((e - b + kCentroidCells - 1) / kCentroidCells);
+    int base = 0;
+    if (lane == 0) {
+      base = atomicAdd(n_large, n);
+      large[atomicAdd(n_large + 1, 1)] = make_int4((int)s, base, n, 0);
     }
-    o[3] = v;
+    base = __shfl(base, 0);
+    for (int q = lane; q < n; q += 64) chunks[base + q] = make_int2((int)s, q);
+    return;
+  }
+  const double4 m = centroid_sum(b, e, lane, idx, geom);
+  if (lane == 0) centroid_write(m, site[s], out + 4 * s);
+}
+__global__ __launch_bounds__(256) void k_centroid_chunks(
+    const int64_t* start, const int32_t* idx, const double4* geom,
+    const int32_t* n_large, const int2* chunks, double4* part) {
+  const int lane = threadIdx.x & 63;
+  for (int q = blockIdx.x * 4 + (threadIdx.x >> 6); q < n_large[0];
+       q += gridDim.x * 4) {
+    const int2 c = chunks[q];
+    const int64_t b = start[c.x] + c.y * kCentroidCells;
+    const double4 m = centroid_sum(b, min(b + kCentroidCells, start[c.x + 1]),
+                                   lane, idx, geom);
+    if (lane == 0) part[q] = m;
+  }
+}
+// a large site's chunks, summed in their order
+__global__ __launch_bounds__(64) void k_centroid_large(
+    const int32_t* n_large, const int4* large, const double4* part,
+    const double4* site, double* out) {
+  for (int h = blockIdx.x * 64 + threadIdx.x; h < n_large[1];
+       h += gridDim.x * 64) {
+    const int4 l = large[h];
+    double4 m = part[l.y];
+    for (int q = 1; q < l.z; ++q) {
+      const double4 p = part[l.y + q];
+      m.x += p.x;
+      m.y += p.y;
+      m.z += p.z;
+      m.w += p.w;
+    }
+    centroid_write(m, site[l.x], out + 4 * (int64_t)l.x);
   }
 }
 

@@ -276,7 +276,8 @@ struct rpd_ctx {
   Buf tet_sel;
   bool has_subset = false;
   // per-site centroids of the last run's cells
-  Buf cs_keys_a, cs_keys_b, cs_vals_a, cs_vals_b, cs_start, cs_out;
+  Buf cs_keys_a, cs_keys_b, cs_vals_a, cs_vals_b, cs_start, cs_out, cs_n,
+      cs_large, cs_chunks, cs_part;
   // power-cell adjacency of the last run's cells
   Buf adj_act, adj_euler, adj_cnt, adj_off, adj_nbr, adj_cpar, adj_err;
   Buf tf_ka, tf_kb, tf_va, tf_vb;
@@ -2922,11 +2923,34 @@ int rpd_site_centroids(rpd_ctx* ctx, double* out, const double** dev_out) {
   const int32_t ns = ctx->n_site;
   if (int rc = cells_by_seed(ctx)) return rc;
   HIP_TRY(ctx->cs_out.need((size_t)std::max(ns, 1) * 32));
+  // (a site over kCentroidCells holds at least that many of the cells)
+  const int64_t n = ctx->st.n_cells;
+  const size_t n_big = (size_t)(n / kCentroidCells) + 1;
+  HIP_TRY(ctx->cs_n.need(8));
+  HIP_TRY(ctx->cs_large.need(n_big * 16));
+  HIP_TRY(ctx->cs_chunks.need(2 * n_big * 8));
+  HIP_TRY(ctx->cs_part.need(2 * n_big * 32));
+  HIP_TRY(zero32(s, ctx->cs_n.p, 2));
   if (ns > 0)
     hipLaunchKernelGGL(k_site_centroid, dim3(ceil_div(ns, 4)), dim3(256), 0, s,
                        ns, ctx->cs_start.as<int64_t>(),
-                       ctx->cs_vals_b.as<int32_t>(), ctx->out_geom.as<double>(),
+                       ctx->cs_vals_b.as<int32_t>(),
+                       ctx->out_geom.as<double4>(), ctx->site.as<double4>(),
+                       ctx->cs_out.as<double>(), ctx->cs_n.as<int32_t>(),
+                       ctx->cs_large.as<int4>(), ctx->cs_chunks.as<int2>());
+  if (ns > 0 && n > kCentroidCells) {
+    hipLaunchKernelGGL(
+        k_centroid_chunks,
+        dim3((int)std::min<int64_t>(1024, ceil_div(2 * n_big, 4))), dim3(256),
+        0, s, ctx->cs_start.as<int64_t>(), ctx->cs_vals_b.as<int32_t>(),
+        ctx->out_geom.as<double4>(), ctx->cs_n.as<int32_t>(),
+        ctx->cs_chunks.as<int2>(), ctx->cs_part.as<double4>());
+    hipLaunchKernelGGL(k_centroid_large,
+                       dim3((int)std::min<int64_t>(64, ceil_div(n_big, 64))),
+                       dim3(64), 0, s, ctx->cs_n.as<int32_t>(),
+                       ctx->cs_large.as<int4>(), ctx->cs_part.as<double4>(),
                        ctx->site.as<double4>(), ctx->cs_out.as<double>());
+  }
   HIP_TRY(hipGetLastError());
   if (out && ns > 0)
     HIP_TRY(hipMemcpyAsync(out, ctx->cs_out.p, (size_t)ns * 32,

@@ -15,6 +15,27 @@ def ctx():
         yield c
 
 
+@pytest.mark.parametrize("n,m", [(8, 1), (9, 1), (9, 2), (16, 1), (20, 3),
+                                 (24, 40)])
+def test_centroids_of_large_sites(ctx, n, m):
+    # 3,072 to 82,944 cells, all in one site or spread over a few: 64-bit
+    # sums of at most 10^5 positive terms, so 1e-11 of the value
+    verts, tets = prep.grid_mesh(n, 0.1, n)
+    inst = prep.build_instance(verts, tets, prep.spheres(m, 0, n + m))
+    ctx.upload(inst)
+    ctx.run()
+    res = ctx.download()
+    got = ctx.site_centroids()
+    want = np.c_[inst.sites[:, :3], np.zeros(inst.n_site)]
+    for s in range(inst.n_site):
+        g = res.geom[res.cells["seed"] == s]
+        if g.size and g[:, 0].sum() != 0:
+            want[s, 3] = g[:, 0].sum()
+            want[s, :3] = (g[:, :1] * g[:, 1:]).sum(0) / want[s, 3]
+    assert np.allclose(got, want, rtol=1e-11, atol=1e-11)
+    assert np.array_equal(got, ctx.site_centroids())
+
+
 @pytest.mark.parametrize("rule,m", [(1, 400), (2, 900), (0, 3), (0, 1)])
 def test_owners_with_hidden_spheres_kept(ctx, rule, m):
     # every sphere a site, hidden ones unflagged with an empty list: a tet's
