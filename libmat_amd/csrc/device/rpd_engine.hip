@@ -3340,12 +3340,16 @@ int mlp_alloc(rpd_ctx* ctx) {
   return 0;
 }
 
+MlpCopies mlp_copies(rpd_ctx* ctx) {
+  return MlpCopies{ctx->mlp_w1t.as<uint16_t>(), ctx->mlp_w2t.as<uint16_t>(),
+                   ctx->mlp_w3t.as<uint16_t>(), ctx->mlp_w2.as<uint16_t>(),
+                   ctx->mlp_w3.as<uint16_t>(),  ctx->mlp_bias.as<float>()};
+}
+
 int mlp_pack(rpd_ctx* ctx) {
-  hipLaunchKernelGGL(k_mlp_pack, dim3(ceil_div(kHid * kHid, 256)), dim3(256),
-                     0, ctx->stream, ctx->mlp_master.as<float>(),
-                     ctx->mlp_w1t.as<uint16_t>(), ctx->mlp_w2t.as<uint16_t>(),
-                     ctx->mlp_w3t.as<uint16_t>(), ctx->mlp_w2.as<uint16_t>(),
-                     ctx->mlp_w3.as<uint16_t>(), ctx->mlp_bias.as<float>());
+  hipLaunchKernelGGL(k_mlp_pack, dim3(ceil_div(kNParam, 256)), dim3(256), 0,
+                     ctx->stream, ctx->mlp_master.as<float>(),
+                     mlp_copies(ctx));
   HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -3359,8 +3363,7 @@ int mlp_step(rpd_ctx* ctx, const uint16_t* X, const float* Y, const float* M,
              float* loss_tiles) {
   hipStream_t s = ctx->stream;
   const int tiles = n_rows / 16;
-  const int tpc = 8;
-  const int chunks = (tiles + tpc - 1) / tpc;
+  const int chunks = (tiles + kTilesPerChunk - 1) / kTilesPerChunk;
   HIP_TRY(ctx->tr_xb.need((size_t)n_rows * kIn * 2));
   HIP_TRY(ctx->tr_h1.need((size_t)n_rows * kHid * 2));
   HIP_TRY(ctx->tr_h2.need((size_t)n_rows * kHid * 2));
@@ -3372,35 +3375,29 @@ int mlp_step(rpd_ctx* ctx, const uint16_t* X, const float* Y, const float* M,
   HIP_TRY(ctx->tr_p3.need((size_t)chunks * kHid * kOut * 4));
   HIP_TRY(ctx->tr_pb.need((size_t)chunks * kBiasN * 4));
   const float inv_count = 1.f / (float)std::max(1, n_valid * kOut);
-  hipLaunchKernelGGL(k_mlp_fb, dim3(ceil_div(tiles, 4)), dim3(256), 0, s,
-                     mlp_dev(ctx), X, Y, M, idx, n_rows, pos_w, inv_count,
+  hipLaunchKernelGGL(k_mlp_fb, dim3(tiles), dim3(64 * kFbWaves), 0, s,
+                     mlp_dev(ctx), X, Y, M, idx, pos_w, inv_count,
                      ctx->tr_xb.as<uint16_t>(), ctx->tr_h1.as<uint16_t>(),
                      ctx->tr_h2.as<uint16_t>(), ctx->tr_dz1.as<uint16_t>(),
                      ctx->tr_dz2.as<uint16_t>(), ctx->tr_dz3.as<uint16_t>(),
                      loss_tiles);
   HIP_TRY(hipGetLastError());
   float* pb = ctx->tr_pb.as<float>();
-  hipLaunchKernelGGL(k_mlp_wgrad, dim3((kIn / 16) * (kHid / 16), chunks),
+  hipLaunchKernelGGL(k_mlp_wgrad,
+                     dim3(kGradBlocks1 + kGradBlocks2 + kGradBlocks3, chunks),
                      dim3(64), 0, s, ctx->tr_xb.as<uint16_t>(),
-                     ctx->tr_dz1.as<uint16_t>(), kIn, kHid, tpc, tiles,
-                     ctx->tr_p1.as<float>(), pb, 0);
-  hipLaunchKernelGGL(k_mlp_wgrad, dim3((kHid / 16) * (kHid / 16), chunks),
-                     dim3(64), 0, s, ctx->tr_h1.as<uint16_t>(),
-                     ctx->tr_dz2.as<uint16_t>(), kHid, kHid, tpc, tiles,
-                     ctx->tr_p2.as<float>(), pb, kHid);
-  hipLaunchKernelGGL(k_mlp_wgrad, dim3((kHid / 16) * (kOut / 16), chunks),
-                     dim3(64), 0, s, ctx->tr_h2.as<uint16_t>(),
-                     ctx->tr_dz3.as<uint16_t>(), kHid, kOut, tpc, tiles,
-                     ctx->tr_p3.as<float>(), pb, 2 * kHid);
+                     ctx->tr_h1.as<uint16_t>(), ctx->tr_h2.as<uint16_t>(),
+                     ctx->tr_dz1.as<uint16_t>(), ctx->tr_dz2.as<uint16_t>(),
+                     ctx->tr_dz3.as<uint16_t>(), tiles,
+                     ctx->tr_p1.as<float>(), ctx->tr_p2.as<float>(),
+                     ctx->tr_p3.as<float>(), pb);
   HIP_TRY(hipGetLastError());
   hipLaunchKernelGGL(k_mlp_update, dim3(ceil_div(kNParam, 256)), dim3(256), 0,
                      s, ctx->mlp_master.as<float>(), ctx->mlp_m1.as<float>(),
                      ctx->mlp_m2.as<float>(), ctx->tr_p1.as<float>(),
                      ctx->tr_p2.as<float>(), ctx->tr_p3.as<float>(), pb,
-                     chunks, adam, grad_out);
+                     chunks, adam, grad_out, mlp_copies(ctx));
   HIP_TRY(hipGetLastError());
-  if (adam.apply)
-    if (int rc = mlp_pack(ctx)) return rc;
   return 0;
 }
 

@@ -533,20 +533,7 @@ __global__ __launch_bounds__(256) void k_labels(int32_t n_tet,
 }
 
 // ------------------------------------------------------------------ MLP
-// One wave per 16-row tile.  Activations pass through LDS to turn the
-// D layout of one layer into the A layout of the next.
 constexpr int kActStride = kHid + 8;  // bf16 per LDS row (bank spread)
-
-struct WaveLds {
-  uint16_t h1[16][kActStride];
-  uint16_t h2[16][kActStride];
-  uint16_t dz[16][kOut + 8];
-};
-
-__device__ __forceinline__ void wsync_l() {
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
 
 // X tile rows (A operand, 3 k-blocks); rows with id < 0 are zero
 __device__ __forceinline__ void load_x(const uint16_t* X, int64_t row_id,
@@ -558,57 +545,6 @@ __device__ __forceinline__ void load_x(const uint16_t* X, int64_t row_id,
     } else {
       a[kb] = bf16x4{0, 0, 0, 0};
     }
-  }
-}
-
-// layers 1-2 of one tile into LDS (h1, h2) and layer 3 logits z[nb][i]
-__device__ __forceinline__ void mlp_forward_tile(const MlpDev& P,
-                                                 const bf16x4 a1[3], int l,
-                                                 WaveLds& W, f32x4 z[2]) {
-  const int col = l % 16, rq = 4 * (l / 16);
-#pragma unroll
-  for (int nb = 0; nb < 8; ++nb) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kb = 0; kb < 3; ++kb)
-      acc = mfma(a1[kb], ld_bf4(P.w1t + (16 * nb + col) * kIn + 16 * kb + rq),
-                 acc);
-    const float b = P.b1[16 * nb + col];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      W.h1[rq + i][16 * nb + col] = f2bf(fmaxf(acc[i] + b, 0.f));
-  }
-  wsync_l();
-  bf16x4 a2[8];
-#pragma unroll
-  for (int kb = 0; kb < 8; ++kb) a2[kb] = ld_bf4(&W.h1[col][16 * kb + rq]);
-#pragma unroll
-  for (int nb = 0; nb < 8; ++nb) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kb = 0; kb < 8; ++kb)
-      acc = mfma(a2[kb],
-                 ld_bf4(P.w2t + (16 * nb + col) * kHid + 16 * kb + rq), acc);
-    const float b = P.b2[16 * nb + col];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      W.h2[rq + i][16 * nb + col] = f2bf(fmaxf(acc[i] + b, 0.f));
-  }
-  wsync_l();
-  bf16x4 a3[8];
-#pragma unroll
-  for (int kb = 0; kb < 8; ++kb) a3[kb] = ld_bf4(&W.h2[col][16 * kb + rq]);
-#pragma unroll
-  for (int nb = 0; nb < 2; ++nb) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kb = 0; kb < 8; ++kb)
-      acc = mfma(a3[kb],
-                 ld_bf4(P.w3t + (16 * nb + col) * kHid + 16 * kb + rq), acc);
-    const float b = P.b3[16 * nb + col];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] += b;
-    z[nb] = acc;
   }
 }
 
@@ -737,144 +673,226 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_mlp_infer(
 }
 
 // Training, forward and backward of one minibatch (rows idx[r], -1 = pad):
-// stores the bf16 activations and output gradients the weight-gradient
-// kernel needs, and per-tile loss sums.  Loss: pos_w-weighted binary cross
-// entropy over valid slots, times inv_count.
-__global__ __launch_bounds__(256) void k_mlp_fb(
+// stores the bf16 inputs, activations and output gradients the weight
+// gradients need, as [tile][feature][16 rows] (a lane of a product holds 4
+// rows of one feature: one 8-byte store here, one 8-byte load there), and
+// per-tile loss sums.  Loss: pos_w-weighted binary cross entropy over valid
+// slots, times inv_count.
+//
+// A step has few tiles (64 for 1,024 rows), so its length is one tile's
+// chain of products: a block of 8 waves takes a tile, each wave one of the 8
+// output blocks of a layer, with its weight fragments loaded before the
+// first product; activations pass between the waves through LDS.  One wave
+// per tile, its weights loaded block by block: 30.6 us a step, 13.1 so (1,024
+// rows).
+constexpr int kFbWaves = kHid / 16;
+__global__ __launch_bounds__(64 * kFbWaves) void k_mlp_fb(
     MlpDev P, const uint16_t* X, const float* Y, const float* Mk,
-    const int32_t* idx, int32_t n_rows, float pos_w, float inv_count,
-    uint16_t* XB, uint16_t* H1, uint16_t* H2, uint16_t* DZ1, uint16_t* DZ2,
-    uint16_t* DZ3, float* loss_tile) {
-  __shared__ WaveLds s_w[4];
-  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int32_t* idx, float pos_w, float inv_count, uint16_t* XT,
+    uint16_t* HT1, uint16_t* HT2, uint16_t* DT1, uint16_t* DT2, uint16_t* DT3,
+    float* loss_tile) {
+  __shared__ uint16_t s_h1[16][kActStride];
+  __shared__ uint16_t s_h2[16][kActStride];
+  __shared__ uint16_t s_dz[16][kOut + 8];
+  const int l = threadIdx.x & 63, nb = threadIdx.x >> 6;
   const int col = l % 16, rq = 4 * (l / 16);
-  const int n_tiles = n_rows / 16;
-  const int tile = blockIdx.x * 4 + wv;
-  if (tile >= n_tiles) return;
-  WaveLds& W = s_w[wv];
-  const int64_t row0 = (int64_t)tile * 16;
-  const int64_t src = idx[row0 + col];
-  bf16x4 a1[3];
-  load_x(X, src, l, a1);
-  // the gathered input rows, for dW1
+  const int64_t tile = blockIdx.x;
+  const int64_t row0 = tile * 16;
+  bf16x4 a1[3], w1[3], w2f[8], w3b[2], w2b[8];
+  load_x(X, idx[row0 + col], l, a1);
 #pragma unroll
-  for (int kb = 0; kb < 3; ++kb) {
-    uint2 v;
-    v.x = (uint32_t)(uint16_t)a1[kb][0] | ((uint32_t)(uint16_t)a1[kb][1] << 16);
-    v.y = (uint32_t)(uint16_t)a1[kb][2] | ((uint32_t)(uint16_t)a1[kb][3] << 16);
-    *reinterpret_cast<uint2*>(XB + (row0 + col) * kIn + 16 * kb + rq) = v;
+  for (int kb = 0; kb < 3; ++kb)
+    w1[kb] = ld_bf4(P.w1t + (16 * nb + col) * kIn + 16 * kb + rq);
+#pragma unroll
+  for (int kb = 0; kb < 8; ++kb) {
+    w2f[kb] = ld_bf4(P.w2t + (16 * nb + col) * kHid + 16 * kb + rq);
+    w2b[kb] = ld_bf4(P.w2 + (16 * nb + col) * kHid + 16 * kb + rq);
   }
-  f32x4 z[2];
-  mlp_forward_tile(P, a1, l, W, z);
-  // h1, h2 tiles to global (row-major [row][128])
-  for (int q = l; q < 16 * kHid; q += 64) {
-    const int r = q / kHid, cc = q % kHid;
-    H1[(row0 + r) * kHid + cc] = W.h1[r][cc];
-    H2[(row0 + r) * kHid + cc] = W.h2[r][cc];
-  }
-  // output gradient and loss (D layout: row rq + i, column 16 nb + col)
-  float lsum = 0.f;
 #pragma unroll
-  for (int nb = 0; nb < 2; ++nb)
+  for (int kb = 0; kb < 2; ++kb)
+    w3b[kb] = ld_bf4(P.w3 + (16 * nb + col) * kOut + 16 * kb + rq);
+  // wave 0 makes the logits: its layer-3 weights and the labels
+  bf16x4 w3f[2][8];
+  float y[2][4], mk[2][4];
+  if (nb == 0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = rq + i, k = 16 * nb + col;
-      const int64_t s = idx[row0 + r];
-      float y = 0.f, m = 0.f;
-      if (s >= 0) {
-        y = Y[s * kOut + k];
-        m = Mk[s * kOut + k];
+    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+      for (int kb = 0; kb < 8; ++kb)
+        w3f[k][kb] = ld_bf4(P.w3t + (16 * k + col) * kHid + 16 * kb + rq);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int64_t r = idx[row0 + rq + i];
+        y[k][i] = r >= 0 ? Y[r * kOut + 16 * k + col] : 0.f;
+        mk[k][i] = r >= 0 ? Mk[r * kOut + 16 * k + col] : 0.f;
       }
-      const float zz = z[nb][i];
-      const float w = y > 0.5f ? pos_w : 1.f;
-      const float p = 1.f / (1.f + expf(-zz));
-      const float g = m * w * (p - y) * inv_count;
-      // softplus(z) - y z, stable
-      const float sp = fmaxf(zz, 0.f) + log1pf(expf(-fabsf(zz)));
-      lsum += m * w * (sp - y * zz);
-      const uint16_t gb = f2bf(g);
-      W.dz[r][k] = gb;
-      DZ3[(row0 + r) * kOut + k] = gb;
     }
-  for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
-  if (l == 0) loss_tile[tile] = lsum * inv_count;
-  wsync_l();
-  // dH2 = dZ3 W3^T, dZ2 = dH2 * [h2 > 0]
-  bf16x4 ad[2];
+  }
+  // four rows rq .. rq + 3 of feature f to [tile][feature][16 rows]
+  auto store4 = [&](uint16_t* T, int n_feat, int f, const uint16_t v[4]) {
+    uint2 w;
+    w.x = (uint32_t)v[0] | ((uint32_t)v[1] << 16);
+    w.y = (uint32_t)v[2] | ((uint32_t)v[3] << 16);
+    *reinterpret_cast<uint2*>(T + ((tile * n_feat + f) * 16 + rq)) = w;
+  };
+  // the gathered input rows, for dW1 (a lane holds 4 features of row col)
+  if (nb < 3) {
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb) ad[kb] = ld_bf4(&W.dz[col][16 * kb + rq]);
+    for (int kb = 0; kb < 3; ++kb)
+      if (nb == kb) {
 #pragma unroll
-  for (int nb = 0; nb < 8; ++nb) {
+        for (int i = 0; i < 4; ++i)
+          XT[(tile * kIn + 16 * kb + rq + i) * 16 + col] = (uint16_t)a1[kb][i];
+      }
+  }
+  // layers 1 and 2: this wave's 16 features
+  uint16_t h1[4], h2[4];
+  {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-      acc = mfma(ad[kb], ld_bf4(P.w3 + (16 * nb + col) * kOut + 16 * kb + rq),
-                 acc);
+    for (int kb = 0; kb < 3; ++kb) acc = mfma(a1[kb], w1[kb], acc);
+    const float b = P.b1[16 * nb + col];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int r = rq + i, cc = 16 * nb + col;
-      const float d = bf2f(W.h2[r][cc]) > 0.f ? acc[i] : 0.f;
-      const uint16_t db = f2bf(d);
-      DZ2[(row0 + r) * kHid + cc] = db;
-      acc[i] = bf2f(db);
+      h1[i] = f2bf(fmaxf(acc[i] + b, 0.f));
+      s_h1[rq + i][16 * nb + col] = h1[i];
     }
-    // keep dZ2 for the next product (h2 rows already used for this block)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) W.h2[rq + i][16 * nb + col] = f2bf(acc[i]);
+    store4(HT1, kHid, 16 * nb + col, h1);
   }
-  wsync_l();
-  // dH1 = dZ2 W2^T, dZ1 = dH1 * [h1 > 0]
-  bf16x4 a2[8];
-#pragma unroll
-  for (int kb = 0; kb < 8; ++kb) a2[kb] = ld_bf4(&W.h2[col][16 * kb + rq]);
-#pragma unroll
-  for (int nb = 0; nb < 8; ++nb) {
+  __syncthreads();
+  {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kb = 0; kb < 8; ++kb)
-      acc = mfma(a2[kb], ld_bf4(P.w2 + (16 * nb + col) * kHid + 16 * kb + rq),
-                 acc);
+      acc = mfma(ld_bf4(&s_h1[col][16 * kb + rq]), w2f[kb], acc);
+    const float b = P.b2[16 * nb + col];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int r = rq + i, cc = 16 * nb + col;
-      const float d = bf2f(W.h1[r][cc]) > 0.f ? acc[i] : 0.f;
-      DZ1[(row0 + r) * kHid + cc] = f2bf(d);
+      h2[i] = f2bf(fmaxf(acc[i] + b, 0.f));
+      s_h2[rq + i][16 * nb + col] = h2[i];
     }
+    store4(HT2, kHid, 16 * nb + col, h2);
+  }
+  __syncthreads();
+  // output gradient and loss (D layout: row rq + i, column 16 k + col)
+  if (nb == 0) {
+    float lsum = 0.f;
+    f32x4 z[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int kb = 0; kb < 8; ++kb) {
+      const bf16x4 a = ld_bf4(&s_h2[col][16 * kb + rq]);
+      z[0] = mfma(a, w3f[0][kb], z[0]);
+      z[1] = mfma(a, w3f[1][kb], z[1]);
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const float b = P.b3[16 * k + col];
+      uint16_t gb[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float zz = z[k][i] + b;
+        const float w = y[k][i] > 0.5f ? pos_w : 1.f;
+        const float p = 1.f / (1.f + expf(-zz));
+        const float g = mk[k][i] * w * (p - y[k][i]) * inv_count;
+        // softplus(z) - y z, stable
+        const float sp = fmaxf(zz, 0.f) + log1pf(expf(-fabsf(zz)));
+        lsum += mk[k][i] * w * (sp - y[k][i] * zz);
+        gb[i] = f2bf(g);
+        s_dz[rq + i][16 * k + col] = gb[i];
+      }
+      store4(DT3, kOut, 16 * k + col, gb);
+    }
+    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
+    if (l == 0) loss_tile[tile] = lsum * inv_count;
+  }
+  __syncthreads();
+  // dH2 = dZ3 W3^T, dZ2 = dH2 * [h2 > 0]: over this wave's columns of s_h2
+  // (wave 0 has read them all)
+  {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+      acc = mfma(ld_bf4(&s_dz[col][16 * kb + rq]), w3b[kb], acc);
+    uint16_t d[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      d[i] = f2bf(bf2f(h2[i]) > 0.f ? acc[i] : 0.f);
+      s_h2[rq + i][16 * nb + col] = d[i];
+    }
+    store4(DT2, kHid, 16 * nb + col, d);
+  }
+  __syncthreads();
+  // dH1 = dZ2 W2^T, dZ1 = dH1 * [h1 > 0]
+  {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = 0; kb < 8; ++kb)
+      acc = mfma(ld_bf4(&s_h2[col][16 * kb + rq]), w2b[kb], acc);
+    uint16_t d[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d[i] = f2bf(bf2f(h1[i]) > 0.f ? acc[i] : 0.f);
+    store4(DT1, kHid, 16 * nb + col, d);
   }
 }
 
 // Weight gradient partials: part[chunk][in][out] = sum over the chunk's
-// rows of A[row][in] * DZ[row][out] (MFMA over 16-row k-steps); one wave
-// per 16x16 output block, blockIdx.y = chunk.  The waves of the first input
-// block also write the chunk's column sums of DZ (the bias gradient
-// partials) to part_b[chunk][b_off + out].
+// rows of A[row][in] * DZ[row][out] (MFMA over 16-row k-steps, the chunk's
+// loads ahead of its products); one wave per 16x16 output block of the three
+// weight matrices (blockIdx.x), blockIdx.y = chunk.  The waves of a matrix's
+// first input block also write the chunk's column sums of DZ (the bias
+// gradient partials) to part_b[chunk][b_off + out].
 constexpr int kBiasN = 2 * kHid + kOut;
-__global__ __launch_bounds__(64) void k_mlp_wgrad(const uint16_t* A,
-                                                  const uint16_t* DZ,
-                                                  int32_t in, int32_t out,
-                                                  int32_t tiles_per_chunk,
-                                                  int32_t n_tiles,
-                                                  float* part, float* part_b,
-                                                  int32_t b_off) {
+constexpr int kTilesPerChunk = 8;
+constexpr int kGradBlocks1 = (kIn / 16) * (kHid / 16);
+constexpr int kGradBlocks2 = (kHid / 16) * (kHid / 16);
+constexpr int kGradBlocks3 = (kHid / 16) * (kOut / 16);
+__global__ __launch_bounds__(64) void k_mlp_wgrad(
+    const uint16_t* XT, const uint16_t* HT1, const uint16_t* HT2,
+    const uint16_t* DT1, const uint16_t* DT2, const uint16_t* DT3,
+    int32_t n_tiles, float* part1, float* part2, float* part3,
+    float* part_b) {
   const int l = threadIdx.x;
+  int blk = blockIdx.x;
+  const uint16_t *A = XT, *DZ = DT1;
+  float* part = part1;
+  int in = kIn, out = kHid, b_off = 0;
+  if (blk >= kGradBlocks1 + kGradBlocks2) {
+    blk -= kGradBlocks1 + kGradBlocks2;
+    A = HT2;
+    DZ = DT3;
+    part = part3;
+    in = kHid;
+    out = kOut;
+    b_off = 2 * kHid;
+  } else if (blk >= kGradBlocks1) {
+    blk -= kGradBlocks1;
+    A = HT1;
+    DZ = DT2;
+    part = part2;
+    in = kHid;
+    b_off = kHid;
+  }
   const int nbo = out / 16;
-  const int mb = blockIdx.x / nbo, nb = blockIdx.x % nbo;
+  const int mb = blk / nbo, nb = blk % nbo;
   const int chunk = blockIdx.y;
   const int col = l % 16, rq = 4 * (l / 16);
+  const int64_t t0 = (int64_t)chunk * kTilesPerChunk;
+  const int nt = (int)min((int64_t)kTilesPerChunk, n_tiles - t0);
+  bf16x4 a[kTilesPerChunk], b[kTilesPerChunk];
+#pragma unroll
+  for (int t = 0; t < kTilesPerChunk; ++t) {
+    const int64_t tile = t0 + (t < nt ? t : 0);
+    a[t] = ld_bf4(A + (tile * in + 16 * mb + col) * 16 + rq);
+    b[t] = ld_bf4(DZ + (tile * out + 16 * nb + col) * 16 + rq);
+  }
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   float bsum = 0.f;
-  const int t0 = chunk * tiles_per_chunk;
-  const int t1 = min(n_tiles, t0 + tiles_per_chunk);
-  for (int tile = t0; tile < t1; ++tile) {
-    const int64_t r0 = (int64_t)tile * 16 + rq;
-    bf16x4 a, b;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      a[i] = (short)A[(r0 + i) * in + 16 * mb + col];
-      b[i] = (short)DZ[(r0 + i) * out + 16 * nb + col];
-      bsum += bf2f((uint16_t)b[i]);
-    }
-    acc = mfma(a, b, acc);
+  for (int t = 0; t < kTilesPerChunk; ++t) {
+    if (t >= nt) break;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bsum += bf2f((uint16_t)b[t][i]);
+    acc = mfma(a[t], b[t], acc);
   }
   float* p = part + (int64_t)chunk * in * out;
 #pragma unroll
@@ -887,8 +905,33 @@ __global__ __launch_bounds__(64) void k_mlp_wgrad(const uint16_t* A,
   }
 }
 
+// the bf16 copies of one master parameter, in the layouts the MFMA kernels
+// read (biases stay binary32)
+struct MlpCopies {
+  uint16_t *w1t, *w2t, *w3t, *w2, *w3;
+  float* bias;
+};
+__device__ __forceinline__ void pack_param(const MlpCopies& c, int p, float v) {
+  if (p < kOffB1) {  // W1[in][out] -> w1t[out][in]
+    const int q = p - kOffW1;
+    c.w1t[(q % kHid) * kIn + q / kHid] = f2bf(v);
+  } else if (p < kOffW2) {
+    c.bias[p - kOffB1] = v;
+  } else if (p < kOffB2) {
+    const int q = p - kOffW2;
+    c.w2t[(q % kHid) * kHid + q / kHid] = c.w2[q] = f2bf(v);
+  } else if (p < kOffW3) {
+    c.bias[kHid + p - kOffB2] = v;
+  } else if (p < kOffB3) {
+    const int q = p - kOffW3;
+    c.w3t[(q % kOut) * kHid + q / kOut] = c.w3[q] = f2bf(v);
+  } else {
+    c.bias[2 * kHid + p - kOffB3] = v;
+  }
+}
+
 // Gradient of every parameter (fixed summation order), optionally an Adam
-// step on the fp32 master copy.
+// step on the fp32 master copy and its bf16 copies.
 struct AdamArgs {
   float lr, beta1, beta2, eps;
   float bc1, bc2;  // 1 - beta^step
@@ -897,7 +940,7 @@ struct AdamArgs {
 __global__ __launch_bounds__(256) void k_mlp_update(
     float* master, float* m1, float* m2, const float* part1,
     const float* part2, const float* part3, const float* part_b,
-    int32_t n_chunks, AdamArgs a, float* grad_out) {
+    int32_t n_chunks, AdamArgs a, float* grad_out, MlpCopies copies) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= kNParam) return;
   const float* src;
@@ -929,35 +972,18 @@ __global__ __launch_bounds__(256) void k_mlp_update(
     const float vv = a.beta2 * m2[p] + (1.f - a.beta2) * g * g;
     m1[p] = mm;
     m2[p] = vv;
-    master[p] -= a.lr * (mm / a.bc1) / (sqrtf(vv / a.bc2) + a.eps);
+    const float v =
+        master[p] - a.lr * (mm / a.bc1) / (sqrtf(vv / a.bc2) + a.eps);
+    master[p] = v;
+    pack_param(copies, p, v);
   }
 }
 
-// bf16 copies of the master weights in the layouts the MFMA kernels read
+// the copies of the whole master (a model set from outside)
 __global__ __launch_bounds__(256) void k_mlp_pack(const float* master,
-                                                  uint16_t* w1t, uint16_t* w2t,
-                                                  uint16_t* w3t, uint16_t* w2,
-                                                  uint16_t* w3, float* bias) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < kIn * kHid) {  // W1[in][out] -> w1t[out][in]
-    const int i = q / kHid, o = q % kHid;
-    w1t[o * kIn + i] = f2bf(master[kOffW1 + q]);
-  }
-  if (q < kHid * kHid) {
-    const int i = q / kHid, o = q % kHid;
-    const uint16_t v = f2bf(master[kOffW2 + q]);
-    w2t[o * kHid + i] = v;
-    w2[q] = v;
-  }
-  if (q < kHid * kOut) {
-    const int i = q / kOut, o = q % kOut;
-    const uint16_t v = f2bf(master[kOffW3 + q]);
-    w3t[o * kHid + i] = v;
-    w3[q] = v;
-  }
-  if (q < kHid) bias[q] = master[kOffB1 + q];
-  if (q < kHid) bias[kHid + q] = master[kOffB2 + q];
-  if (q < kOut) bias[2 * kHid + q] = master[kOffB3 + q];
+                                                  MlpCopies copies) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < kNParam) pack_param(copies, p, master[p]);
 }
 
 // ------------------------------------------------- learned candidate sets
