@@ -182,8 +182,14 @@ __global__ __launch_bounds__(64, (clip_min_waves<G, C>())) void k_clip(
   __shared__ double4 s_pl[G][P];
   __shared__ int32_t s_src[G][P];
   __shared__ uint8_t s_h[G][P];
-  __shared__ uint8_t s_bn[G][P];
-  __shared__ uint8_t s_cyc[G][P + 1];
+  // the cavity boundary: successor bytes of the serial walk; up to 16
+  // planes, first the planes' directed edges (16 out, 16 in), and the cycle
+  // is packed in a register
+  constexpr bool kPacked = P <= 16;
+  __shared__ uint32_t s_bd[G][kPacked ? P : (P + 3) / 4];
+  __shared__ uint8_t s_cyc[kPacked ? 1 : G][P + 1];
+  uint8_t(*const s_bn)[sizeof(s_bd[0])] =
+      reinterpret_cast<uint8_t(*)[sizeof(s_bd[0])]>(s_bd);
   __shared__ uint32_t s_ver[G][V];
   // s_adj[p]: bit q (q < p) set iff the edge list holds the pair (q, p)
   using AdjT = typename std::conditional<
@@ -384,8 +390,51 @@ __global__ __launch_bounds__(64, (clip_min_waves<G, C>())) void k_clip(
     // conflicting vertex of F goes to nb_v - 1 (j = 1) or just below the
     // (j-1)-th kept vertex of B; the k-th kept vertex of B takes the place
     // of the k-th conflicting vertex of F; a conflicting vertex v of B goes
-    // to v - 1.
-    {
+    // to v - 1.  (Up to 32 vertices the masks are one word.)
+    if constexpr (V <= 32) {
+      const uint32_t cm = (uint32_t)conf_lo;
+      const int keep = nb_v - nr;
+      const int m = keep + (int)((cm >> keep) & 1);
+      const uint32_t lo_m = (1u << m) - 1u;  // m <= nb_v - 1 < 32
+      const uint32_t f = cm & lo_m;
+      const uint32_t b = ~cm & ~lo_m & (nb_v >= 32 ? ~0u : (1u << nb_v) - 1u);
+      uint32_t val[VS];
+      int dst[VS];
+#pragma unroll
+      for (int q = 0; q < VS; ++q) {
+        val[q] = 0;
+        dst[q] = -1;
+      }
+#pragma unroll
+      for (int q = 0; q < VS; ++q) {
+        if (q > 0 && ballot(nb_v > q * L) == 0) break;
+        const int v = q * L + j;
+        if (v < nb_v) {
+          val[q] = s_ver[g][v];
+          const bool c = (cm >> v) & 1;
+          const bool front = v < m;
+          // conflicting in F: the jj-th one of F; kept in B: the kk-th
+          // highest of B takes the kk-th lowest of F's places
+          const int jj = __popc(f & ((2u << v) - 1u));
+          const int kk = __popc(b >> v);
+          int n = front ? jj - 1 : kk;  // set bits to take
+          uint32_t w = front ? __brev(b) : f;
+          dst[q] = front ? v : v - 1;
+          if (front == c && n > 0) {
+            for (int i = 1; i < n; ++i) w &= w - 1;
+            const int at = __ffs((int)w) - 1;
+            dst[q] = front ? 30 - at : at;
+          } else if (front && c) {
+            dst[q] = nb_v - 1;
+          }
+        }
+      }
+      wsync();
+#pragma unroll
+      for (int q = 0; q < VS; ++q)
+        if (dst[q] >= 0) s_ver[g][dst[q]] = val[q];
+      wsync();
+    } else {
       const int nk = nb_v - nr;
       const int m = nk + (int)mbit(conf_lo, conf_hi, nk);
       uint64_t f_lo, f_hi, b_lo, b_hi;  // F's conflicts, B's kept vertices
@@ -438,75 +487,146 @@ __global__ __launch_bounds__(64, (clip_min_waves<G, C>())) void k_clip(
     nb_v -= nr;
     (void)nv_old;
 
-    // ---- cavity boundary (convex_cell.cu:618-678), serial per cell
-    for (int p = j; p < P; p += L) s_bn[g][p] = kEnd;
-    wsync();
+    // ---- cavity boundary (convex_cell.cu:618-678) and its cycle
+    // The reference grows the removed region triangle by triangle (the
+    // serial walk below: one dependent LDS round trip after another, for the
+    // longest of the wavefront's cells).  Where the removed triangles form a
+    // disk -- their directed edges without a reverse make one cycle -- the
+    // walk always ends with that cycle (a disk's triangulation can be grown
+    // in any order), so up to 16 planes it is built at once: every lane adds
+    // its triangles' edges to the planes' masks, lanes then read their
+    // planes' successors, and all lanes hold the cycle, 4 bits a plane.  It
+    // starts at the first removed triangle's first plane; if that plane is
+    // cut off altogether, the reference moves the start to the plane before
+    // it in the last triangle added around it, the second of three when
+    // there are three.  Everything else takes the walk.
+    // (1.57 M tets: 1.77 -> 1.70 ms, the 8-cell shape of 32 vertices 0.90 ->
+    // 0.64 ms on 16 uneven instances, together with the one-word vertex move
+    // and the area sums below.  Growing larger fans for their start in
+    // registers cost more than the walk, 1.76 ms; masks of 32 and 64 bits for
+    // the shapes over 16 planes gave nothing: their walks are few.)
     uint32_t first = kEnd;
-    {
-      int iter = 0, t = nb_v, r = nr;
-      while (r > 0) {
-        if (iter++ > 65535) {
-          status = RPD_INCONSISTENT_BOUNDARY;
-          break;
+    uint64_t cyc = 0;
+    int nbd = 0;
+    bool walk = true;
+    // the plane before plane p in the triangle w (kEnd: p is not in it)
+    auto before = [](uint32_t w, uint32_t p) -> uint32_t {
+      const uint32_t a = w & 255, b = (w >> 8) & 255, c = (w >> 16) & 255;
+      return a == p ? c : b == p ? a : c == p ? b : kEnd;
+    };
+    if constexpr (kPacked) {
+      for (int p = j; p < P; p += L) s_bd[g][p] = 0;
+      wsync();
+      for (int q = j; q < nr; q += L) {
+        const uint32_t w = s_ver[g][nb_v + q];
+        const uint32_t a = w & 255, b = (w >> 8) & 255, c = (w >> 16) & 255;
+        atomicOr(&s_bd[g][a], (1u << b) | (65536u << c));
+        atomicOr(&s_bd[g][b], (1u << c) | (65536u << a));
+        atomicOr(&s_bd[g][c], (1u << a) | (65536u << b));
+      }
+      wsync();
+      uint32_t nx_lo = 0, nx_hi = 0, on = 0;  // bit 16 of on: no simple cycle
+      for (int p = j; p < P; p += L) {
+        const uint32_t w = s_bd[g][p];
+        const uint32_t o = w & ~(w >> 16) & 0xffffu;
+        if (o != 0) {
+          const uint64_t n = (uint64_t)(uint32_t)(__ffs((int)o) - 1) << (4 * p);
+          nx_lo |= (uint32_t)n;
+          nx_hi |= (uint32_t)(n >> 32);
+          on |= (1u << p) | ((o & (o - 1)) ? 65536u : 0u);
         }
-        const uint32_t tw = s_ver[g][t];
-        const uint32_t pa = tw & 255, pb = (tw >> 8) & 255,
-                       pc = (tw >> 16) & 255;
-        const uint32_t ba = s_bn[g][pa], bb = s_bn[g][pb], bc = s_bn[g][pc];
-        const bool in0 = ba != kEnd, in1 = bb != kEnd, in2 = bc != kEnd;
-        const bool n0 = bb == pa, n1 = bc == pb, n2 = ba == pc;
-        bool simple = true;
-        if (!n0 && !n1 && in1) simple = false;
-        if (!n1 && !n2 && in2) simple = false;
-        if (!n2 && !n0 && in0) simple = false;
-        if (!n0 && !n1 && !n2) {
-          if (first == kEnd) {
-            wsync();
-            s_bn[g][pa] = pb;
-            s_bn[g][pb] = pc;
-            s_bn[g][pc] = pa;
-            first = pa;
-            wsync();
-          } else {
-            simple = false;
+      }
+      nx_lo = group_or<L>(nx_lo);
+      nx_hi = group_or<L>(nx_hi);
+      on = group_or<L>(on);
+      const uint64_t nx = ((uint64_t)nx_hi << 32) | nx_lo;
+      const int len = __popc(on & 0xffffu);
+      auto next = [&](uint32_t p) { return (uint32_t)(nx >> (4 * p)) & 15u; };
+      uint32_t at = s_ver[g][nb_v] & 255;
+      if (!((on >> at) & 1) && nr == 3)  // all three lie around it
+        at = before(s_ver[g][nb_v + 1], at) & 31u;
+      if ((on >> at) & 1) {
+        uint32_t p = at;
+        do {
+          cyc |= (uint64_t)p << (4 * nbd);
+          ++nbd;
+          p = next(p);
+        } while (p != at && nbd < len);
+        walk = p != at || nbd != len || on > 0xffffu;
+        first = at;
+      }
+    }
+    if (walk) {
+      first = kEnd;
+      wsync();
+      for (int p = j; p < P; p += L) s_bn[g][p] = kEnd;
+      wsync();
+      {
+        int iter = 0, t = nb_v, r = nr;
+        while (r > 0) {
+          if (iter++ > 65535) {
+            status = RPD_INCONSISTENT_BOUNDARY;
+            break;
           }
+          const uint32_t tw = s_ver[g][t];
+          const uint32_t pa = tw & 255, pb = (tw >> 8) & 255,
+                         pc = (tw >> 16) & 255;
+          const uint32_t ba = s_bn[g][pa], bb = s_bn[g][pb], bc = s_bn[g][pc];
+          const bool in0 = ba != kEnd, in1 = bb != kEnd, in2 = bc != kEnd;
+          const bool n0 = bb == pa, n1 = bc == pb, n2 = ba == pc;
+          bool simple = true;
+          if (!n0 && !n1 && in1) simple = false;
+          if (!n1 && !n2 && in2) simple = false;
+          if (!n2 && !n0 && in0) simple = false;
+          if (!n0 && !n1 && !n2) {
+            if (first == kEnd) {
+              wsync();
+              s_bn[g][pa] = pb;
+              s_bn[g][pb] = pc;
+              s_bn[g][pc] = pa;
+              first = pa;
+              wsync();
+            } else {
+              simple = false;
+            }
+          }
+          if (!simple) {
+            ++t;
+            if (t == nb_v + r) t = nb_v;
+            continue;
+          }
+          wsync();
+          if (!n0) s_bn[g][pa] = pb;
+          if (!n1) s_bn[g][pb] = pc;
+          if (!n2) s_bn[g][pc] = pa;
+          wsync();
+          if (n0 && n1) {
+            if (first == pb) first = s_bn[g][pb];
+            wsync();
+            s_bn[g][pb] = kEnd;
+            wsync();
+          }
+          if (n1 && n2) {
+            if (first == pc) first = s_bn[g][pc];
+            wsync();
+            s_bn[g][pc] = kEnd;
+            wsync();
+          }
+          if (n2 && n0) {
+            if (first == pa) first = s_bn[g][pa];
+            wsync();
+            s_bn[g][pa] = kEnd;
+            wsync();
+          }
+          const int last = nb_v + r - 1;
+          const uint32_t lw = s_ver[g][last];
+          wsync();
+          s_ver[g][t] = lw;
+          s_ver[g][last] = tw;
+          wsync();
+          t = nb_v;
+          --r;
         }
-        if (!simple) {
-          ++t;
-          if (t == nb_v + r) t = nb_v;
-          continue;
-        }
-        wsync();
-        if (!n0) s_bn[g][pa] = pb;
-        if (!n1) s_bn[g][pb] = pc;
-        if (!n2) s_bn[g][pc] = pa;
-        wsync();
-        if (n0 && n1) {
-          if (first == pb) first = s_bn[g][pb];
-          wsync();
-          s_bn[g][pb] = kEnd;
-          wsync();
-        }
-        if (n1 && n2) {
-          if (first == pc) first = s_bn[g][pc];
-          wsync();
-          s_bn[g][pc] = kEnd;
-          wsync();
-        }
-        if (n2 && n0) {
-          if (first == pa) first = s_bn[g][pa];
-          wsync();
-          s_bn[g][pa] = kEnd;
-          wsync();
-        }
-        const int last = nb_v + r - 1;
-        const uint32_t lw = s_ver[g][last];
-        wsync();
-        s_ver[g][t] = lw;
-        s_ver[g][last] = tw;
-        wsync();
-        t = nb_v;
-        --r;
       }
     }
     if (status != RPD_SUCCESS) break;
@@ -517,14 +637,16 @@ __global__ __launch_bounds__(64, (clip_min_waves<G, C>())) void k_clip(
       }
       continue;
     }
-
-    // ---- boundary cycle
-    int nbd = 0;
-    {
+    if (walk) {
+      cyc = 0;
+      nbd = 0;
       uint32_t cir = first;
       do {
         if (nbd >= P || cir >= (uint32_t)P) break;
-        if (j == 0) s_cyc[g][nbd] = (uint8_t)cir;
+        if constexpr (kPacked)
+          cyc |= (uint64_t)cir << (4 * nbd);
+        else if (j == 0)
+          s_cyc[g][nbd] = (uint8_t)cir;
         ++nbd;
         cir = s_bn[g][cir];
       } while (cir != first);
@@ -534,6 +656,13 @@ __global__ __launch_bounds__(64, (clip_min_waves<G, C>())) void k_clip(
       }
     }
     wsync();
+    // plane q of the cycle
+    auto cycle = [&](int q) -> uint32_t {
+      if constexpr (kPacked)
+        return (uint32_t)(cyc >> (4 * q)) & 15u;
+      else
+        return s_cyc[g][q];
+    };
     // ---- new edges (cur, cir) (convex_cell.cu:604-616, 752-758)
     if (nb_e + nbd > E) {
       status = kFull ? RPD_EDGE_OVERFLOW : kStatusRerunLarge;
@@ -542,7 +671,7 @@ __global__ __launch_bounds__(64, (clip_min_waves<G, C>())) void k_clip(
     const uint32_t hcur = s_h[g][cur];
     uint32_t adj_lo = 0, adj_hi = 0;  // the planes now joined to cur
     for (int q = j; q < nbd; q += L) {
-      const uint32_t c2 = s_cyc[g][q];
+      const uint32_t c2 = cycle(q);
       const uint32_t hz = max(hcur, (uint32_t)s_h[g][c2]);
       const uint32_t lo = min((uint32_t)cur, c2), hi = max((uint32_t)cur, c2);
       wedge[nb_e + q] = lo | (hi << 8) | (hz << 16);
@@ -562,8 +691,8 @@ __global__ __launch_bounds__(64, (clip_min_waves<G, C>())) void k_clip(
       const int q = q0 + j;
       int kind = 0;
       if (q < nbd) {
-        const uint32_t c1 = s_cyc[g][q];
-        const uint32_t c2 = s_cyc[g][(q + 1) % nbd];
+        const uint32_t c1 = cycle(q);
+        const uint32_t c2 = cycle(q + 1 < nbd ? q + 1 : 0);
         if (nb_v + q + 1 >= V) {
           kind = 1;
         } else {
@@ -705,6 +834,34 @@ __global__ __launch_bounds__(64, (clip_min_waves<G, C>())) void k_clip(
       }
       // per-plane sums over the group's lanes (fixed butterfly order);
       // lane p % L keeps plane p
+      if constexpr (L == 4) {
+        // a quad's lanes read each other's three contributions (DPP
+        // broadcasts) and pick those of their own planes: every lane works
+        // for its planes, instead of all four summing each plane in turn
+        // (12 planes: 148 instead of 264 instructions)
+        const uint32_t pk = ia | (ib << 8) | (ic << 16);
+        const uint32_t pk_s[4] = {quad_perm<0x00>(pk), quad_perm<0x55>(pk),
+                                  quad_perm<0xAA>(pk), quad_perm<0xFF>(pk)};
+        const double ca_s[4] = {quad_perm<0x00>(ca), quad_perm<0x55>(ca),
+                                quad_perm<0xAA>(ca), quad_perm<0xFF>(ca)};
+        const double cb_s[4] = {quad_perm<0x00>(cb), quad_perm<0x55>(cb),
+                                quad_perm<0xAA>(cb), quad_perm<0xFF>(cb)};
+        const double cc_s[4] = {quad_perm<0x00>(cc), quad_perm<0x55>(cc),
+                                quad_perm<0xAA>(cc), quad_perm<0xFF>(cc)};
+#pragma unroll
+        for (int pi = 0; pi < PA; ++pi) {
+          if (pi > 0 && ballot(nb_p > pi * L) == 0) break;
+          const uint32_t p = (uint32_t)(pi * L + j);
+          double c[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            c[u] = (pk_s[u] >> 16) == p ? cc_s[u] : 0.0;
+            c[u] = ((pk_s[u] >> 8) & 255) == p ? cb_s[u] : c[u];
+            c[u] = (pk_s[u] & 255) == p ? ca_s[u] : c[u];
+          }
+          acc[pi] += (c[0] + c[2]) + (c[1] + c[3]);
+        }
+      } else
 #pragma unroll
       for (int pi = 0; pi < PA; ++pi) {
 #pragma unroll
