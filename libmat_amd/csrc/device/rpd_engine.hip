@@ -24,6 +24,7 @@
 #include "rpd_prep.h"
 #include "../common/rpd_classgrid.h"
 #include "../common/rpd_nbrlist.h"
+#include "../common/rpd_rng.h"
 #include "rpd_stages.hip"
 #include "rpd_learn.hip"
 #include "rpd_nbr.hip"
@@ -3450,10 +3451,9 @@ int rpd_mlp_init(rpd_ctx* ctx, uint64_t seed) {
   std::vector<float> p(kNParam, 0.f);
   auto fill = [&](int off, int in, int out, uint64_t stream) {
     const double lim = std::sqrt(6.0 / (in + out));
+    const RpdRngStream rng(seed, stream);
     for (int q = 0; q < in * out; ++q)
-      p[off + q] =
-          (float)((2.0 * rpd_rng_uniform(seed, stream, (uint64_t)q) - 1.0) *
-                  lim);
+      p[off + q] = (float)((2.0 * rng.uniform((uint64_t)q) - 1.0) * lim);
   };
   fill(kOffW1, kIn, kHid, 11);
   fill(kOffW2, kHid, kHid, 12);
@@ -3516,18 +3516,26 @@ int rpd_mlp_train(rpd_ctx* ctx, const rpd_train_cfg* tc, float* loss) {
   HIP_TRY(hipSetDevice(ctx->device));
   const int64_t n = ctx->n_tet, B = tc->batch;
   const int64_t n_pad = (n + B - 1) / B * B;
-  std::vector<int32_t> order(n_pad, -1);
-  HIP_TRY(ctx->tr_idx.need((size_t)n_pad * 4));
-  for (int e = 0; e < tc->epochs; ++e) {
+  // two orders in turn: the next epoch's is made while the device works on
+  // (and may still copy) this one's
+  std::vector<int32_t> orders[2];
+  for (int q = 0; q < std::min(2, tc->epochs); ++q) orders[q].assign(n_pad, -1);
+  auto shuffle = [&](int e) {
+    std::vector<int32_t>& order = orders[e & 1];
+    const RpdRngStream rng(tc->seed, 1000 + e);
     for (int64_t i = 0; i < n; ++i) order[i] = (int32_t)i;
     for (int64_t i = n - 1; i > 0; --i) {  // Fisher-Yates
-      const int64_t j = (int64_t)(rpd_rng_uniform(tc->seed, 1000 + e,
-                                                  (uint64_t)i) *
-                                  (double)(i + 1));
+      const int64_t j =
+          (int64_t)(rng.uniform((uint64_t)i) * (double)(i + 1));
       std::swap(order[i], order[std::min(j, i)]);
     }
-    HIP_TRY(hipMemcpyAsync(ctx->tr_idx.p, order.data(), (size_t)n_pad * 4,
-                           hipMemcpyHostToDevice, ctx->stream));
+  };
+  HIP_TRY(ctx->tr_idx.need((size_t)n_pad * 4));
+  shuffle(0);
+  for (int e = 0; e < tc->epochs; ++e) {
+    HIP_TRY(hipMemcpyAsync(ctx->tr_idx.p, orders[e & 1].data(),
+                           (size_t)n_pad * 4, hipMemcpyHostToDevice,
+                           ctx->stream));
     HIP_TRY(ctx->tr_loss.need((size_t)(n_pad / 16) * 4));
     int nb = 0;
     for (int64_t b0 = 0; b0 < n_pad; b0 += B) {
@@ -3549,6 +3557,7 @@ int rpd_mlp_train(rpd_ctx* ctx, const rpd_train_cfg* tc, float* loss) {
         return rc;
       ++nb;
     }
+    if (e + 1 < tc->epochs) shuffle(e + 1);
     // mean over the epoch's steps of each step's loss
     double el = 0;
     if (int rc = sum_device(ctx, ctx->tr_loss.as<float>(), n_pad / 16, &el))

@@ -13,23 +13,13 @@
 #include "../common/rpd_classgrid.h"
 #include "../common/rpd_nbrlist.h"
 #include "../common/rpd_predicates.h"
+#include "../common/rpd_rng.h"
 
 namespace {
 
 // ------------------------------------------------------------------ RNG
-inline uint64_t mix64(uint64_t z) {
-  z += 0x9E3779B97F4A7C15ULL;
-  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBULL;
-  return z ^ (z >> 31);
-}
-inline uint64_t rng_u64(uint64_t seed, uint64_t stream, uint64_t index) {
-  uint64_t h = mix64(seed);
-  h = mix64(h ^ (stream * 0xD1B54A32D192ED03ULL));
-  return mix64(h ^ index);
-}
 inline double rng_uniform(uint64_t seed, uint64_t stream, uint64_t index) {
-  return (double)(rng_u64(seed, stream, index) >> 11) * 0x1.0p-53;
+  return RpdRngStream(seed, stream).uniform(index);
 }
 // standard normal by Box-Muller from draws (2*index, 2*index+1)
 inline double rng_normal(uint64_t seed, uint64_t stream, uint64_t index) {
