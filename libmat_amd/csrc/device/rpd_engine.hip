@@ -3019,13 +3019,15 @@ int rpd_power_neighbors_gpu(rpd_ctx* ctx, int32_t n, const double* xyzw,
     d.cell_base = (int64_t)starts.size();
     const int64_t id_base = (int64_t)ids.size();
     for (size_t q = 0; q < g.start.size(); ++q) {
-      // the cell's largest weight, rounded up to binary32
+      // the cell's largest weight, rounded up to binary32; -1: no member
       double w = 0;
-      if (q + 1 < g.start.size())
+      const bool some =
+          q + 1 < g.start.size() && g.start[q] < g.start[q + 1];
+      if (some)
         for (int64_t v = g.start[q]; v < g.start[q + 1]; ++v)
           w = std::max(w, xyzw[4 * (int64_t)g.ids[v] + 3]);
       starts.push_back(id_base + g.start[q]);
-      cell_w.push_back(std::nextafter((float)w, INFINITY));
+      cell_w.push_back(some ? std::nextafter((float)w, INFINITY) : -1.f);
     }
     ids.insert(ids.end(), g.ids.begin(), g.ids.end());
   }

@@ -93,6 +93,32 @@ __device__ __forceinline__ void nb_dot(const rpd_d4& e, double me,
   eps = b < RPD_FILTER_MAX ? RPD_FILTER_C * b + RPD_FILTER_ABS : INFINITY;
 }
 
+// Reductions over a wavefront: within rows of 16 lanes by DPP rotations, the
+// four rows by reads of their first lanes (no LDS-routed shuffle).
+template <int C>
+__device__ __forceinline__ float row_ror(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_mov_dpp(__float_as_int(v), 0x120 + C, 0xF, 0xF, false));
+}
+template <class Op>
+__device__ __forceinline__ float wave_reduce(float v, Op op) {
+  v = op(v, row_ror<8>(v));
+  v = op(v, row_ror<4>(v));
+  v = op(v, row_ror<2>(v));
+  v = op(v, row_ror<1>(v));
+  return op(op(lane_value(v, 0), lane_value(v, 16)),
+            op(lane_value(v, 32), lane_value(v, 48)));
+}
+__device__ __forceinline__ float wave_max(float v) {
+  return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ __forceinline__ float wave_min(float v) {
+  return wave_reduce(v, [](float a, float b) { return fminf(a, b); });
+}
+__device__ __forceinline__ float wave_add(float v) {
+  return wave_reduce(v, [](float a, float b) { return a + b; });
+}
+
 // One wavefront per sphere.  The cell's vertices live in registers, vertex
 // slot 64 q + lane in slot q of a lane: homogeneous coordinates X with
 // X.w > 0 (the plane triple is ordered for it), the sum of its cofactor
@@ -116,9 +142,13 @@ __device__ __forceinline__ void nb_dot(const rpd_d4& e, double me,
 // device.  50,000 spheres of the boundary rule: one kernel of 256-vertex
 // cells in LDS (42 KB a wavefront, every candidate clipped, the cut edges
 // found by one lane per removed vertex scanning all vertices) took
-// 203 ms, this one 14 ms with the larger cells (5,003 uniform spheres: 2.3
-// and 0.7 ms).  The small tier at 2, 3 and 4 wavefronts per SIMD (the
-// register limit): 14.7, 11.8 and 15.0 ms (4 spills).
+// 203 ms, this one 8.8 ms with the larger cells (5,003 uniform spheres: 2.3
+// and 0.54 ms).  The grid search is half of it there: 96 chunks of 64 grid
+// cells a sphere, 161 before rows and faces outside the reach of every
+// vertex were left out (11.9 -> 7.8 ms without the larger cells, together
+// with reductions by DPP, binary32 corners and 32-bit cell numbers).  The
+// small tier at 2, 3 and 4 wavefronts per SIMD (the register limit), before
+// that: 14.7, 11.8 and 15.0 ms (4 spills).
 //
 // valid[i]: 1 valid, 0 hidden, -1 capacity or topology failure; counts[i] /
 // lists[i * kNbOut ..]: neighbour ids, ascending.
@@ -211,16 +241,11 @@ __device__ __forceinline__ void power_cell(
         sy += uy[q];
         sz += uz[q];
       }
-    for (int off = 32; off > 0; off >>= 1) {
-      r2 = fmaxf(r2, __shfl_xor(r2, off));
-      sx += __shfl_xor(sx, off);
-      sy += __shfl_xor(sy, off);
-      sz += __shfl_xor(sz, off);
-    }
+    r2 = wave_max(r2);
     const float inv = 1.0f / (float)nv;
-    mx = sx * inv;
-    my = sy * inv;
-    mz = sz * inv;
+    mx = wave_add(sx) * inv;
+    my = wave_add(sy) * inv;
+    mz = wave_add(sz) * inv;
     float d2 = 0;
 #pragma unroll
     for (int q = 0; q < kVS; ++q)
@@ -228,7 +253,7 @@ __device__ __forceinline__ void power_cell(
         const float dx = ux[q] - mx, dy = uy[q] - my, dz = uz[q] - mz;
         d2 = fmaxf(d2, dx * dx + dy * dy + dz * dz);
       }
-    for (int off = 32; off > 0; off >>= 1) d2 = fmaxf(d2, __shfl_xor(d2, off));
+    d2 = wave_max(d2);
     R2 = r2 * 1.00001f;
     rm = sqrtf(d2) * 1.00001f + 1e-5f * sqrtf(r2);
   };
@@ -404,6 +429,8 @@ __device__ __forceinline__ void power_cell(
     const NbGrid& g = G.g[c];
     if (!g.used) continue;
     int64_t q0[3], rmin = 0, rmax = 0;
+    int g_lo[3], g_hi[3];  // the grid's cells, relative to q0
+    float off[3];          // corner of cell q0 less the centre
     for (int a = 0; a < 3; ++a) {
       q0[a] = (int64_t)floor(((&si.x)[a] - g.org[a]) / g.cs);
       const int64_t lo = q0[a], hi = q0[a] - (g.dim[a] - 1);
@@ -412,11 +439,24 @@ __device__ __forceinline__ void power_cell(
       if (d2 > rmax) rmax = d2;
       if (-lo > rmin) rmin = -lo;  // rings before the grid: none
       if (hi > rmin) rmin = hi;
+      g_lo[a] = (int)max(-lo, (int64_t)-0x7fffffff);
+      g_hi[a] = (int)max(min(-hi, (int64_t)0x7fffffff), (int64_t)-0x7fffffff);
+      off[a] = (float)(g.org[a] + (double)q0[a] * g.cs - (&si.x)[a]);
     }
+    const int64_t cell0 =
+        g.cell_base + q0[0] +
+        (int64_t)g.dim[0] * (q0[1] + (int64_t)g.dim[1] * q0[2]);
     const float csf = (float)g.cs, wi = (float)si.w;
-    // (d2: squared distance of a vertex to a cell's box, vv: to the centre)
-    auto reaches = [&](float d2, float vv, float wl) {
-      return !(d2 > vv - wi + wl + 1e-5f * (vv + fabsf(wi) + wl + d2));
+    const float wm = (float)g.wmax * 1.00001f, ics = 1.0f / csf;
+    // A sphere of weight up to wl in a cell's box cuts a vertex off only if
+    // d2 <= vv - w_i + wl (d2: squared distance of the vertex to the box,
+    // vv: to the centre), here with 1e-5 of every term for the rounding:
+    // not (d2' > vertex_side + wl'), primes for the factors 1 -+ 1e-5
+    auto vertex_side = [&](float x, float y, float z) {
+      return 1.00001f * (x * x + y * y + z * z) - wi + 1e-5f * fabsf(wi);
+    };
+    auto box_side = [&](float x, float y, float z, float wl) {
+      return 0.99999f * (x * x + y * y + z * z) - wl;
     };
     int qn = 0;  // spheres waiting in s_q
     bool done = false;
@@ -427,27 +467,75 @@ __device__ __forceinline__ void power_cell(
         done = r > rmax ||
                (r >= 1 && (double)(r - 1) * g.cs > bound * (1 + 1e-9) + 1e-12);
       }
+      const int ri = (int)r;
+      int d_lo[3] = {g_lo[0], g_lo[1], g_lo[2]};  // cells worth a look
+      int d_hi[3] = {g_hi[0], g_hi[1], g_hi[2]};
+      // From the third shell on (more than two chunks) also those that meet
+      // the bounding box of the balls in which a sphere of the class would
+      // have to lie to cut a vertex off: the cell of a sphere near a
+      // boundary reaches far on one side only, and R counts for all.
+      if (!done && r >= 3) {
+        float lx = INFINITY, ly = INFINITY, lz = INFINITY;
+        float hx = -INFINITY, hy = -INFINITY, hz = -INFINITY;
+#pragma unroll
+        for (int q = 0; q < kVS; ++q)
+          if ((alive[q] >> lane) & 1) {
+            const float vv = ux[q] * ux[q] + uy[q] * uy[q] + uz[q] * uz[q];
+            const float t = vv - wi + wm + 1e-5f * (vv + fabsf(wi) + wm);
+            if (!(t < 0)) {
+              const float rad =
+                  t < 1e30f ? __builtin_amdgcn_sqrtf(t) * 1.0001f : INFINITY;
+              lx = fminf(lx, ux[q] - rad);
+              ly = fminf(ly, uy[q] - rad);
+              lz = fminf(lz, uz[q] - rad);
+              hx = fmaxf(hx, ux[q] + rad);
+              hy = fmaxf(hy, uy[q] + rad);
+              hz = fmaxf(hz, uz[q] + rad);
+            }
+          }
+        const float l[3] = {wave_min(lx), wave_min(ly), wave_min(lz)};
+        const float h[3] = {wave_max(hx), wave_max(hy), wave_max(hz)};
+        bool inside = true;  // nothing of this shell or a later one
+        for (int a = 0; a < 3; ++a) {
+          // (cell d covers off + d cs .. off + (d + 1) cs)
+          const float fl = (l[a] - off[a]) * ics, fh = (h[a] - off[a]) * ics;
+          const int cl = (int)fminf(
+              fmaxf(floorf(fl - 1e-5f * fabsf(fl) - 0.01f), -1e9f), 1e9f);
+          const int ch = (int)fmaxf(
+              fminf(floorf(fh + 1e-5f * fabsf(fh) + 0.01f), 1e9f), -1e9f);
+          d_lo[a] = max(d_lo[a], cl);
+          d_hi[a] = min(d_hi[a], ch);
+          inside = inside && d_lo[a] > -ri && d_hi[a] < ri;
+        }
+        done = inside || d_lo[0] > d_hi[0] || d_lo[1] > d_hi[1] ||
+               d_lo[2] > d_hi[2];
+      }
       // the shell's cells in [k_lo[u], k_hi[u]): the rows of its two z
-      // faces that lie in the grid, and the slabs that do
+      // faces and the slabs between them that hold cells worth a look
       int k_lo[3] = {0, 0, 0}, k_hi[3] = {0, 0, 0};
       if (!done) {
-        const int ri = (int)r, side = 2 * ri + 1, face = side * side;
-        const int y0 = (int)(q0[1] - r < 0 ? r - q0[1] : 0);
-        const int y1 = (int)min((int64_t)(side - 1), g.dim[1] - 1 - q0[1] + r);
-        for (int u = 0; u < 2; ++u) {
-          const int64_t z = u == 0 ? q0[2] - r : q0[2] + r;
-          if (z >= 0 && z < g.dim[2] && y0 <= y1 && (u == 0 || r > 0)) {
-            k_lo[u] = u * face + y0 * side;
-            k_hi[u] = u * face + (y1 + 1) * side;
-          }
+        const int side = 2 * ri + 1, face = side * side;
+        const int y0 = max(d_lo[1], -ri) + ri, y1 = min(d_hi[1], ri) + ri;
+        if (y0 <= y1 && d_lo[2] <= -ri && d_hi[2] >= -ri) {
+          k_lo[0] = y0 * side;
+          k_hi[0] = (y1 + 1) * side;
         }
-        const int64_t s0 = max((int64_t)0, r - 1 - q0[2]);
-        const int64_t s1 = min(2 * r - 2, g.dim[2] - 1 - q0[2] + r - 1);
-        if (s0 <= s1) {
-          k_lo[2] = 2 * face + (int)s0 * 8 * ri;
-          k_hi[2] = 2 * face + (int)(s1 + 1) * 8 * ri;
+        if (y0 <= y1 && ri > 0 && d_lo[2] <= ri && d_hi[2] >= ri) {
+          k_lo[1] = face + y0 * side;
+          k_hi[1] = face + (y1 + 1) * side;
+        }
+        const int s0 = max(d_lo[2], 1 - ri) + ri - 1;
+        const int s1 = min(d_hi[2], ri - 1) + ri - 1;
+        if (s0 <= s1 && (d_lo[0] <= -ri || d_hi[0] >= ri || d_lo[1] <= -ri ||
+                         d_hi[1] >= ri)) {
+          k_lo[2] = 2 * face + s0 * 8 * ri;
+          k_hi[2] = 2 * face + (s1 + 1) * 8 * ri;
         }
       }
+      // margin of a cell's box: 1e-5 of a cell, and the rounding of its
+      // corner in binary32 (off + d cs)
+      const float mg = (1e-5f + 2e-7f * (float)(ri + 1)) * csf;
+      const float wd = csf + 2 * mg;
       // the next chunk of 64 cells (from a multiple of 64) at or after k
       // that meets one of the ranges; INT_MAX: none
       auto chunk_from = [&](int k) {
@@ -466,7 +554,7 @@ __device__ __forceinline__ void power_cell(
         // by vertex (binary32 about the centre c, 1e-5 of every term for
         // its rounding): lanes take the cells and the vertices are
         // broadcast, or the other way round, whichever loop is shorter
-        int64_t a0 = 0, a1 = 0;
+        int64_t a0 = 0, a1 = 0, cell = 0;
         const int k = k0 + lane;
         float lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0}, wc = 0;
         bool near = false;
@@ -474,51 +562,46 @@ __device__ __forceinline__ void power_cell(
             ((k >= k_lo[0] && k < k_hi[0]) || (k >= k_lo[1] && k < k_hi[1]) ||
              (k >= k_lo[2] && k < k_hi[2]))) {
           int dx, dy, dz;
-          shell_cell((int)r, k, dx, dy, dz);
-          const int64_t x = q0[0] + dx, y = q0[1] + dy, z = q0[2] + dz;
-          if (x >= 0 && y >= 0 && z >= 0 && x < g.dim[0] && y < g.dim[1] &&
-              z < g.dim[2]) {
-            const int64_t cell =
-                g.cell_base + x + (int64_t)g.dim[0] * (y + (int64_t)g.dim[1] * z);
-            a0 = start[cell];
-            a1 = start[cell + 1];
-            wc = cell_w[cell];
-            const double bx[3] = {g.org[0] + (double)x * g.cs - si.x,
-                                  g.org[1] + (double)y * g.cs - si.y,
-                                  g.org[2] + (double)z * g.cs - si.z};
-            for (int a = 0; a < 3; ++a) {
-              lo[a] = (float)bx[a] - 1e-5f * csf;
-              hi[a] = (float)bx[a] + 1.00001f * csf;
-            }
+          shell_cell(ri, k, dx, dy, dz);
+          if (dx >= d_lo[0] && dx <= d_hi[0] && dy >= d_lo[1] &&
+              dy <= d_hi[1] && dz >= d_lo[2] && dz <= d_hi[2]) {
+            cell = cell0 + dx + (int64_t)g.dim[0] * (dy + g.dim[1] * dz);
+            wc = cell_w[cell];  // below 0: no member
+            lo[0] = fmaf((float)dx, csf, off[0]) - mg;
+            lo[1] = fmaf((float)dy, csf, off[1]) - mg;
+            lo[2] = fmaf((float)dz, csf, off[2]) - mg;
+            for (int a = 0; a < 3; ++a) hi[a] = lo[a] + wd;
             const float ex = fmaxf(0.f, fmaxf(lo[0] - mx, mx - hi[0]));
             const float ey = fmaxf(0.f, fmaxf(lo[1] - my, my - hi[1]));
             const float ez = fmaxf(0.f, fmaxf(lo[2] - mz, mz - hi[2]));
-            const float far = sqrtf(ex * ex + ey * ey + ez * ez) * 0.99999f;
+            const float far =
+                __builtin_amdgcn_sqrtf(ex * ex + ey * ey + ez * ez) * 0.99999f;
             const float sl = R2 - wi + wc + 1e-5f * (R2 + fabsf(wi) + wc);
-            near = a0 < a1 && !(far > rm && (far - rm) * (far - rm) > sl);
+            near = wc >= 0 && !(far > rm && (far - rm) * (far - rm) > sl);
           }
         }
         uint64_t nearm = ballot(near);
         if (nearm != 0) {
+          const float wl = 1.00001f * wc;
           if (__popcll(nearm) < nv) {
             uint64_t todo = nearm;
             while (todo) {
               const int l = __ffsll((long long)todo) - 1;
               todo &= todo - 1;
               const float x0 = lane_value(lo[0], l), y0 = lane_value(lo[1], l),
-                          z0 = lane_value(lo[2], l), x1 = lane_value(hi[0], l),
-                          y1 = lane_value(hi[1], l), z1 = lane_value(hi[2], l),
-                          wl = lane_value(wc, l);
+                          z0 = lane_value(lo[2], l), wv = lane_value(wl, l);
               bool cuts = false;
 #pragma unroll
               for (int q = 0; q < kVS; ++q) {
-                const float uu =
-                    ux[q] * ux[q] + uy[q] * uy[q] + uz[q] * uz[q];
-                const float ex = fmaxf(0.f, fmaxf(x0 - ux[q], ux[q] - x1));
-                const float ey = fmaxf(0.f, fmaxf(y0 - uy[q], uy[q] - y1));
-                const float ez = fmaxf(0.f, fmaxf(z0 - uz[q], uz[q] - z1));
+                const float ex =
+                    ux[q] - __builtin_amdgcn_fmed3f(ux[q], x0, x0 + wd);
+                const float ey =
+                    uy[q] - __builtin_amdgcn_fmed3f(uy[q], y0, y0 + wd);
+                const float ez =
+                    uz[q] - __builtin_amdgcn_fmed3f(uz[q], z0, z0 + wd);
                 cuts = cuts || (((alive[q] >> lane) & 1) &&
-                                reaches(ex * ex + ey * ey + ez * ez, uu, wl));
+                                !(box_side(ex, ey, ez, wv) >
+                                  vertex_side(ux[q], uy[q], uz[q])));
               }
               if (ballot(cuts) == 0) nearm &= ~(1ull << l);
             }
@@ -527,18 +610,19 @@ __device__ __forceinline__ void power_cell(
             uint64_t cm = 0;
 #pragma unroll
             for (int q = 0; q < kVS; ++q) {
-              const float uu = ux[q] * ux[q] + uy[q] * uy[q] + uz[q] * uz[q];
+              const float vs = vertex_side(ux[q], uy[q], uz[q]);
               uint64_t v = alive[q];
               while (v && cm != nearm) {
                 const int l = __ffsll((long long)v) - 1;
                 v &= v - 1;
                 const float vx = lane_value(ux[q], l),
                             vy = lane_value(uy[q], l),
-                            vz = lane_value(uz[q], l), vv = lane_value(uu, l);
-                const float ex = fmaxf(0.f, fmaxf(lo[0] - vx, vx - hi[0]));
-                const float ey = fmaxf(0.f, fmaxf(lo[1] - vy, vy - hi[1]));
-                const float ez = fmaxf(0.f, fmaxf(lo[2] - vz, vz - hi[2]));
-                cuts = cuts || reaches(ex * ex + ey * ey + ez * ez, vv, wc);
+                            vz = lane_value(uz[q], l);
+                const float ex = vx - __builtin_amdgcn_fmed3f(vx, lo[0], hi[0]);
+                const float ey = vy - __builtin_amdgcn_fmed3f(vy, lo[1], hi[1]);
+                const float ez = vz - __builtin_amdgcn_fmed3f(vz, lo[2], hi[2]);
+                cuts = cuts ||
+                       !(box_side(ex, ey, ez, wl) > lane_value(vs, l));
                 cm = ballot(near && cuts);
               }
             }
@@ -546,7 +630,10 @@ __device__ __forceinline__ void power_cell(
           }
           near = (nearm >> lane) & 1;
         }
-        if (!near) a1 = a0;
+        if (near) {
+          a0 = start[cell];
+          a1 = start[cell + 1];
+        }
         const int kn = k0 == 0x7fffffff ? k0 : chunk_from(k0 + 64);
         // waiting spheres are clipped when 64 are there, at the end of the
         // first shells (whose spheres shrink the cell) and of the class

@@ -74,3 +74,29 @@ def test_lattice_ties(ctx, k):
         assert (np.diff(mine) > 0).all() and near[i][mine].all()
         assert set(np.nonzero(face[i])[0]) <= set(mine)
         assert all(i in ids[off[j]:off[j + 1]] for j in mine)
+
+
+@pytest.mark.parametrize("shift", [0.0, 1000.0])
+@pytest.mark.parametrize("kind", ["slab", "line", "corners"])
+def test_cells_that_reach_far_on_one_side(ctx, kind, shift):
+    # shells of many grid cells of which a one-sided or flat cell needs a
+    # few rows: spheres near a face of the box, along a diagonal, and in two
+    # small clusters of different weight classes (each outside the other's
+    # grid); general position, so the lists are the host builder's
+    rng = np.random.default_rng(11)
+    p = rng.random((400, 3))
+    w = np.full(400, 1e-4) * (1 + rng.random(400))
+    if kind == "slab":
+        p[:, 2] = 0.02 + 0.001 * p[:, 2]
+    elif kind == "line":
+        p = 0.1 + 0.8 * p[:, :1] + 0.002 * p
+    else:
+        p = np.where(np.arange(400)[:, None] < 200, 0.05 + 0.02 * p,
+                     0.9 + 0.03 * p)
+        w[:200] *= 1e-2
+    box = np.asarray(prep.UNIT_BOX) + shift
+    xyzw = np.c_[p + shift, w]
+    want = prep.power_neighbors(xyzw, box)
+    got = ctx.power_neighbors(xyzw, box)
+    for a, b in zip(want, got):
+        assert np.array_equal(a, b)
