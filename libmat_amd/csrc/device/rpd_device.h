@@ -39,9 +39,9 @@ struct DevSites {
   const uint32_t* flags;
   const int64_t* knn_off;
   const int32_t* knn_ids;   // neighbours in ascending site id (clip order)
-  const int32_t* knn_near;  // the same lists (nearest bisector first for
-                            // the relation, list order for the learned
-                            // path), bit 31 set for unflagged sites
+  const int32_t* knn_near;  // learned path: the same lists, nearest
+                            // bisector first (k_site_inline), bit 31 set
+                            // for unflagged sites
   const double4* knn_site_near;  // the spheres of knn_near, inline
   const double4* knn_bis;  // power bisector of each knn_ids entry (zero
                            // for a -1 entry), in knn_ids order

@@ -85,11 +85,10 @@ __device__ __forceinline__ f32x4 mfma(bf16x4 a, bf16x4 b, f32x4 c) {
 }
 
 // ------------------------------------------------------------- features
-// neighbour lists in list order with their spheres inline (flag in the
-// id word, near_word)
 // One wavefront per site: its neighbour list nearest bisector first (the
 // signed distance of the site's centre to each bisector, then the list
-// position), written with the neighbour spheres inline.  The relation test
+// position), written with the neighbour spheres inline (flag in the id
+// word, near_word).  The relation test
 // meets a rejecting neighbour early in that order (its outcome does not
 // depend on the order); lists longer than kNearMax keep their order.
 __global__ __launch_bounds__(64) void k_site_inline(DevSites S,

@@ -470,8 +470,8 @@ __device__ __forceinline__ void power_cell(
       const int ri = (int)r;
       int d_lo[3] = {g_lo[0], g_lo[1], g_lo[2]};  // cells worth a look
       int d_hi[3] = {g_hi[0], g_hi[1], g_hi[2]};
-      // From the third shell on (more than two chunks) also those that meet
-      // the bounding box of the balls in which a sphere of the class would
+      // From the third shell on (four chunks and more; the box costs about
+      // one) also those that meet the bounding box of the balls in which a sphere of the class would
       // have to lie to cut a vertex off: the cell of a sphere near a
       // boundary reaches far on one side only, and R counts for all.
       if (!done && r >= 3) {
