@@ -1105,10 +1105,14 @@ int plain_candidates(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out) {
 int site_inline(rpd_ctx* ctx, RunState& R) {
   // (one wavefront per site: the lists' lengths are read on the device, so
   // a captured run follows sphere updates that change them)
+  const size_t nk = (size_t)std::max<int64_t>(ctx->n_knn, 1);
+  HIP_TRY(ctx->rel_pl.need(nk * 16));
+  HIP_TRY(ctx->rel_aux.need(nk * 8));
   if (R.ns > 0)
     hipLaunchKernelGGL(k_site_inline, dim3(R.ns), dim3(64), 0, R.s, R.S,
-                       ctx->knn_near.as<int32_t>(),
-                       ctx->knn_site_near.as<double4>());
+                       R.inst_d, R.site_inst_d, ctx->knn_near.as<int32_t>(),
+                       ctx->knn_site_near.as<double4>(),
+                       ctx->rel_pl.as<float4>(), ctx->rel_aux.as<float2>());
   HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -1201,7 +1205,9 @@ int learned_candidates(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out) {
   HIP_TRY(ctx->tet_off.need(((size_t)nt + 1) * 8));
   HIP_TRY(zero32(s, ctx->tet_count.as<int64_t>() + nt, 2));
   hipLaunchKernelGGL(k_learn_count, dim3(ceil_div(nt, 64)), dim3(64), 0, s, nt,
-                     R.M, R.S, ctx->knn.as<int32_t>(), ctx->sel.as<uint32_t>(),
+                     R.M, R.S, R.inst_d, R.tet_inst_d,
+                     ctx->rel_pl.as<float4>(), ctx->rel_aux.as<float2>(),
+                     ctx->knn.as<int32_t>(), ctx->sel.as<uint32_t>(),
                      ctx->omask.as<uint32_t>(), ctx->tet_count.as<int64_t>());
   HIP_TRY(hipGetLastError());
   if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[12], s));
@@ -2679,10 +2685,8 @@ int rpd_graph_build(rpd_ctx* ctx, const rpd_run_cfg* cfg, double headroom) {
     const size_t nk = (size_t)std::max<int64_t>(grow(ctx->n_knn, f, 1024), 1);
     HIP_TRY(ctx->knn_bis.need(nk * 32));
     HIP_TRY(ctx->knn_bisf.need(nk * 16));
-    if (!R.cfg.learned) {
-      HIP_TRY(ctx->rel_pl.need(nk * 16));
-      HIP_TRY(ctx->rel_aux.need(nk * 8));
-    }
+    HIP_TRY(ctx->rel_pl.need(nk * 16));
+    HIP_TRY(ctx->rel_aux.need(nk * 8));
     HIP_TRY(ctx->knn_ids.need_keep(nk * 4, (size_t)ctx->n_knn * 4,
                                    ctx->stream));
     HIP_TRY(ctx->knn_near.need_keep(nk * 4, (size_t)ctx->n_knn * 4,
@@ -2768,9 +2772,8 @@ int rpd_graph_run(rpd_ctx* ctx, int32_t* replayed) {
   // gives this call's results)
   const size_t nk = (size_t)std::max<int64_t>(ctx->n_knn, 1);
   if (graph_signature(ctx) != ctx->graph_sig || nk * 32 > ctx->knn_bis.cap ||
-      nk * 16 > ctx->knn_bisf.cap ||
-      (!ctx->graph_cfg.learned &&
-       (nk * 16 > ctx->rel_pl.cap || nk * 8 > ctx->rel_aux.cap))) {
+      nk * 16 > ctx->knn_bisf.cap || nk * 16 > ctx->rel_pl.cap ||
+      nk * 8 > ctx->rel_aux.cap) {
     const rpd_run_cfg c = ctx->graph_cfg;
     return rpd_graph_build(ctx, &c, ctx->graph_headroom);
   }

@@ -90,25 +90,40 @@ __device__ __forceinline__ f32x4 mfma(bf16x4 a, bf16x4 b, f32x4 c) {
 // position), written with the neighbour spheres inline (flag in the id
 // word, near_word).  The relation test
 // meets a rejecting neighbour early in that order (its outcome does not
-// depend on the order); lists longer than kNearMax keep their order.
-__global__ __launch_bounds__(64) void k_site_inline(DevSites S,
-                                                    int32_t* knn_near,
-                                                    double4* knn_site_near) {
+// depend on the order); lists longer than kNearMax keep their order.  In the
+// same order the bisectors in binary32 (rel_plane), and in the list's first
+// entry of rel_aux the largest of their error bounds.
+__global__ __launch_bounds__(64) void k_site_inline(
+    DevSites S, const InstInfo* inst, const int32_t* site_inst,
+    int32_t* knn_near, double4* knn_site_near, float4* rel_pl,
+    float2* rel_aux) {
   __shared__ double s_key[kNearMax];
   __shared__ int32_t s_near[kNearMax];
   const int i = blockIdx.x;
   const int lane = threadIdx.x;
   const int64_t k0 = S.knn_off[i];
   const int deg = (int)(S.knn_off[i + 1] - k0);
+  const rpd_d4 si = ld4(S.site + i);
+  const double* dom = inst[site_inst[i]].dom;
+  float eps = 0;
+  auto write = [&](int k, int m) {
+    const double4 sm = S.site[m];
+    knn_near[k0 + k] = near_word(S, m);
+    knn_site_near[k0 + k] = sm;
+    float2 aux;
+    rel_plane(rpd_bisector(si, rpd_d4{sm.x, sm.y, sm.z, sm.w}), si, sm, 0.0,
+              0.0, dom, rel_pl[k0 + k], aux);
+    eps = fmaxf(eps, aux.x);
+  };
+  auto finish = [&]() {
+    for (int off = 32; off > 0; off >>= 1) eps = fmaxf(eps, __shfl_xor(eps, off));
+    if (lane == 0 && deg > 0) rel_aux[k0] = make_float2(eps, 0.f);
+  };
   if (deg > kNearMax) {
-    for (int k = lane; k < deg; k += 64) {
-      const int m = S.knn_ids[k0 + k];
-      knn_near[k0 + k] = near_word(S, m);
-      knn_site_near[k0 + k] = S.site[m];
-    }
+    for (int k = lane; k < deg; k += 64) write(k, S.knn_ids[k0 + k]);
+    finish();
     return;
   }
-  const rpd_d4 si = ld4(S.site + i);
   for (int k = lane; k < deg; k += 64) {
     const rpd_d4 e = rpd_bisector(si, ld4(S.site + S.knn_ids[k0 + k]));
     double key = (e.x * si.x + e.y * si.y + e.z * si.z + e.w) /
@@ -126,11 +141,8 @@ __global__ __launch_bounds__(64) void k_site_inline(DevSites S,
     s_near[r] = S.knn_ids[k0 + k];
   }
   wsync();
-  for (int k = lane; k < deg; k += 64) {
-    const int m = s_near[k];
-    knn_near[k0 + k] = near_word(S, m);
-    knn_site_near[k0 + k] = S.site[m];
-  }
+  for (int k = lane; k < deg; k += 64) write(k, s_near[k]);
+  finish();
 }
 
 __device__ __forceinline__ double pdist(const double c[3], const double4& s) {
@@ -997,16 +1009,57 @@ __global__ __launch_bounds__(256) void k_sel_topk(int32_t n_tet, int32_t k,
 // selected proposals (owners always) that pass the reference relation
 // (voronoi.cu:154-193): their slot mask replaces sel, their count is
 // written; only such spheres are clipped, as on the plain path
-__global__ __launch_bounds__(64) void k_learn_count(int32_t n_tet, DevMesh M,
-                                                    DevSites S,
-                                                    const int32_t* knn,
-                                                    uint32_t* sel,
-                                                    const uint32_t* omask,
-                                                    int64_t* count) {
+//
+// The relation is tested with the binary32 bisectors of k_site_inline at the
+// corners about the centre of the domain box, two a look; a value within the
+// list's error bound leaves the binary64 test to decide.  Bound by the
+// lanes' diverging lists; with the binary64 power distances of every
+// neighbour 1.57 M tets took 417 us, this way 291 (six instances of 50,000
+// to 500,000 tets 336 and 228); binary64, two or four neighbours ahead, 378.
+__global__ __launch_bounds__(64) void k_learn_count(
+    int32_t n_tet, DevMesh M, DevSites S, const InstInfo* inst,
+    const int32_t* tet_inst, const float4* __restrict__ rel_pl,
+    const float2* __restrict__ rel_aux, const int32_t* knn, uint32_t* sel,
+    const uint32_t* omask, int64_t* count) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n_tet) return;
   TetLoad L;
   load_tet(M, t, L);
+  const double* dom = inst[tet_inst[t]].dom;
+  float cx[4], cy[4], cz[4];
+  for (int k = 0; k < 4; ++k) {
+    cx[k] = (float)(L.V[k].x - 0.5 * (dom[0] + dom[3]));
+    cy[k] = (float)(L.V[k].y - 0.5 * (dom[1] + dom[4]));
+    cz[k] = (float)(L.V[k].z - 0.5 * (dom[2] + dom[5]));
+  }
+  auto side = [&](const float4& p) {  // the largest value at a corner
+    float v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      v[k] = fmaf(p.z, cz[k], fmaf(p.y, cy[k], fmaf(p.x, cx[k], p.w)));
+    return v[0] == v[0] && v[1] == v[1] && v[2] == v[2] && v[3] == v[3]
+               ? fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]))
+               : NAN;
+  };
+  auto relates = [&](int i) {
+    if (S.flags[i] != 1u) return false;
+    const int64_t k0 = S.knn_off[i], k1 = S.knn_off[i + 1];
+    if (k0 == k1) return true;
+    const float eps = rel_aux[k0].x;
+    bool open = false;
+    float4 n0 = rel_pl[k0], n1 = rel_pl[min(k0 + 1, k1 - 1)];
+    for (int64_t q = k0; q < k1; q += 2) {
+      const float4 p0 = n0, p1 = n1;
+      if (q + 2 < k1) {
+        n0 = rel_pl[q + 2];
+        n1 = rel_pl[min(q + 3, k1 - 1)];
+      }
+      const float v0 = side(p0), v1 = side(p1);
+      if (v0 < -eps || v1 < -eps) return false;
+      open = open || !(v0 > eps) || !(v1 > eps);
+    }
+    return !open || relation(S, L, i);
+  };
   const uint32_t s = sel[t] | omask[t];
   uint32_t pass = 0;
   int n = 0;
@@ -1015,8 +1068,7 @@ __global__ __launch_bounds__(64) void k_learn_count(int32_t n_tet, DevMesh M,
     const int k = __ffs(rest) - 1;
     const int id = knn[(int64_t)t * kOut + k];
     if (id < 0) break;
-    uint32_t it = 0;
-    if (relation(S, L, id, &it)) {
+    if (relates(id)) {
       pass |= 1u << k;
       ++n;
     }
@@ -1169,8 +1221,7 @@ __global__ __launch_bounds__(256) void k_closure_split(
   ukeys[u] = k;
   TetLoad L;
   load_tet(M, (int)(k >> 32), L);
-  uint32_t it = 0;
-  pass[u] = relation(S, L, (int)(k & 0xffffffffu), &it) ? 1 : 0;
+  pass[u] = relation(S, L, (int)(k & 0xffffffffu)) ? 1 : 0;
 }
 
 // (a captured run: n_u on the device, at most cap new candidates)
@@ -1261,8 +1312,7 @@ __global__ __launch_bounds__(64) void k_brute(
     const int s = I.site_off + s0 + lane;
     bool r = false;
     if (s0 + lane < I.n_site) {
-      uint32_t it = 0;
-      r = relation(S, L, s, &it);
+      r = relation(S, L, s);
     }
     const uint64_t b = __ballot(r);
     const int64_t at = o + n + __popcll(b & ((1ull << lane) - 1));

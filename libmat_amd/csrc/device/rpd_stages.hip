@@ -380,9 +380,9 @@ __device__ __forceinline__ void load_tet(const DevMesh& M, int t,
 // relates to the tet iff for every neighbour m some corner v has
 // pd(v, m) > pd(v, i).  The neighbours are visited nearest bisector first
 // (the outcome does not depend on the order), their spheres read inline,
-// one ahead.  *iters counts the neighbour tests made.
+// one ahead.
 __device__ __forceinline__ bool relation(const DevSites& S, const TetLoad& L,
-                                         int i, uint32_t* iters) {
+                                         int i) {
   if (S.flags[i] != 1u) return false;
   const rpd_d4 si = ld4(S.site + i);
   double pdi[4];
@@ -394,7 +394,6 @@ __device__ __forceinline__ bool relation(const DevSites& S, const TetLoad& L,
   for (int64_t q = k0; q < k1; ++q) {
     const rpd_d4 sm{nxt.x, nxt.y, nxt.z, nxt.w};
     if (q + 1 < k1) nxt = S.knn_site_near[q + 1];
-    ++*iters;
     bool ok = false;
 #pragma unroll
     for (int k = 0; k < 4; ++k)

@@ -82,6 +82,44 @@ def test_frames(ctx, shift, scale):
                                    box=np.array([lo] * 3 + [hi] * 3)))
 
 
+def proposed(ctx, inst):
+    # proposals are tested with binary32 planes of their own: what they let
+    # through is in the plain relation, and the cells are the plain path's
+    ctx.upload(inst)
+    ctx.run()
+    off, ids = ctx.relation()
+    want = ctx.download()
+    pairs = set(zip(np.repeat(np.arange(inst.n_tet), np.diff(off)), ids))
+    ctx.run(learned=2, proposal_k=32)
+    off, ids = ctx.relation()
+    assert set(zip(np.repeat(np.arange(inst.n_tet), np.diff(off)),
+                   ids)) <= pairs
+    got = ctx.download()
+    for k in ("cells", "words", "geom", "areas"):
+        assert np.array_equal(getattr(got, k), getattr(want, k))
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 127, 128, 129, 140])
+def test_proposal_list_lengths(ctx, n):
+    verts, tets = prep.grid_mesh(4, 0.1, n)
+    proposed(ctx, prep.build_instance(verts, tets, star(n)))
+
+
+@pytest.mark.parametrize("shift,scale", [(0.0, 0.0), (1000.0, 1.0),
+                                         (-3.0e5, 1.0), (0.0, 1e-7),
+                                         (2.0, 1e6)])
+def test_proposal_frames_and_ties(ctx, shift, scale):
+    if scale == 0:  # ties: bisectors through the grid's vertices
+        verts, tets = prep.grid_mesh(4, 0.0, 0)
+        return proposed(ctx, prep.build_instance(verts, tets, lattice(4)))
+    verts, tets = prep.grid_mesh(6, 0.1, 2)
+    sph = prep.spheres(150, 0, 8)
+    sph = np.c_[sph[:, :3] * scale + shift, sph[:, 3] * scale]
+    lo, hi = -1e-6 * scale + shift, (1 + 1e-6) * scale + shift
+    proposed(ctx, prep.build_instance(verts * scale + shift, tets, sph,
+                                      box=np.array([lo] * 3 + [hi] * 3)))
+
+
 def test_subsets_and_meshes_in_turn(ctx):
     # the tet order of the grid follows the mesh and the subset in use
     rng = np.random.default_rng(3)
