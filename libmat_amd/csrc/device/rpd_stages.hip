@@ -129,26 +129,44 @@ __device__ __forceinline__ int rel_rows(const int r[6]) {
 // value at any point of the box (three fused products and the rounding of
 // plane and point: 5 u sum |e_a| h_a + 4 u |d|, h the box's half extents,
 // u = 2^-24; 4e-7 covers it) plus the rounding of the two binary64 power
-// distances that decide the relation, aux.y the distance term of a tet's
+// distances that decide the relation and what coefficients, points and
+// products below the normal range lose, aux.y the distance term of a tet's
 // corners from its centroid.  Beyond aux.x the sign is the relation's.
+// Where a value could leave binary32's range (d and the power distances grow
+// with the square of the coordinates, so from extents of about 1e18 on) the
+// plane is zero and its bound infinite: it narrows no row and decides no
+// tet.
+constexpr double kRelMax = 1e37;
 __device__ __forceinline__ void rel_plane(const rpd_d4& e, const rpd_d4& si,
                                           const double4& sm, double nrm,
                                           double rho, const double* dom,
                                           float4& pl, float2& aux) {
-  double d = e.w, h = 0, far2 = 0;
+  const double sum = fabs(e.x) + fabs(e.y) + fabs(e.z);
+  double d = e.w, h = 0, far2 = 0, half = 0;
   for (int a = 0; a < 3; ++a) {
     const double ea = a == 0 ? e.x : a == 1 ? e.y : e.z;
     const double c = 0.5 * (dom[a] + dom[3 + a]);
     const double m = fmax(fabs(dom[a]), fabs(dom[3 + a]));
+    const double ha = (dom[3 + a] - dom[a]) * 0.5;
     d += ea * c;
-    h += fabs(ea) * (dom[3 + a] - dom[a]) * 0.5;
+    h += fabs(ea) * ha;
+    half += ha;
     far2 += m * m;
   }
   const double s2 = si.x * si.x + si.y * si.y + si.z * si.z + fabs(si.w) +
                     sm.x * sm.x + sm.y * sm.y + sm.z * sm.z + fabs(sm.w);
+  const double eps =
+      4e-7 * (h + fabs(d)) + 1e-14 * (far2 + s2) + 1.2e-38 * (half + sum);
+  const double far = nrm * rho;
+  // (negated, so that a NaN is out of range too)
+  if (!(h + fabs(d) + half + sum + eps + far < kRelMax)) {
+    pl = make_float4(0.f, 0.f, 0.f, 0.f);
+    aux = make_float2(INFINITY, 0.f);
+    return;
+  }
   pl = make_float4((float)e.x, (float)e.y, (float)e.z, (float)d);
-  aux.x = (float)(4e-7 * (h + fabs(d)) + 1e-14 * (far2 + s2)) + 1e-36f;
-  aux.y = (float)(nrm * rho) * 1.000001f;
+  aux.x = (float)eps + 1e-36f;
+  aux.y = (float)far * 1.000001f;
 }
 
 __global__ __launch_bounds__(64) void k_site_bbox(DevSites S,
@@ -594,8 +612,11 @@ __global__ __launch_bounds__(64) void k_rel_pairs(
       // bins of [xlo, xhi], with 1e-3 of a bin for the rounding
       const float inv = (float)g.inv_bs, ox = (float)o[0];
       const float flo = (xlo - ox) * inv - 1e-3f, fhi = (xhi - ox) * inv + 1e-3f;
-      const int a = max(r[0], (int)fminf(fmaxf(floorf(flo), -1.f), (float)(g.dim[0] - 1)));
-      const int b = min(r[3], (int)fminf(fmaxf(floorf(fhi), -1.f), (float)(g.dim[0] - 1)));
+      // (a bound that is not a number narrows nothing)
+      const float last = (float)(g.dim[0] - 1);
+      const int a = flo > 0.f ? max(r[0], (int)fminf(floorf(flo), last)) : r[0];
+      const int b =
+          fhi < last ? min(r[3], (int)fmaxf(floorf(fhi), -1.f)) : r[3];
       if (a <= b) {
         const int64_t base =
             I.bin_base + (int64_t)g.dim[0] * (y + (int64_t)g.dim[1] * z);

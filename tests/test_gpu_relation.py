@@ -2,6 +2,7 @@
 around the plane table's and the box polytope's capacities, one site, no
 site near, ties, grids of one bin, and coordinates far from the origin or
 of another scale.  The relation sets are compared with the oracle's."""
+import dataclasses
 import os
 import sys
 
@@ -80,6 +81,31 @@ def test_frames(ctx, shift, scale):
     lo, hi = -1e-6 * scale + shift, (1 + 1e-6) * scale + shift
     check(ctx, prep.build_instance(verts, tets, sph,
                                    box=np.array([lo] * 3 + [hi] * 3)))
+
+
+def far_frame(scale):
+    """A small instance at a scale where the squares of its coordinates and
+    the bisectors' constant terms approach or leave binary32's range."""
+    verts, tets = prep.grid_mesh(6, 0.1, 2)
+    inst = prep.build_instance(verts, tets, prep.spheres(150, 0, 8))
+    return dataclasses.replace(
+        inst, verts=inst.verts * scale,
+        sites=inst.sites * np.array([scale] * 3 + [scale * scale]))
+
+
+@pytest.mark.parametrize("scale", [1e17, 1e19, 5e19, 1e20, 1e25])
+def test_frames_beyond_binary32(ctx, scale):
+    check(ctx, far_frame(scale))
+
+
+@pytest.mark.parametrize("scale", [1e17, 1e19, 5e19, 1e20, 1e25])
+def test_proposal_frames_beyond_binary32(ctx, scale):
+    # every proposal the plain relation holds passes the proposals' own test
+    ctx.upload(far_frame(1.0))
+    ctx.run(learned=2, proposal_k=32)
+    want = ctx.stats()["learned"]
+    proposed(ctx, far_frame(scale))
+    assert ctx.stats()["learned"] == want
 
 
 def proposed(ctx, inst):
