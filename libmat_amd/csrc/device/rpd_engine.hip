@@ -1073,6 +1073,7 @@ int plain_candidates(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out) {
     cap = n_cand;  // again, with a list that holds them
     HIP_TRY(zero32(s, ctx->tet_count.p, 2 * ((int64_t)nt + 1)));
     HIP_TRY(zero32(s, n_pairs, 1));
+    if (R.cfg.count_work) HIP_TRY(zero32(s, ctx->rel_work.p, 64 * 4 * 2));
   }
   R.seen.n_cand = n_cand;
   const size_t nc = (size_t)std::max<int64_t>(n_cand, 1);

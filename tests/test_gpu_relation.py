@@ -192,3 +192,45 @@ def test_graph_follows_a_new_mesh_of_the_same_sizes(ctx):
         assert np.array_equal(got.cells, want.cells)
         assert np.array_equal(got.words, want.words)
         assert np.array_equal(got.geom, want.geom)
+
+
+def unlisted(inst):
+    """The same instance without neighbour lists: every sphere relates to
+    every tet, far more pairs than a run expects of its sizes."""
+    return dataclasses.replace(
+        inst, knn_off=np.zeros(inst.n_site + 1, np.int64),
+        knn_ids=np.zeros(0, np.int32))
+
+
+def test_more_pairs_than_the_list_holds():
+    verts, tets = prep.grid_mesh(6, 0.1, 2)
+    inst = unlisted(prep.build_instance(verts, tets, prep.spheres(300, 0, 8)))
+    with Context(0) as ctx:  # (a list of its own, as a first run finds it)
+        ctx.upload(inst)
+        st = [ctx.run(count_work=True) for _ in range(2)]
+        off, ids = ctx.relation()
+    n = inst.n_tet * inst.n_site
+    for s in st:  # the first pass, which ran out of room, counts nothing
+        assert s["n_candidates"] == n and s["relation_work"][0] == n
+    assert st[0]["relation_work"] == st[1]["relation_work"]
+    assert np.array_equal(off, np.arange(inst.n_tet + 1) * inst.n_site)
+    assert np.array_equal(ids.reshape(inst.n_tet, -1),
+                          np.tile(np.arange(inst.n_site), (inst.n_tet, 1)))
+
+
+def test_more_pairs_than_a_captured_list_holds():
+    verts, tets = prep.grid_mesh(6, 0.1, 2)
+    few = prep.build_instance(verts, tets, prep.spheres(300, 0, 8))
+    with Context(0) as ctx:
+        for inst in (few, unlisted(few), few):
+            ctx.upload(few)
+            ctx.graph_build()
+            ctx.update_sites(inst.sites, inst.flags, inst.knn_off,
+                             inst.knn_ids)
+            st, replayed = ctx.graph_run()
+            assert replayed == (inst is few)
+            got = ctx.download()
+            ctx.run()
+            want = ctx.download()
+            for k in ("cells", "words", "geom", "areas"):
+                assert np.array_equal(getattr(got, k), getattr(want, k))
