@@ -48,10 +48,14 @@ struct Buf;
 // Bump allocator over the scratch for the duration of one rpd_run_noalloc
 // call: Bufs that ask for memory get a block of it; their own blocks are
 // remembered and put back when the call ends.  Nothing is freed or
-// allocated while it is active.
+// allocated while it is active.  Blocks that a stage asks for under
+// ArenaTemps come from the scratch's end and are handed out again when that
+// stage is over: later work on the same stream may overwrite them.
 struct Arena {
   char* base = nullptr;
   size_t cap = 0, used = 0, high = 0;
+  size_t top = 0;  // bytes taken from the end
+  bool temps = false;
   std::vector<std::pair<Buf*, std::pair<void*, size_t>>> saved;
   bool has(const Buf* b) const {
     for (const auto& x : saved)
@@ -62,15 +66,21 @@ struct Arena {
   bool exhausted = false;
   void* take(size_t bytes) {
     const size_t b = (std::max<size_t>(bytes, 256) + 255) & ~(size_t)255;
-    if (used + b > cap) {
+    if (used + top + b > cap) {
       exhausted = true;
       return nullptr;
     }
-    void* q = base + used;
-    used += b;
-    high = std::max(high, used);
+    char* q = base + used;
+    if (temps) {
+      top += b;
+      q = base + cap - top;
+    } else {
+      used += b;
+    }
+    high = std::max(high, used + top);
     return q;
   }
+  void drop_temps();
   void restore();
 };
 thread_local Arena* t_arena = nullptr;
@@ -166,6 +176,15 @@ struct Buf {
 void Arena::touch(Buf* b) {
   if (!has(b)) saved.push_back({b, {b->p, b->cap}});
 }
+void Arena::drop_temps() {
+  for (auto& x : saved)
+    if (static_cast<char*>(x.first->p) >= base + cap - top &&
+        static_cast<char*>(x.first->p) < base + cap) {
+      x.first->p = nullptr;
+      x.first->cap = 0;
+    }
+  top = 0;
+}
 void Arena::restore() {
   for (auto& x : saved) {
     x.first->p = x.second.first;
@@ -173,6 +192,20 @@ void Arena::restore() {
   }
   saved.clear();
 }
+
+// Blocks needed while one of these is open are an arena's temporary ones; it
+// ends with close(), or with the stage (on an error the arena ends too).
+struct ArenaTemps {
+  ArenaTemps() {
+    if (t_arena) t_arena->temps = true;
+  }
+  ~ArenaTemps() { close(); }
+  void close() {
+    if (t_arena) t_arena->temps = false;
+  }
+  ArenaTemps(const ArenaTemps&) = delete;
+  ArenaTemps& operator=(const ArenaTemps&) = delete;
+};
 
 constexpr int kCounters = 16 + 128;
 
@@ -997,6 +1030,9 @@ int64_t pairs_guess(const rpd_ctx* ctx) {
 int plain_candidates(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out) {
   hipStream_t s = R.s;
   const int32_t nt = R.nt, ns = R.ns;
+  HIP_TRY(ctx->tet_count.need(((size_t)nt + 1) * 8));
+  HIP_TRY(ctx->tet_off.need(((size_t)nt + 1) * 8));
+  ArenaTemps temps;  // the rest but the candidates serves this stage alone
   if (int rc = ensure_bins(ctx, s, R.n_bins, R.inst_d)) return rc;
   const rpd_ctx::Bins& bb = ctx->has_subset ? ctx->sub_bins : ctx->bins;
   const MeshBins B{bb.first.as<int32_t>(), bb.tet.as<int32_t>(),
@@ -1017,8 +1053,6 @@ int plain_candidates(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out) {
   if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[10], s));
   HIP_TRY(exclusive_sum<int64_t>(ctx, ctx->parts.as<int64_t>(),
                                  ctx->part_off.as<int64_t>(), ns + 1));
-  HIP_TRY(ctx->tet_count.need(((size_t)nt + 1) * 8));
-  HIP_TRY(ctx->tet_off.need(((size_t)nt + 1) * 8));
   HIP_TRY(zero32(s, ctx->tet_count.p, 2 * ((int64_t)nt + 1)));
   if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[11], s));
   uint32_t* const n_pairs = (uint32_t*)(R.cnt + 8);
@@ -1030,6 +1064,9 @@ int plain_candidates(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out) {
       (uint32_t)std::max<int64_t>(1, std::min<int64_t>(6144, (int64_t)ns * 8));
   const uint32_t chunk = nt < 200000 ? 64 : 256;
   int64_t cap = R.graph ? R.cap.n_cand : pairs_guess(ctx);
+  if (t_arena)  // (a run that fits needs far more than this per pair later)
+    cap = std::min<int64_t>(
+        cap, (int64_t)(t_arena->cap - t_arena->used - t_arena->top) / 16);
   int64_t n_cand = 0, place_room = 0;
   for (;;) {
     int64_t room = cap + (int64_t)waves * chunk;
@@ -1080,6 +1117,7 @@ int plain_candidates(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out) {
   HIP_TRY(ctx->pair_seg.need(nc * 8));
   HIP_TRY(ctx->tet_fill.need((size_t)nt * 4));
   HIP_TRY(zero32(s, ctx->tet_fill.p, nt));
+  temps.close();
   HIP_TRY(ctx->cand.need(nc * sizeof(Cand)));
   HIP_TRY(ctx->rel_ids.need(nc * 4));
   if (n_cand > 0) {
@@ -1097,6 +1135,10 @@ int plain_candidates(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out) {
                        ctx->rel_ids.as<int32_t>());
   }
   HIP_TRY(hipGetLastError());
+  if (t_arena) {
+    t_arena->drop_temps();
+    ctx->bins.ready = false;
+  }
   if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[13], s));
   *n_cand_out = n_cand;
   return 0;
@@ -3287,7 +3329,8 @@ int rpd_run_noalloc(rpd_ctx* ctx, const rpd_instance_desc* desc,
                   "rpd_run_noalloc: the instance needs more than the " +
                       std::to_string(kScratchBytes >> 20) +
                       " MiB device scratch (used " +
-                      std::to_string(A.used >> 20) + " MiB before the "
+                      std::to_string((A.used + A.top) >> 20) +
+                      " MiB before the "
                       "request that failed)",
                   -4);
     return rc;

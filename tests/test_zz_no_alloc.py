@@ -119,3 +119,22 @@ def test_noalloc_refuses_an_instance_over_the_scratch(ctx):
     rc, _, err = ctx.run_noalloc(big, _out(bufs, 16, 16, 16))
     print(f"[noalloc] {big.n_tet} tets: rc {rc}: {err}", flush=True)
     assert rc == -4 and "scratch" in err
+
+
+def test_noalloc_takes_the_largest_instances(ctx):
+    # 215,622 tets and 307,628 candidates: the clip's slots leave little of
+    # the scratch, so what the relation needs has to be given back to them
+    verts, tets = prep.grid_mesh(33, 0.1, 3)
+    inst = prep.build_instance(verts, tets, prep.spheres(100, 0, 5))
+    ctx.upload(inst)
+    st = ctx.run(cells_per_wave=8)
+    ref = ctx.download()
+    n = (st["n_cells"], st["n_words"], st["n_areas"])
+    bufs = _buffers(*n)
+    rc, st, err = ctx.run_noalloc(inst, _out(bufs, *n))
+    assert rc == 0, err
+    print(f"[noalloc] {inst.n_tet} tets: scratch used "
+          f"{st['scratch_bytes'] / 2**20:.1f} MiB", flush=True)
+    _same(RPDResult(bufs[0].host(np.uint8).view(CELL_DTYPE),
+                    bufs[1].host(np.uint32), bufs[2].host(np.float64),
+                    bufs[3].host(np.float64)), ref)
