@@ -1100,8 +1100,6 @@ int plain_candidates(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out) {
                                {&n_listed, n_pairs, 4},
                                {reg64, R.cnt + 16, sizeof(reg64)}}));
     for (int q = 0; q < 64; ++q) n_reg += reg64[q];
-    if (n_reg >= (1LL << 31))
-      return fail(ctx, "rpd_run: too many sphere-bin registrations");
     ctx->st.n_bin_registrations = n_reg;
     if (n_cand >= (1LL << 31))
       return fail(ctx, "rpd_run: too many candidates");

@@ -8,6 +8,7 @@ import sys
 
 import numpy as np
 import pytest
+from scipy.spatial import cKDTree
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, os.path.join(HERE, "..", "oracle"))
@@ -234,3 +235,21 @@ def test_more_pairs_than_a_captured_list_holds():
             want = ctx.download()
             for k in ("cells", "words", "geom", "areas"):
                 assert np.array_equal(getattr(got, k), getattr(want, k))
+
+
+def test_boxes_of_more_than_2_31_bins(ctx):
+    # lists too long for the box polytope: every sphere's box is the domain,
+    # 8,400 times 262,144 bins in all; the cells fill the cube
+    verts, tets = prep.grid_mesh(64, 0.1, 3)
+    n, k = 8400, 123
+    p = np.random.default_rng(4).random((n, 3))
+    ids = np.sort(cKDTree(p).query(p, k + 1)[1][:, 1:], axis=1)
+    adj = prep.tet_adjacency(verts.shape[0], tets)
+    ctx.upload(prep.Instance(verts, tets, *adj, np.c_[p, np.zeros(n)],
+                             np.ones(n, np.uint32),
+                             np.arange(n + 1, dtype=np.int64) * k,
+                             ids.astype(np.int32).ravel()))
+    st = ctx.run()
+    assert st["n_bbox_fallback"] == n
+    assert st["n_bin_registrations"] > 1 << 31
+    assert abs(ctx.download().geom[:, 0].sum() - 1) < 1e-9
