@@ -282,7 +282,7 @@ struct rpd_ctx {
   Buf knn_bis;
   Buf knn_bisf;
   // pipeline
-  Buf bbox, rel_pl, rel_aux, parts, part_off, keys_a, keys_b;
+  Buf bbox, rel_pl, rel_aux, parts, part_off, part_rows, keys_a, keys_b;
   Buf tet_count, tet_off, pairs, pair_seg, tet_fill, cand, rel_ids;
   // int32[kCounters]: fallback, n_rerun_large, n_rerun_exact, ...,
   // [6] n_rerun_full (after the middle tier), [7] overflow of a captured
@@ -1044,10 +1044,12 @@ int plain_candidates(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out) {
   HIP_TRY(ctx->rel_aux.need(nk * 8));
   HIP_TRY(ctx->parts.need(((size_t)ns + 1) * 8));
   HIP_TRY(ctx->part_off.need(((size_t)ns + 1) * 8));
+  HIP_TRY(ctx->part_rows.need(((size_t)ns + 1) * 4));
   hipLaunchKernelGGL(k_site_bbox, dim3(ns + 1), dim3(64), 0, s, R.S, R.inst_d,
                      R.site_inst_d, ctx->bbox.as<double>(),
                      ctx->rel_pl.as<float4>(), ctx->rel_aux.as<float2>(),
-                     ctx->parts.as<int64_t>(),
+                     B.first, ctx->parts.as<int64_t>(),
+                     ctx->part_rows.as<int32_t>(),
                      (unsigned long long*)(R.cnt + 16), R.cnt + 0);
   HIP_TRY(hipGetLastError());
   if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[10], s));
@@ -1057,12 +1059,15 @@ int plain_candidates(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out) {
   if (!R.graph) HIP_TRY(hipEventRecord(ctx->ev[11], s));
   uint32_t* const n_pairs = (uint32_t*)(R.cnt + 8);
   unsigned long long* const count = ctx->tet_count.as<unsigned long long>();
-  // wavefronts that walk the parts: enough to fill the chip, few enough
-  // that most take several; their chunks of the pair list, small where the
-  // list is
-  const uint32_t waves =
-      (uint32_t)std::max<int64_t>(1, std::min<int64_t>(6144, (int64_t)ns * 8));
-  const uint32_t chunk = nt < 200000 ? 64 : 256;
+  // Wavefronts that walk the parts (no more than there can be parts), and
+  // their chunks of the pair list.  1.57 M tets with 18,000 sites: 1,536
+  // wavefronts 0.85 ms, 3,072 0.55, 6,144 0.53, 12,288 0.51; chunks of 64
+  // 0.80 (the list's counter is one address), 128 0.54, 256, 512 and 1,024
+  // 0.53 ms; with 2,600 sites 0.65, 0.41, 0.32 and 0.32, 0.32.  Larger
+  // numbers of either only lengthen the list.
+  const uint32_t waves = (uint32_t)std::max<int64_t>(
+      1, std::min<int64_t>(6144, (int64_t)ns * (nt / kPartTets + 1)));
+  const uint32_t chunk = 256;
   int64_t cap = R.graph ? R.cap.n_cand : pairs_guess(ctx);
   if (t_arena)  // (a run that fits needs far more than this per pair later)
     cap = std::min<int64_t>(
@@ -1077,7 +1082,8 @@ int plain_candidates(rpd_ctx* ctx, RunState& R, int64_t* n_cand_out) {
       hipLaunchKernelGGL(
           k_rel_pairs, dim3(waves), dim3(64), 0, s, R.M, R.S, B, R.inst_d,
           R.site_inst_d, ctx->bbox.as<double>(), ctx->rel_pl.as<float4>(),
-          ctx->rel_aux.as<float2>(), ctx->part_off.as<int64_t>(), count,
+          ctx->rel_aux.as<float2>(), ctx->part_off.as<int64_t>(),
+          ctx->part_rows.as<int32_t>(), count,
           ctx->pairs.as<int2>(), n_pairs, chunk, room,
           R.cfg.count_work ? ctx->rel_work.as<unsigned long long>() : nullptr);
     HIP_TRY(hipGetLastError());

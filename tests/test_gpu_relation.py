@@ -253,3 +253,26 @@ def test_boxes_of_more_than_2_31_bins(ctx):
     assert st["n_bbox_fallback"] == n
     assert st["n_bin_registrations"] > 1 << 31
     assert abs(ctx.download().geom[:, 0].sum() - 1) < 1e-9
+
+
+def graded(n, p, sph):
+    """The grid with its corners' coordinates to the p-th power: most tets
+    in few bins of the candidate grid."""
+    verts, tets = prep.grid_mesh(n, 0.1, 3)
+    return prep.build_instance(np.clip(verts, 0, 1) ** p, tets, sph)
+
+
+@pytest.mark.parametrize("m", [1, 3, 40])
+def test_graded_mesh(ctx, m):
+    # rows of several thousand tets and rows of none: parts cut by count
+    check(ctx, graded(20, 4, prep.spheres(m, 0, 5)))
+
+
+@pytest.mark.parametrize("p,m", [(1, 1), (1, 5), (4, 100)])
+def test_relation_is_spread_over_the_chip(ctx, p, m):
+    # few spheres, or most tets in few bins: the relation is no serial walk
+    # of some wavefronts (3.7, 1.3 and 5.4 ms when it was; the clip takes
+    # 0.4 to 0.7 ms, the relation a third of that)
+    ctx.upload(graded(64, p, prep.spheres(m, 0, 5)))
+    ms = np.array([ctx.run()["ms_kernel"] for _ in range(6)])
+    assert ms[:, 2].min() < ms[:, 5].min()
