@@ -324,9 +324,10 @@ int rpd_site_centroids(rpd_ctx* ctx, double* out, const double** dev_out);
  * at the capacity.  rpd_graph_run replays the graph on the current data
  * (rpd_update_sites_batch may replace spheres and neighbour lists between
  * runs) and reads the counts back once; if one went past its capacity, or
- * the batch's per-instance tet or site counts, its mesh, the tet subset
- * switch or a device buffer changed, it captures again through rpd_graph_build (whose
- * eager run gives the results) and sets *replayed = 0, else 1.  Results
+ * the batch's per-instance tet or site counts, the size of its grids, the
+ * tet subset switch or a device buffer changed, it captures again through
+ * rpd_graph_build (whose eager run gives the results) and sets *replayed =
+ * 0, else 1.  A mesh of the same sizes may be uploaded between runs.  Results
  * are read as after rpd_run.  Plain and learned paths (cfg->learned 0, 1
  * or 2); count_work = 0, small_tier = 1.  A learned capture holds the
  * certificate, one closure round more than its eager run needed (a replay

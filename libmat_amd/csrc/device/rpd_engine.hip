@@ -296,6 +296,9 @@ struct rpd_ctx {
   } bins, sub_bins;
   Buf bin_n, bin_rank;
   int64_t mesh_id = 0;  // counts the uploads
+  // the upload whose instance table is in the pinned block (-1: that of an
+  // allocation-free call), and that table's grid cells
+  int64_t pin_inst_id = -1, n_bins = 0, n_sg = 0;
   Buf rerun_large, rerun_full, rerun_exact, loc, sizes, offs, drops, stats64,
       work, rel_work;
   Buf scan_tmp;
@@ -333,7 +336,7 @@ struct rpd_ctx {
   RunCaps graph_cap{};
   rpd_run_cfg graph_cfg{};
   double graph_headroom = 0;
-  int64_t graph_bins = 0;  // cells of the candidate grid
+  int64_t graph_bins = 0, graph_sg = 0;  // grid cells at the capture
   std::vector<int64_t> graph_sig;
   // learned proposals: features, model (fp32 master, Adam state, bf16
   // copies), certificate and fallback
@@ -949,6 +952,9 @@ int upload_inst_info(rpd_ctx* ctx, RunState& R) {
     ctx->pin_inst_cap = bytes;
   }
   std::memcpy(ctx->pin_inst, ii.data(), bytes);
+  ctx->pin_inst_id = t_arena ? -1 : ctx->mesh_id;
+  ctx->n_bins = n_bins;
+  ctx->n_sg = n_sg;
   HIP_TRY(hipMemcpyAsync(ctx->inst_dev.p, ctx->pin_inst, bytes,
                          hipMemcpyHostToDevice, R.s));
   if (!R.graph) {
@@ -2644,7 +2650,6 @@ std::vector<int64_t> graph_signature(const rpd_ctx* ctx) {
     v.push_back(I.n_site);
   }
   v.push_back(ctx->has_subset);
-  v.push_back(ctx->mesh_id);  // a new mesh has its own bins and domain boxes
   v.push_back((int64_t)(intptr_t)ctx->pin_inst);
   v.push_back((int64_t)g_buf_generation.load());
   return v;
@@ -2802,6 +2807,7 @@ int rpd_graph_build(rpd_ctx* ctx, const rpd_run_cfg* cfg, double headroom) {
   ctx->graph_headroom = headroom;
   ctx->graph_sig = graph_signature(ctx);
   ctx->graph_bins = P.n_bins;
+  ctx->graph_sg = P.n_sg;
   ctx->st = st_eager;  // the eager run's results are the current ones
   return 0;
 }
@@ -2814,17 +2820,31 @@ int rpd_graph_run(rpd_ctx* ctx, int32_t* replayed) {
   if (!ctx->has_mesh || !ctx->has_sites)
     return fail(ctx, "rpd_graph_run: no resident instance");
   HIP_TRY(hipSetDevice(ctx->device));
-  // the batch or a buffer changed since the capture, or the neighbour
-  // lists outgrew the captured bisector table: capture again (its eager run
-  // gives this call's results)
+  const bool learned = ctx->graph_cfg.learned != 0;
+  hipStream_t s = ctx->stream;
+  // the replay copies the instance table from the pinned block: this batch's
+  // belongs there (a new mesh, or an allocation-free call in between)
+  if (ctx->pin_inst_id != ctx->mesh_id) {
+    RunState P;
+    P.s = s;
+    if (int rc = upload_inst_info(ctx, P)) return rc;
+  }
+  const bool grids = learned ? ctx->n_sg == ctx->graph_sg
+                             : ctx->n_bins <= ctx->graph_bins;
+  if (!learned && grids)  // (of a new mesh or subset)
+    if (int rc = ensure_bins(ctx, s, ctx->n_bins,
+                             ctx->inst_dev.as<InstInfo>()))
+      return rc;
+  // the batch, its grids or a buffer changed since the capture, or the
+  // neighbour lists outgrew the captured bisector table: capture again (its
+  // eager run gives this call's results)
   const size_t nk = (size_t)std::max<int64_t>(ctx->n_knn, 1);
-  if (graph_signature(ctx) != ctx->graph_sig || nk * 32 > ctx->knn_bis.cap ||
-      nk * 16 > ctx->knn_bisf.cap || nk * 16 > ctx->rel_pl.cap ||
-      nk * 8 > ctx->rel_aux.cap) {
+  if (!grids || graph_signature(ctx) != ctx->graph_sig ||
+      nk * 32 > ctx->knn_bis.cap || nk * 16 > ctx->knn_bisf.cap ||
+      nk * 16 > ctx->rel_pl.cap || nk * 8 > ctx->rel_aux.cap) {
     const rpd_run_cfg c = ctx->graph_cfg;
     return rpd_graph_build(ctx, &c, ctx->graph_headroom);
   }
-  const bool learned = ctx->graph_cfg.learned != 0;
   if (learned && ctx->tet_off.p != ctx->graph_tet_off) {
     // an eager learned run since the capture swapped the offset buffers
     // the graph writes: swap them back
@@ -2839,11 +2859,6 @@ int rpd_graph_run(rpd_ctx* ctx, int32_t* replayed) {
   ctx->last_geometry = false;
   ctx->has_results = false;
   ctx->adj_ready = false;
-  hipStream_t s = ctx->stream;
-  if (!learned && ctx->has_subset && !ctx->sub_bins.ready)  // a new subset
-    if (int rc = ensure_bins(ctx, s, ctx->graph_bins,
-                             ctx->inst_dev.as<InstInfo>()))
-      return rc;
   HIP_TRY(hipEventRecord(ctx->ev[0], s));
   HIP_TRY(hipGraphLaunch(ctx->graph_exec, s));
   HIP_TRY(hipEventRecord(ctx->ev[4], s));

@@ -16,6 +16,7 @@ import oracle  # noqa: E402
 from libmat_amd import prep  # noqa: E402
 from libmat_amd.rpd import Context  # noqa: E402
 from rpd_compare import compare_relation, compare_with_oracle  # noqa: E402
+from test_zz_no_alloc import _buffers, _out  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -193,6 +194,37 @@ def test_graph_follows_a_new_mesh_of_the_same_sizes(ctx):
         assert np.array_equal(got.cells, want.cells)
         assert np.array_equal(got.words, want.words)
         assert np.array_equal(got.geom, want.geom)
+
+
+@pytest.mark.parametrize("learned", [0, 2])
+def test_graph_replays_on_meshes_of_the_same_sizes(ctx, learned):
+    # and after an allocation-free call, which has an instance of its own
+    small = prep.build_instance(*prep.grid_mesh(2, 0.1, 1),
+                                prep.spheres(30, 0, 1))
+    small.verts[:] *= 0.5
+    insts = []
+    for seed, scale in ((1, 1.0), (2, 1.0), (3, 4.0)):
+        inst = prep.build_instance(*prep.grid_mesh(6, 0.1, seed),
+                                   prep.spheres(40, 0, 5))
+        insts.append(dataclasses.replace(
+            inst, verts=inst.verts * scale,
+            sites=inst.sites * np.array([scale] * 3 + [scale * scale])))
+    ctx.upload(insts[0])
+    ctx.graph_build(headroom=1.0, learned=learned)
+    n = (1 << 13, 1 << 19, 1 << 17)
+    bufs = _buffers(*n)
+    for inst in insts[::-1] + insts:
+        ctx.upload(inst)
+        for _ in range(2):
+            rc, _, err = ctx.run_noalloc(small, _out(bufs, *n))
+            assert rc == 0, err
+            _, replayed = ctx.graph_run()
+            assert replayed
+            got = ctx.download()
+            ctx.run(learned=learned)
+            want = ctx.download()
+            for k in ("cells", "words", "geom", "areas"):
+                assert np.array_equal(getattr(got, k), getattr(want, k))
 
 
 def unlisted(inst):
