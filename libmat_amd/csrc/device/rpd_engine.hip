@@ -3070,6 +3070,10 @@ int rpd_power_neighbors_gpu(rpd_ctx* ctx, int32_t n, const double* xyzw,
   std::vector<int64_t> starts;
   std::vector<int32_t> ids;
   std::vector<float> cell_w;
+  double reach = 0;
+  for (int a = 0; a < 6; ++a) reach = std::max(reach, std::fabs(box[a]));
+  const int exp2 = std::min(500, std::max(-500, std::ilogb(reach)));
+  const NbUnit unit{std::ldexp(1.0, exp2), std::ldexp(1.0, -exp2)};
   for (int c = 0; c < kRpdClasses; ++c) {
     const RpdClassGrid& g = grids[c];
     NbGrid& d = G.g[c];
@@ -3084,7 +3088,8 @@ int rpd_power_neighbors_gpu(rpd_ctx* ctx, int32_t n, const double* xyzw,
     d.cell_base = (int64_t)starts.size();
     const int64_t id_base = (int64_t)ids.size();
     for (size_t q = 0; q < g.start.size(); ++q) {
-      // the cell's largest weight, rounded up to binary32; -1: no member
+      // the cell's largest weight in square units, rounded up to binary32;
+      // -1: no member
       double w = 0;
       const bool some =
           q + 1 < g.start.size() && g.start[q] < g.start[q + 1];
@@ -3092,7 +3097,9 @@ int rpd_power_neighbors_gpu(rpd_ctx* ctx, int32_t n, const double* xyzw,
         for (int64_t v = g.start[q]; v < g.start[q + 1]; ++v)
           w = std::max(w, xyzw[4 * (int64_t)g.ids[v] + 3]);
       starts.push_back(id_base + g.start[q]);
-      cell_w.push_back(some ? std::nextafter((float)w, INFINITY) : -1.f);
+      cell_w.push_back(
+          some ? std::nextafter((float)(w * unit.inv * unit.inv), INFINITY)
+               : -1.f);
     }
     ids.insert(ids.end(), g.ids.begin(), g.ids.end());
   }
@@ -3126,7 +3133,7 @@ int rpd_power_neighbors_gpu(rpd_ctx* ctx, int32_t n, const double* xyzw,
   if (n > 0) {
     hipLaunchKernelGGL((k_power_nbrs<1, 64>), dim3(n), dim3(64), 0, s, n,
                        (const int32_t*)nullptr, (const int32_t*)nullptr,
-                       ctx->nb_sph.as<double4>(), ctx->nb_box.as<double>(), G,
+                       ctx->nb_sph.as<double4>(), ctx->nb_box.as<double>(), G, unit,
                        ctx->nb_start.as<int64_t>(), ctx->nb_ids.as<int32_t>(),
                        ctx->nb_cellw.as<float>(), ctx->nb_valid.as<int32_t>(), ctx->nb_cnt.as<int32_t>(),
                        ctx->nb_lists.as<int32_t>(), counters + 2, counters);
@@ -3136,7 +3143,7 @@ int rpd_power_neighbors_gpu(rpd_ctx* ctx, int32_t n, const double* xyzw,
                        dim3(std::min(n, 2048)), dim3(64), 0, s, n,
                        (const int32_t*)(counters + 2),
                        (const int32_t*)counters, ctx->nb_sph.as<double4>(),
-                       ctx->nb_box.as<double>(), G,
+                       ctx->nb_box.as<double>(), G, unit,
                        ctx->nb_start.as<int64_t>(), ctx->nb_ids.as<int32_t>(),
                        ctx->nb_cellw.as<float>(), ctx->nb_valid.as<int32_t>(), ctx->nb_cnt.as<int32_t>(),
                        ctx->nb_lists.as<int32_t>(), (int32_t*)nullptr,

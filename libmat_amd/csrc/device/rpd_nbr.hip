@@ -78,12 +78,22 @@ __device__ __forceinline__ int shell_size(int r) {
 __device__ __noinline__ int nb_exact_w(rpd_d4 p1, rpd_d4 p2, rpd_d4 p3) {
   return rpd_exact_w_sign(p1, p2, p3);
 }
+// The builder's unit of length, a power of two near the box's largest
+// coordinate (1 for the unit cube): filter bounds and binary32 positions are
+// taken in it, so neither depends on the scale of the spheres.
+struct NbUnit {
+  double len, inv;  // and its reciprocal
+};
+
 // dot(e, X) and the filter bound of its sign: rpd_filtered_sign4 with
-// sum |e_r| Q_r replaced by the larger max |e_r| * sum Q_r (the sum and the
-// product fall short by at most 4u relative, which the 8 % slack of the
-// constant over gamma_10 covers; products may fuse into the sums, no
-// monomial then passing through more roundings).  An unrepresentable bound
-// is infinite: nothing is decided.
+// sum |e_r| Q_r replaced by the larger me * sq, me = max(|e_xyz|, |e_w| / len)
+// and sq = Q_x + Q_y + Q_z + len Q_w (the sum and the product fall short by
+// at most 4u relative, which the 8 % slack of the constant over gamma_10
+// covers; products may fuse into the sums, no monomial then passing through
+// more roundings).  e_w and Q_xyz carry one length more than e_xyz and Q_w:
+// without the unit the bound is too wide by the scale or its reciprocal, and
+// from 1e12 on every sign was open (6,000 spheres 10 -> 2,500 ms).  An
+// unrepresentable bound is infinite: nothing is decided.
 __device__ __forceinline__ void nb_dot(const rpd_d4& e, double me,
                                        const rpd_d4& X, double sq, double& s,
                                        double& eps) {
@@ -155,7 +165,7 @@ __device__ __forceinline__ float wave_add(float v) {
 template <int kVS, int kP>
 __device__ __forceinline__ void power_cell(
     int i, const double4* __restrict__ sph, const double* box,
-    const NbGrids& G, const int64_t* __restrict__ start,
+    const NbGrids& G, const NbUnit& unit, const int64_t* __restrict__ start,
     const int32_t* __restrict__ ids, int32_t* valid, int32_t* counts,
     int32_t* lists, int32_t* rerun, int32_t* n_rerun, double4* s_pl,
     int32_t* s_src, uint32_t* s_new, int32_t* s_q, uint8_t* s_used,
@@ -164,11 +174,13 @@ __device__ __forceinline__ void power_cell(
   const int lane = threadIdx.x;
   const double4 sd = sph[i];
   const rpd_d4 si{sd.x, sd.y, sd.z, sd.w};
+  // the centre in units
+  const double cx = si.x * unit.inv, cy = si.y * unit.inv, cz = si.z * unit.inv;
   rpd_d4 X[kVS];
   double sq[kVS];
   uint32_t tr[kVS];     // planes a | b << 8 | c << 16, bit 31: X.w is 0
   uint64_t alive[kVS];  // slots in use
-  float ux[kVS], uy[kVS], uz[kVS];  // position less the sphere's centre
+  float ux[kVS], uy[kVS], uz[kVS];  // position less the centre, in units
 #pragma unroll
   for (int q = 0; q < kVS; ++q) {
     X[q] = rpd_d4{0, 0, 0, 1};
@@ -200,11 +212,11 @@ __device__ __forceinline__ void power_cell(
       trq = a | (b << 8) | (c << 16) | (sw == 0 ? 0x80000000u : 0u);
     }
     Xq = Y;
-    sqq = ((Q.x + Q.y) + Q.z) + Q.w;
-    const double iw = rcp64(Y.w);
-    uxq = (float)(Y.x * iw - si.x);
-    uyq = (float)(Y.y * iw - si.y);
-    uzq = (float)(Y.z * iw - si.z);
+    sqq = fma(Q.w, unit.len, (Q.x + Q.y) + Q.z);
+    const double iw = rcp64(Y.w) * unit.inv;
+    uxq = (float)fma(Y.x, iw, -cx);
+    uyq = (float)fma(Y.y, iw, -cy);
+    uzq = (float)fma(Y.z, iw, -cz);
   };
 
   // the domain box: x >= x0, x <= x1, y >= y0, y <= y1, z >= z0, z <= z1
@@ -388,11 +400,12 @@ __device__ __forceinline__ void power_cell(
       const double4 sj = sph[j];
       const double dx = sj.x - si.x, dy = sj.y - si.y, dz = sj.z - si.z;
       const double d = sqrt(dx * dx + dy * dy + dz * dz);
-      const double Rc = sqrt((double)R2) * (1 + 1e-9) + 1e-12;
+      const double Rc = sqrt((double)R2) * unit.len * (1 + 1e-9) + 1e-12;
       const double bj = Rc + sqrt(fmax(0.0, Rc * Rc - si.w + sj.w));
       may = !(d > bj * (1 + 1e-9) + 1e-12);
       e = rpd_bisector(si, rpd_d4{sj.x, sj.y, sj.z, sj.w});
-      me = fmax(fmax(fabs(e.x), fabs(e.y)), fmax(fabs(e.z), fabs(e.w)));
+      me = fmax(fmax(fabs(e.x), fabs(e.y)),
+                fmax(fabs(e.z), fabs(e.w) * unit.inv));
     }
     const uint64_t reach = ballot(may);
     if (reach == 0) return;
@@ -441,13 +454,16 @@ __device__ __forceinline__ void power_cell(
       if (hi > rmin) rmin = hi;
       g_lo[a] = (int)max(-lo, (int64_t)-0x7fffffff);
       g_hi[a] = (int)max(min(-hi, (int64_t)0x7fffffff), (int64_t)-0x7fffffff);
-      off[a] = (float)(g.org[a] + (double)q0[a] * g.cs - (&si.x)[a]);
+      off[a] = (float)((g.org[a] + (double)q0[a] * g.cs - (&si.x)[a]) *
+                       unit.inv);
     }
     const int64_t cell0 =
         g.cell_base + q0[0] +
         (int64_t)g.dim[0] * (q0[1] + (int64_t)g.dim[1] * q0[2]);
-    const float csf = (float)g.cs, wi = (float)si.w;
-    const float wm = (float)g.wmax * 1.00001f, ics = 1.0f / csf;
+    const float csf = (float)(g.cs * unit.inv);
+    const float wi = (float)(si.w * unit.inv * unit.inv);
+    const float wm = (float)(g.wmax * unit.inv * unit.inv) * 1.00001f;
+    const float ics = 1.0f / csf;
     // A sphere of weight up to wl in a cell's box cuts a vertex off only if
     // d2 <= vv - w_i + wl (d2: squared distance of the vertex to the box,
     // vv: to the centre), here with 1e-5 of every term for the rounding:
@@ -461,7 +477,7 @@ __device__ __forceinline__ void power_cell(
     int qn = 0;  // spheres waiting in s_q
     bool done = false;
     for (int64_t r = rmin; !done && !empty && !fail; ++r) {
-      const double R = sqrt((double)R2) * (1 + 1e-9) + 1e-12;
+      const double R = sqrt((double)R2) * unit.len * (1 + 1e-9) + 1e-12;
       {
         const double bound = R + sqrt(fmax(0.0, R * R - si.w + g.wmax));
         done = r > rmax ||
@@ -705,8 +721,8 @@ template <int kVS, int kP>
 __global__ __launch_bounds__(64, (kVS == 1 ? 3 : 1)) void k_power_nbrs(
     int32_t n, const int32_t* items, const int32_t* n_items,
     const double4* __restrict__ sph, const double* box, NbGrids G,
-    const int64_t* __restrict__ start, const int32_t* __restrict__ ids,
-    const float* __restrict__ cell_w, int32_t* valid, int32_t* counts,
+    NbUnit unit, const int64_t* __restrict__ start,
+    const int32_t* __restrict__ ids, const float* __restrict__ cell_w, int32_t* valid, int32_t* counts,
     int32_t* lists, int32_t* rerun, int32_t* n_rerun) {
   __shared__ double4 s_pl[kP];
   __shared__ int32_t s_src[kP];
@@ -716,9 +732,9 @@ __global__ __launch_bounds__(64, (kVS == 1 ? 3 : 1)) void k_power_nbrs(
   __shared__ uint8_t s_map[kP];
   const int32_t m = items ? min(n, *n_items) : n;
   for (int32_t q = blockIdx.x; q < m; q += gridDim.x)
-    power_cell<kVS, kP>(items ? items[q] : q, sph, box, G, start, ids, valid,
-                        counts, lists, rerun, n_rerun, s_pl, s_src, s_new,
-                        s_q, s_used, s_map, cell_w);
+    power_cell<kVS, kP>(items ? items[q] : q, sph, box, G, unit, start, ids,
+                        valid, counts, lists, rerun, n_rerun, s_pl, s_src,
+                        s_new, s_q, s_used, s_map, cell_w);
 }
 
 // One thread per list entry (i, k): every entry's sphere must be valid and
