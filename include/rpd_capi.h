@@ -238,7 +238,9 @@ int rpd_get_stats(const rpd_ctx* ctx, rpd_stats* out);
  * device time of the cell clipping.  Fails (non-zero, rpd_last_error)
  * when a cell needs more than 186 bisector planes at once, 256 vertices or
  * 160 neighbours; planes that no longer carry a vertex are dropped as the
- * cell is clipped, so only the final cell's size counts. */
+ * cell is clipped, so only the final cell's size counts.  The context keeps
+ * the builder's device buffers (about 0.7 KB per sphere of the largest set)
+ * until it is destroyed. */
 typedef struct rpd_nbr rpd_nbr;
 int rpd_power_neighbors_gpu(rpd_ctx* ctx, int32_t n, const double* xyzw,
                             const double* box, double* ms_out,

@@ -395,7 +395,8 @@ __global__ __launch_bounds__(64, (clip_min_waves<G, C>())) void k_clip(
       const uint32_t cm = (uint32_t)conf_lo;
       const int keep = nb_v - nr;
       const int m = keep + (int)((cm >> keep) & 1);
-      const uint32_t lo_m = (1u << m) - 1u;  // m <= nb_v - 1 < 32
+      // (m <= nb_v: all but the last vertex kept; nb_v < V <= 32)
+      const uint32_t lo_m = (1u << m) - 1u;
       const uint32_t f = cm & lo_m;
       const uint32_t b = ~cm & ~lo_m & (nb_v >= 32 ? ~0u : (1u << nb_v) - 1u);
       uint32_t val[VS];

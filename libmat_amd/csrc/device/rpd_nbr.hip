@@ -6,8 +6,10 @@
 // empty; its neighbours are the spheres whose bisector carries a face of
 // the cell.  This is the restatement of the reference's CGAL regular
 // triangulation step (triangulation.cxx:62-144, get_RT_neighbors_given_
-// spheres :396-438) that the host builder rpd_power_neighbors computes; the
-// per-sphere lists are symmetrised on the host (rpd_nbr_from_lists).
+// spheres :396-438) that the host builder rpd_power_neighbors computes.
+// Lists that are their own symmetric closure (k_nbr_check) are packed on the
+// device; where bisectors meet in one point they may not be, and the host
+// closes them (rpd_nbr_from_lists).
 //
 // Candidates come from weight-class grids (rpd_classgrid.h): class by
 // class, shells of grid cells at Chebyshev distance r around the sphere's
@@ -69,10 +71,6 @@ __device__ __forceinline__ void shell_cell(int r, int k, int& dx, int& dy,
     dx = (p2 & 1) ? r : -r;
     dy = -r + 1 + (p2 >> 1);
   }
-}
-
-__device__ __forceinline__ int shell_size(int r) {
-  return r == 0 ? 1 : 2 * (2 * r + 1) * (2 * r + 1) + (2 * r - 1) * 8 * r;
 }
 
 __device__ __noinline__ int nb_exact_w(rpd_d4 p1, rpd_d4 p2, rpd_d4 p3) {

@@ -548,9 +548,10 @@ __device__ __noinline__ bool relation_exact(const DevMesh& M,
 
 // Tet-sphere relation (voronoi.cu:154-193), sphere by sphere: a tet is
 // related to sphere i iff every neighbour's bisector leaves one of its
-// corners on i's side.  A part takes kRelRows grid rows (y, z) of the
-// sphere's box: one quad of lanes per row bounds the x range that the pushed
-// planes leave of it; the tets of the ranges are then tested 64 at a time,
+// corners on i's side.  A wavefront takes a part of the sphere's box
+// (kPartTets): the lanes of a row (y, z), four of them for each of kRelRows
+// rows, bound the x range that the pushed planes leave of it; the tets of the
+// ranges are then tested 64 at a time,
 // their corners read contiguously, the planes read from LDS by all lanes at
 // once, nearest first, until no lane is left.  Values within a plane's error
 // bound leave a pair open, and relation_exact decides it.
@@ -558,15 +559,15 @@ __device__ __noinline__ bool relation_exact(const DevMesh& M,
 // Bound by instruction issue (18 per plane and 64 tets).  One thread per tet
 // over the spheres registered in its bin, in binary64, was bound by the
 // divergence of 64 different lists and, on small meshes, by their length:
-// 1.57 M tets, 18,000 sites: binning, counting and filling 2.8 ms, this
-// with the pair lists 0.65 ms; 16 instances of 2,000 to 200,000 tets with up
+// 1.57 M tets, 18,000 sites: binning, counting and filling 2.6 ms, this
+// with the pair lists 0.64 ms; 16 instances of 2,000 to 200,000 tets with up
 // to 20,000 sites (bin lists past 128, tested twice) 11.7 -> 0.57 ms; 6,000
-// tets 0.55 -> 0.04 ms.
+// tets 0.55 -> 0.03 ms.
 //
 // Related pairs are counted per tet (nothing waits for these atomics) and go
-// to an unordered list.  A wavefront takes list
-// entries in chunks (one atomic at one address for 64 pairs took 2.0 ms of
-// 2.5 at 3.5 M pairs) and marks what it leaves of its last one.
+// to an unordered list.  A wavefront takes list entries in chunks (one atomic
+// at one address for 64 pairs took 2.0 ms of 2.5 at 3.5 M pairs) and marks
+// what it leaves of its last one.
 constexpr int kRelPl = 128;
 __global__ __launch_bounds__(64) void k_rel_pairs(
     DevMesh M, DevSites S, MeshBins B, const InstInfo* inst,

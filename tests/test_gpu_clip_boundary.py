@@ -1,6 +1,6 @@
 """The clip's cavity boundary in every shape: cells of few and of many planes
-(packed cycle up to 16 planes, masks of 32 and 64 bits above), facets cut
-off altogether, and ties, against the oracle's serial walk."""
+(the packed cycle in shapes of up to 16 planes, the serial walk above),
+facets cut off altogether, and ties, against the oracle's serial walk."""
 import os
 import sys
 
