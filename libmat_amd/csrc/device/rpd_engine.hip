@@ -297,7 +297,7 @@ struct rpd_ctx {
   Buf bin_n, bin_rank;
   int64_t mesh_id = 0;  // counts the uploads
   // the upload whose instance table is in the pinned block (-1: that of an
-  // allocation-free call), and that table's grid cells
+  // allocation-free call, or of other site counts), and its grid cells
   int64_t pin_inst_id = -1, n_bins = 0, n_sg = 0;
   Buf rerun_large, rerun_full, rerun_exact, loc, sizes, offs, drops, stats64,
       work, rel_work;
@@ -591,6 +591,8 @@ int rpd_update_sites_batch(rpd_ctx* ctx, int32_t n_inst,
   int32_t max_deg = 0;
   for (int32_t b = 0; b < n_inst; ++b) {
     const rpd_sites_desc& d = sd[b];
+    if (d.n_site != ctx->inst[b].n_site)  // the instance table holds it
+      ctx->pin_inst_id = -1;
     ctx->inst[b].n_site = d.n_site;
     ctx->inst[b].site_off = so;
     if (d.n_site) std::memcpy(&site[4 * so], d.sites, (size_t)d.n_site * 32);

@@ -227,6 +227,28 @@ def test_graph_replays_on_meshes_of_the_same_sizes(ctx, learned):
                 assert np.array_equal(getattr(got, k), getattr(want, k))
 
 
+@pytest.mark.parametrize("learned", [0, 2])
+def test_graph_after_a_run_on_other_site_counts(ctx, learned):
+    # the counts are the capture's again, the instance table in between was
+    # not
+    verts, tets = prep.grid_mesh(6, 0.1, 1)
+    some = [[prep.sites_both(prep.spheres(m, 0, m))[1] for m in ms]
+            for ms in ((40, 70), (300, 9))]
+    adj = prep.tet_adjacency(verts.shape[0], tets)
+    ctx.upload_batch([prep.Instance(verts, tets, *adj, *s) for s in some[0]])
+    ctx.graph_build(headroom=1.0, learned=learned)
+    for _ in range(2):
+        ctx.update_sites_batch(some[1])
+        ctx.run(learned=learned)
+        ctx.update_sites_batch(some[0])
+        ctx.graph_run()
+        got = ctx.download()
+        ctx.run(learned=learned)
+        want = ctx.download()
+        for k in ("cells", "words", "geom", "areas"):
+            assert np.array_equal(getattr(got, k), getattr(want, k))
+
+
 def unlisted(inst):
     """The same instance without neighbour lists: every sphere relates to
     every tet, far more pairs than a run expects of its sizes."""
