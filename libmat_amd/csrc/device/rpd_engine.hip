@@ -921,6 +921,20 @@ int upload_inst_info(rpd_ctx* ctx, RunState& R) {
       return nb;
     };
     const int64_t nb = grid(I.n_tet / 6.0, o.g);
+    // the tets' grid with its longest axis first
+    int f = 0;
+    for (int a = 1; a < 3; ++a)
+      if (o.g.dim[a] > o.g.dim[f]) f = a;
+    const BinGrid n = o.g;
+    for (int k = 0; k < 3; ++k) {
+      const int a = k == 0 ? f : k <= f ? k - 1 : k;
+      o.ax[k] = a;
+      o.g.org[k] = n.org[a];
+      o.g.dim[k] = n.dim[a];
+      o.gdom[k] = I.dom[a];
+      o.gdom[3 + k] = I.dom[3 + a];
+    }
+    o.ax[3] = 0;
     o.bin_base = n_bins;
     n_bins += nb;
     const int64_t ng = grid(I.n_site / 2.0, o.sg);

@@ -322,6 +322,37 @@ def test_graded_mesh(ctx, m):
     check(ctx, graded(20, 4, prep.spheres(m, 0, 5)))
 
 
+def squeezed(n, p, scale, m):
+    """The grid graded by the p-th power, then scaled per axis, and its
+    spheres."""
+    verts, tets = prep.grid_mesh(n, 0.1, 3)
+    scale = np.asarray(scale, float)
+    sph = prep.spheres(m, 0, 5)
+    sph[:, :3] *= scale
+    sph[:, 3] *= scale.min()
+    return prep.build_instance(
+        np.clip(verts, 0, 1) ** p * scale, tets, sph,
+        box=np.r_[-1e-6 * scale, (1 + 1e-6) * scale])
+
+
+@pytest.mark.parametrize("p", [1, 3])
+@pytest.mark.parametrize("scale", [
+    (0.02, 1, 1), (1, 0.02, 1), (1, 1, 0.02), (0.5, 0.02, 1), (1, 0.02, 0.02),
+    (0.02, 1, 0.02), (0.02, 0.02, 1), (0.02, 0.5, 1)])
+def test_flat_and_long_meshes(ctx, scale, p):
+    # the grid's rows run along its longest axis
+    check(ctx, squeezed(9, p, scale, 25))
+
+
+@pytest.mark.parametrize("p", [1, 3])
+@pytest.mark.parametrize("scale", [(0.002, 1, 1), (1, 0.002, 1)])
+def test_relation_of_a_flat_mesh_is_spread_over_the_chip(ctx, scale, p):
+    # (boxes and relation of one sphere took 7 to 15 ms, the clip 0.5)
+    ctx.upload(squeezed(64, p, scale, 1))
+    ms = np.array([ctx.run()["ms_kernel"] for _ in range(6)])
+    assert (ms[:, 0] + ms[:, 2]).min() < ms[:, 5].min()
+
+
 @pytest.mark.parametrize("p,m", [(1, 1), (1, 5), (4, 100)])
 def test_relation_is_spread_over_the_chip(ctx, p, m):
     # few spheres, or most tets in few bins: the relation is no serial walk
